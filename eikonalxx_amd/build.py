@@ -40,11 +40,13 @@ def compile_flags():
             "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 
 
-# Per-source flags.  The column kernels are scheduled for instruction-level
-# parallelism: their steps are bound by VALU issue and dependency latency at
-# a residency the LDS fixes, not by registers.
+# Per-source flags.  The column and band kernels are scheduled for
+# instruction-level parallelism: their steps are bound by VALU issue and
+# dependency latency at a residency that LDS (3D) or the few waves of a
+# problem (2D) fix, not by registers.
 SOURCE_FLAGS = {
     "ekx_kernels3d.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
+    "ekx_kernels2d.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
 }
 
 

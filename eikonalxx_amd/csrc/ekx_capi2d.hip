@@ -75,6 +75,41 @@ template <typename T> struct Buf
     }
 };
 
+// The band kernel's buffers: skewed travel times (work) and skewed cells,
+// none (both counts 0) for grids that it does not take.  Memory that the device does not have
+// is no error: the solve then runs the level kernel, which needs neither.
+bool allocate_bands(Buf<double> &work, int64_t workValues,
+                    Buf<double> &cells, int64_t cellValues)
+{
+    if (work.allocate((size_t) workValues) == EKX_OK &&
+        cells.allocate((size_t) cellValues) == EKX_OK)
+    {
+        return true;
+    }
+    (void) hipGetLastError();
+    work.release();
+    cells.release();
+    return false;
+}
+
+// Slowness range of a model, and whether the band kernel's unscaled square
+// roots cover it on a grid: h s within [2^-345, 2^500] (2^-700 <= hs0 hs0,
+// and no determinant overflows).
+struct Range2D
+{
+    double lo = std::numeric_limits<double>::infinity(), hi = 0;
+    void add(double v)
+    {
+        lo = std::min(lo, v);
+        hi = std::max(hi, v);
+    }
+    bool scaled(const ekx_geometry2d &g) const
+    {
+        return std::min(g.dx, g.dz)*lo >= 0x1p-345 &&
+               std::max(g.dx, g.dz)*hi <= 0x1p500;
+    }
+};
+
 std::string f2s(double v) { return std::to_string(v); }
 
 struct Loc2D
@@ -128,6 +163,13 @@ static Problem2D problem2d(const ekx_geometry2d &g, const ekx_solver_options &o)
     p.dz_dx = g.dz/g.dx;
     p.cosTheta = g.dx/std::hypot(g.dx, g.dz);
     p.sinTheta = g.dz/std::hypot(g.dx, g.dz);
+    p.dxinv = 1/g.dx;
+    p.dzinv = 1/g.dz;
+    p.hx2inv = 1/(g.dx*g.dx);
+    p.hz2inv = 1/(g.dz*g.dz);
+    p.twoOverH = 2/g.dx;
+    p.twoOverH2 = 2/(g.dx*g.dx);
+    p.halfOverH2 = 1/(2*(g.dx*g.dx));
     return p;
 }
 
@@ -174,12 +216,15 @@ struct ekx_solver2d
     Loc2D source{};
     std::vector<Loc2D> stations;
     Buf<double> S, T, stationOut, stationX, stationZ;
+    // band kernel: skewed travel times and cells (empty: level kernel)
+    Buf<double> W, C;
     Buf<int> stationCX, stationCZ;
     Buf<Problem2D> dProblem;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool initialized = false, haveModel = false, haveSource = false;
     bool haveField = false;
+    bool scaled = false;            // the model suits the band kernel
     std::vector<double> stationTimes;
     // travel-time gradient (2 values per node) of the current field
     Buf<double> G;
@@ -192,6 +237,17 @@ struct ekx_solver2d
         if (stream) { (void) hipStreamDestroy(stream); }
     }
 };
+
+// The band kernel's cells from the model in S.
+static ekx_status skew_model(ekx_solver2d *h)
+{
+    if (h->C.ptr)
+    {
+        EKX2_HIP(launch_skew_cells2d(h->geometry.nx, h->geometry.nz,
+                                     h->S.ptr, h->C.ptr, h->stream));
+    }
+    return EKX_OK;
+}
 
 static ekx_status require2d(const ekx_solver2d *h)
 {
@@ -251,6 +307,11 @@ ekx_status ekx_solver2d_initialize(ekx_solver2d *h,
         EKX2_CHECK(h->S.allocate((size_t) (g->nx - 1)*(g->nz - 1)));
         EKX2_CHECK(h->T.allocate((size_t) g->nx*g->nz));
         EKX2_CHECK(h->dProblem.allocate(1));
+        const bool bands = fits_bands2d(g->nx, g->nz);
+        allocate_bands(h->W, bands ? band_values2d(g->nx, g->nz) : 0, h->C,
+                       bands ? cell_values2d(g->nx, g->nz) : 0);
+        p.wOffset = 0;
+        p.cOffset = 0;
         EKX2_HIP(hipMemsetAsync(h->T.ptr, 0, h->T.count*sizeof(double),
                                 h->stream));
         EKX2_HIP(hipStreamSynchronize(h->stream));
@@ -275,15 +336,19 @@ ekx_status ekx_solver2d_set_slowness(ekx_solver2d *h, int64_t n,
             return fail2(EKX_EINVAL, "Number of cells = " + std::to_string(n) +
                                          " must equal " + std::to_string(nCell));
         }
+        Range2D range;
         for (int64_t i = 0; i < n; ++i)
         {
             if (!(s[i] > 0))
             {
                 return fail2(EKX_EINVAL, "Non-positive slowness detected");
             }
+            range.add(s[i]);
         }
+        h->scaled = range.scaled(h->geometry);
         EKX2_HIP(hipMemcpyAsync(h->S.ptr, s, (size_t) n*sizeof(double),
                                 hipMemcpyHostToDevice, h->stream));
+        EKX2_CHECK(skew_model(h));
         EKX2_HIP(hipStreamSynchronize(h->stream));
         h->haveModel = true;
         return EKX_OK;
@@ -309,19 +374,24 @@ ekx_status ekx_solver2d_set_nodal_velocities(ekx_solver2d *h, int64_t n,
         {
             return fail2(EKX_EINVAL, "unknown ordering");
         }
+        Range2D range;
         for (int64_t i = 0; i < n; ++i)
         {
             if (!(v[i] > 0))
             {
                 return fail2(EKX_EINVAL, "Non-positive velocities detected");
             }
+            range.add(1/v[i]);
         }
+        // (a cell's slowness is 4 over the sum of its corners' velocities)
+        h->scaled = range.scaled(h->geometry);
         Buf<double> dv;
         EKX2_CHECK(dv.allocate((size_t) n));
         EKX2_HIP(hipMemcpyAsync(dv.ptr, v, (size_t) n*sizeof(double),
                                 hipMemcpyHostToDevice, h->stream));
         EKX2_HIP(launch_nodal_to_cell2d(h->geometry.nx, h->geometry.nz, dv.ptr,
                                         ordering, h->S.ptr, h->stream));
+        EKX2_CHECK(skew_model(h));
         EKX2_HIP(hipStreamSynchronize(h->stream));
         h->haveModel = true;
         return EKX_OK;
@@ -417,7 +487,8 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
                                 hipMemcpyHostToDevice, h->stream));
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
         EKX2_HIP(launch_solve2d(h->dProblem.ptr, 1, h->geometry.nz, h->T.ptr,
-                                h->S.ptr, h->stream));
+                                h->S.ptr, h->scaled ? h->W.ptr : nullptr,
+                                h->C.ptr, h->stream));
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         const int ns = (int) h->stations.size();
         if (ns > 0)
@@ -565,6 +636,9 @@ struct ekx_batch2d
     std::vector<ekx_geometry2d> geoms;
     std::vector<Problem2D> problems;
     Buf<double> S, T;
+    // band kernel: skewed travel times per problem and cells per model
+    // (empty: level kernel)
+    Buf<double> W, C;
     Buf<Problem2D> dProblems;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -631,8 +705,10 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
         h->problems.assign(n, Problem2D{});
         // models: one device copy per distinct host pointer
         std::vector<const double *> models;
-        std::vector<int64_t> modelOffset;
-        int64_t tTotal = 0, sTotal = 0;
+        std::vector<int64_t> modelOffset, cellOffset;
+        std::vector<Range2D> ranges;
+        int64_t tTotal = 0, sTotal = 0, wTotal = 0, cTotal = 0;
+        bool bands = true;
         h->maxNz = 0;
         for (int i = 0; i < n; ++i)
         {
@@ -659,8 +735,10 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
             if (m == models.size())
             {
                 // a new model: every cell positive (checked once per model)
+                Range2D range;
                 for (int64_t c = 0; c < nCell; ++c)
                 {
+                    range.add(in[i].slowness[c]);
                     if (!(in[i].slowness[c] > 0))
                     {
                         return fail2(EKX_EINVAL, "problem " + std::to_string(i) +
@@ -669,8 +747,11 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
                     }
                 }
                 models.push_back(in[i].slowness);
+                ranges.push_back(range);
                 modelOffset.push_back(sTotal);
                 sTotal += nCell;
+                cellOffset.push_back(cTotal);
+                cTotal += cell_values2d(g.nx, g.nz);
             }
             else
             {
@@ -689,6 +770,10 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
             p.sOffset = modelOffset[m];
             p.tOffset = tTotal;
             tTotal += (int64_t) g.nx*g.nz;
+            p.cOffset = cellOffset[m];
+            p.wOffset = wTotal;
+            wTotal += band_values2d(g.nx, g.nz);
+            bands = bands && fits_bands2d(g.nx, g.nz) && ranges[m].scaled(g);
             h->geoms[i] = g;
             h->problems[i] = p;
             h->maxNz = std::max(h->maxNz, g.nz);
@@ -696,21 +781,29 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
         EKX2_CHECK(h->S.allocate((size_t) sTotal));
         EKX2_CHECK(h->T.allocate((size_t) tTotal));
         EKX2_CHECK(h->dProblems.allocate((size_t) n));
+        bands = allocate_bands(h->W, bands ? wTotal : 0, h->C,
+                               bands ? cTotal : 0) && bands;
         for (size_t m = 0; m < models.size(); ++m)
         {
-            int64_t nCell = 0;
+            ekx_geometry2d g{};
             for (int i = 0; i < n; ++i)
             {
                 if (in[i].slowness == models[m])
                 {
-                    nCell = (int64_t) (in[i].geometry.nx - 1)*
-                            (in[i].geometry.nz - 1);
+                    g = in[i].geometry;
                     break;
                 }
             }
+            const int64_t nCell = (int64_t) (g.nx - 1)*(g.nz - 1);
             EKX2_HIP(hipMemcpyAsync(h->S.ptr + modelOffset[m], models[m],
                                     (size_t) nCell*sizeof(double),
                                     hipMemcpyHostToDevice, h->stream));
+            if (bands)
+            {
+                EKX2_HIP(launch_skew_cells2d(
+                    g.nx, g.nz, h->S.ptr + modelOffset[m],
+                    h->C.ptr + cellOffset[m], h->stream));
+            }
         }
         EKX2_HIP(hipMemcpyAsync(h->dProblems.ptr, h->problems.data(),
                                 (size_t) n*sizeof(Problem2D),
@@ -729,7 +822,7 @@ ekx_status ekx_batch2d_solve(ekx_batch2d *h)
         const int n = (int) h->problems.size();
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
         EKX2_HIP(launch_solve2d(h->dProblems.ptr, n, h->maxNz, h->T.ptr,
-                                h->S.ptr, h->stream));
+                                h->S.ptr, h->W.ptr, h->C.ptr, h->stream));
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         EKX2_HIP(hipEventSynchronize(h->ev1));
         float ms = 0;

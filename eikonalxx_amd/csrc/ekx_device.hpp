@@ -221,8 +221,56 @@ struct Problem2D
     double srcOffX, srcOffZ;
     double srcSlowness;
     double dx_dz, dz_dx, cosTheta, sinTheta;  // solver2d.hpp:41-46
+    // quotients of the factored update (h: dx on a uniform grid)
+    double dxinv, dzinv, hx2inv, hz2inv;      // 1/dx, 1/dz, 1/dx^2, 1/dz^2
+    double twoOverH, twoOverH2, halfOverH2;   // 2/h, 2/h^2, 1/(2 h^2)
     int64_t tOffset;
     int64_t sOffset;
+    // band kernel: first values of the skewed travel times and cells
+    int64_t wOffset;
+    int64_t cOffset;
 };
+
+// Band kernel of the 2D solve: bands of 64 rows, and per band step records
+// of 64 travel times (two buffers) and of 65 cells (one set per sweep
+// direction).  Lane i is i columns behind lane 0, so nx + 63 steps, rounded
+// up to whole groups of 8, pass every column through a band.  Lanes outside
+// the grid's columns write too: up to 63 + 7 records on either side of the
+// nx + 63 that hold nodes, whose padding also takes the prefetch.
+constexpr int kMaxBands2d = 16;
+constexpr int kCellRecord2d = 65;
+constexpr int kBandPad2d = 72;
+
+__host__ __device__ inline int bands2d(int nz) { return (nz + 63)/64; }
+
+__host__ __device__ inline int band_records2d(int nx)
+{
+    return nx + 63 + 2*kBandPad2d;
+}
+
+// travel-time work of one problem
+__host__ __device__ inline int64_t band_values2d(int nx, int nz)
+{
+    return 2*(int64_t) bands2d(nz)*band_records2d(nx)*64;
+}
+
+// cell records of one band and sweep direction: the steps rounded up to
+// whole groups of 8, and the group that the prefetch runs ahead
+__host__ __device__ inline int cell_steps2d(int nx)
+{
+    return (nx + 63 + 7)/8*8 + 8;
+}
+
+__host__ __device__ inline int64_t cell_values2d(int nx, int nz)
+{
+    return 4*(int64_t) bands2d(nz)*cell_steps2d(nx)*kCellRecord2d;
+}
+
+// Grids that the band kernel takes: at most 16 bands (the waves of a
+// workgroup), and lane offsets that stay well within 32 bits.
+__host__ __device__ inline bool fits_bands2d(int nx, int nz)
+{
+    return nz <= 64*kMaxBands2d && nx <= 65536;
+}
 
 } // namespace ekx

@@ -144,12 +144,17 @@ hipError_t launch_layered_velocity(int nx, int ny, int nz, int nLayers,
                                    double mean, double sd, const double *g,
                                    double *v, hipStream_t stream);
 
-// The whole 2D solve, one 256-thread workgroup per problem: the latest
-// levels in LDS when every problem has at most 256 rows (maxNz), else
-// memory only, with a barrier per level.
+// The whole 2D solve, one workgroup per problem.  work and cells: the band
+// kernel's buffers (Problem2D::wOffset, cOffset; every grid within
+// fits_bands2d, at most maxNz rows, and h s within [2^-345, 2^500]); work
+// null: the level kernel.
 hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
                           int maxNz, double *T, const double *S,
+                          double *work, const double *cells,
                           hipStream_t stream);
+// The band kernel's cell records of one model (cell_values2d values).
+hipError_t launch_skew_cells2d(int nx, int nz, const double *s, double *out,
+                               hipStream_t stream);
 hipError_t launch_stations2d(const Problem2D *dProblem, int n,
                              const double *xOff, const double *zOff,
                              const int *cellX, const int *cellZ,

@@ -8,263 +8,751 @@
 // earlier levels, so the result equals the serial loop of
 // Solver2DSweep::updateFSM (include/private/solver2d.hpp:203-327).
 //
-// One workgroup owns one problem for the whole solve; levels are separated
-// by workgroup barriers, and for grids of up to 256 rows the last three
-// levels of a sweep live in LDS.  2D grids are small (config of the
-// reference's own 2D tests: 201 x 201), so one launch covers the entire
-// solve.
+// One workgroup owns one problem for the whole solve, so one launch covers
+// it: the band kernel (64 rows per wave) up to 1024 rows, the level kernel
+// (global memory, a block barrier per level) for what it does not take.
 #include "ekx_kernels.hpp"
+#include "ekx_sqrt.hpp"
+
+#include <type_traits>
 
 namespace ekx
 {
+
+// Distance of node (ix, iz) from the source.
+__device__ __forceinline__ double distance2d(int ix, int iz, double dx,
+                                             double dz, double xs, double zs)
+{
+    double x = ix*dx;
+    double z = iz*dz;
+    double deltaX = x - xs;
+    double deltaZ = z - zs;
+    return ::hypot(deltaX, deltaZ);
+}
 
 // computeAnalyticalTravelTime 2D (solverUtilities2d.hpp:159-174).
 __device__ __forceinline__ double analytic_time2d(int ix, int iz, double dx,
                                                   double dz, double xs,
                                                   double zs, double slow)
 {
-    double x = ix*dx;
-    double z = iz*dz;
-    double deltaX = x - xs;
-    double deltaZ = z - zs;
-    double distance = ::hypot(deltaX, deltaZ);
-    return slow*distance;
+    return slow*distance2d(ix, iz, dx, dz, xs, zs);
 }
 
-// (solverUtilities2d.hpp:192-215)
+// (solverUtilities2d.hpp:192-215), given the distance r
 __device__ __forceinline__ void analytic_time_deriv2d(
     int ix, int iz, double dx, double dz, double xs, double zs, double slow,
-    double &t, double &dtdx, double &dtdz)
+    double r, double &t, double &dtdx, double &dtdz)
 {
     double x = ix*dx;
     double z = iz*dz;
     double deltaX = x - xs;
     double deltaZ = z - zs;
-    double distance = ::hypot(deltaX, deltaZ);
-    t = slow*distance;
+    t = slow*r;
     dtdx = 0;
     dtdz = 0;
-    if (distance > 0)
+    if (r > 0)
     {
-        dtdx = (slow*deltaX)/distance;
-        dtdz = (slow*deltaZ)/distance;
+        dtdx = (slow*deltaX)/r;
+        dtdz = (slow*deltaZ)/r;
     }
 }
 
 constexpr double kSqrt1_2 = 0.70710678118654752440;
 
-// finiteDifference, uniform grid (solverUtilities2d.hpp:345-472).
-__device__ double fd2d_uniform(const Problem2D &p, int ix, int iz, int signX,
-                               int signZ, int ixShift, int izShift,
-                               double s0, double s1, double s3, double t1,
-                               double t2, double t3)
+// v where valid, else a number above HUGE (HUGE's next high word): one
+// select instead of two, the low word does not matter.
+__device__ __forceinline__ double valid_or_huge(double v, bool valid)
 {
-    const double huge = kHuge;
-    const double h = p.dx;
-    const double sourceSlowness = p.srcSlowness;
-    double tUpd = huge;
-    double t0x = t1 + h*fmin(s0, s3);
-    double t0z = t3 + h*fmin(s0, s1);
-    double t0Update1 = fmin(t0x, t0z);
-    double hs0 = h*s0;
-    double dTx = t3 - t2;
-    double dTz = t1 - t2;
-    double sx = kSqrt1_2*s0;
-    double sz = kSqrt1_2*s0;
-    if (abs(p.srcCellX - ix) > p.radius || abs(p.srcCellZ - iz) > p.radius)
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t hi = valid ? (uint32_t) (u >> 32) : 0x4202A060u;
+    return __builtin_bit_cast(double,
+                              ((uint64_t) hi << 32) | (uint32_t) u);
+}
+
+// The Cartesian part of finiteDifference, uniform grid
+// (solverUtilities2d.hpp:345-400).  Branch-free: every candidate is
+// evaluated and the invalid ones are replaced by a number above HUGE, so
+// the three square roots of a node run side by side; along a front nearly
+// every wave has lanes that need each of them.  deta and detb of the
+// reference are positive whenever their other conditions hold (0 <= dT <=
+// h s0 / sqrt 2), so their own tests are left out; 2 (hs0 hs0) is exact, so
+// the fused form of detc rounds once like the reference's subtraction.
+//
+// SCALED (the models the band kernel gets): 2^-700 <= hs0 hs0 in every cell, so every valid
+// determinant is in the range of sqrt_normal_range: deta and detb are at
+// least about half of hs0 hs0, and a positive detc = 2 q - c c is q-sized
+// or, where the terms cancel, a multiple of their last place, 2^-53 q.
+template <bool SCALED>
+__device__ __forceinline__ double cartesian2d_uniform(
+    double h, double s0, double s1, double s3, double t1, double t2,
+    double t3)
+{
+    double best = fmin(t1 + h*fmin(s0, s3), t3 + h*fmin(s0, s1));
+    const double hs0 = h*s0;
+    const double q = hs0*hs0;
+    const double dTx = t3 - t2;
+    const double dTz = t1 - t2;
+    const double hs = h*(kSqrt1_2*s0);
+    const double deta = q - dTz*dTz;
+    const double detb = q - dTx*dTx;
+    const double dtCross = t1 - t3;
+    const double detc = fma(2.0, q, -(dtCross*dtCross));
+    const bool ca = dTz >= 0 && dTz <= hs;
+    const bool cb = dTx >= 0 && dTx <= hs;
+    const bool cc = dTx >= 0 && dTz >= 0 && detc > 0 && t3 <= t1 + hs0 &&
+                    t1 <= t3 + hs0;
+    double ra, rb, rc;
+    if constexpr (SCALED)
     {
-        double t0a = huge;
-        double deta = hs0*hs0 - dTz*dTz;
-        if (dTz >= 0 && deta >= 0 && dTz <= h*sz)
-        {
-            t0a = t1 + h*::sqrt(deta);
-        }
-        double t0b = huge;
-        double detb = hs0*hs0 - dTx*dTx;
-        if (dTx >= 0 && detb >= 0 && dTx <= h*sx)
-        {
-            t0b = t3 + h*::sqrt(detb);
-        }
-        double t0Update2 = fmin(t0a, t0b);
-        double dtCross = t1 - t3;
-        double detc = 2*(hs0*hs0) - dtCross*dtCross;
-        double t0Update3 = huge;
-        if (dTx >= 0 && dTz >= 0 && detc > 0 &&
-            t3 <= t1 + hs0 && t1 <= t3 + hs0)
-        {
-            t0Update3 = t2 + ::sqrt(detc);
-        }
-        tUpd = fmin(fmin(t0Update1, t0Update2), t0Update3);
+        ra = sqrt_normal_range(deta);
+        rb = sqrt_normal_range(detb);
+        rc = sqrt_normal_range(detc);
     }
     else
     {
-        double t0Update3 = huge;
-        if (dTx >= 0 && dTz >= 0 && t1 < t3 + hs0 && t3 < t1 + hs0)
-        {
-            double dt0dx, dt0dz, t0;
-            const double xs = p.srcOffX, zs = p.srcOffZ;
-            analytic_time_deriv2d(ix, iz, h, h, xs, zs, sourceSlowness, t0,
-                                  dt0dx, dt0dz);
-            double tau1 = t1 - analytic_time2d(ix + ixShift, iz, h, h, xs, zs,
-                                               sourceSlowness);
-            double tau2 = t2 - analytic_time2d(ix + ixShift, iz + izShift, h,
-                                               h, xs, zs, sourceSlowness);
-            double tau3 = t3 - analytic_time2d(ix, iz + izShift, h, h, xs, zs,
-                                               sourceSlowness);
-            dt0dx = signX*dt0dx;
-            dt0dz = signZ*dt0dz;
-            double tauX = tau1 - tau3 + tau2;
-            double tauZ = tau3 - tau1 + tau2;
-            const double one = 1, two = 2, four = 4;
-            double h2 = h*h;
-            double a = one/h2;
-            double b = two/h*(dt0dx + dt0dz) - two/h2*tau2;
-            double c = one/(two*h2)*(tauX*tauX + tauZ*tauZ)
-                     - two/h*(dt0dx*tauX + dt0dz*tauZ)
-                     + two*(sourceSlowness*sourceSlowness - s0*s0);
-            double det = b*b - four*a*c;
-            if (det >= 0)
-            {
-                double tau = (-b + ::sqrt(det))/(two*a);
-                t0Update3 = t0 + tau;
-            }
-            if (t0Update3 < t1 || t0Update3 < t3) { t0Update3 = huge; }
-        }
-        tUpd = fmin(t0Update1, t0Update3);
+        ra = ::sqrt(ca ? deta : q);
+        rb = ::sqrt(cb ? detb : q);
+        rc = ::sqrt(cc ? detc : q);
     }
-    return tUpd;
+    best = fmin(best, valid_or_huge(t1 + h*ra, ca));
+    best = fmin(best, valid_or_huge(t3 + h*rb, cb));
+    return fmin(best, valid_or_huge(t2 + rc, cc));
 }
 
-// finiteDifference, non-uniform grid (solverUtilities2d.hpp:474-614).
-__device__ double fd2d_nonuniform(const Problem2D &p, int ix, int iz,
-                                  int signX, int signZ, int ixShift,
-                                  int izShift, double s0, double s1,
-                                  double s3, double t1, double t2, double t3)
+// The spacings and ratios of the Cartesian updates.
+struct Grid2D
 {
-    const double huge = kHuge;
+    double dx, dz, dx_dz, dz_dx, cosTheta, sinTheta;
+};
+
+__device__ __forceinline__ Grid2D grid2d(const Problem2D &p)
+{
+    return Grid2D{p.dx, p.dz, p.dx_dz, p.dz_dx, p.cosTheta, p.sinTheta};
+}
+
+// The same, non-uniform grid (solverUtilities2d.hpp:474-560).
+template <bool SCALED>
+__device__ __forceinline__ double cartesian2d_nonuniform(
+    const Grid2D &p, double s0, double s1, double s3, double t1, double t2,
+    double t3)
+{
     const double dx = p.dx, dz = p.dz;
     const double dx_dz = p.dx_dz, dz_dx = p.dz_dx;
     const double cosTheta = p.cosTheta, sinTheta = p.sinTheta;
-    const double sourceSlowness = p.srcSlowness;
-    double tUpd = huge;
+    double best = fmin(t1 + dx*fmin(s0, s3), t3 + dz*fmin(s0, s1));
+    const double dTx = t3 - t2;
+    const double dTz = t1 - t2;
+    const double sx = cosTheta*s0;
+    const double sz = sinTheta*s0;
+    const double hxs0 = dx*s0;
+    const double hzs0 = dz*s0;
+    const double deta = hzs0*hzs0 - dTz*dTz;
+    const double detb = hxs0*hxs0 - dTx*dTx;
+    const double tildeTx = t1 - t3 + t2;
+    const double tildeTz = t3 - t1 + t2;
+    const double dtCross = t1 - t3;
+    const double detc = hxs0*hxs0 + hzs0*hzs0 - dtCross*dtCross;
+    const bool ca = dTz >= 0 && deta >= 0 && dTz <= dz*sz;
+    const bool cb = dTx >= 0 && detb >= 0 && dTx <= dx*sx;
+    const bool cc = dTx >= 0 && dTz >= 0 && detc > 0 && t1 < t3 + hzs0 &&
+                    t3 < t1 + hxs0;
+    double ra, rb, rc;
+    if constexpr (SCALED)
+    {
+        // With very unequal spacings a valid deta or detb can cancel to
+        // zero; the root then taken, 2^-500, adds nothing to t1 or t3,
+        // which are at least dT, about h s0 there.
+        ra = sqrt_normal_range(fmax(deta, 0x1p-1000));
+        rb = sqrt_normal_range(fmax(detb, 0x1p-1000));
+        rc = sqrt_normal_range(detc);
+    }
+    else
+    {
+        ra = ::sqrt(ca ? deta : 1.0);
+        rb = ::sqrt(cb ? detb : 1.0);
+        rc = ::sqrt(cc ? detc : 1.0);
+    }
+    best = fmin(best, valid_or_huge(t1 + dx_dz*ra, ca));
+    best = fmin(best, valid_or_huge(t3 + dz_dx*rb, cb));
+    double tc = tildeTx*dz_dx + tildeTz*dx_dz + 2*rc;
+    tc = (cosTheta*sinTheta)*tc;
+    // a negative candidate is dropped (t0Update3 < 0 of the reference)
+    return fmin(best, valid_or_huge(tc, cc && !(tc < 0)));
+}
+
+// A sweep's directions (bit 0: x decreasing, bit 1: z decreasing) and the
+// first node of each permuted axis that it updates: 1, or the source
+// quadrant in an initialisation sweep (getLoopLimits,
+// solverUtilities2d.hpp:1004-1053).
+struct Sweep2D
+{
+    int negX, negZ, signX, signZ, izShift, jx0, jz0;
+};
+
+__device__ __forceinline__ Sweep2D make_sweep2d(const Problem2D &p, int sweep,
+                                                int initialize)
+{
+    Sweep2D s;
+    s.negX = sweep & 1;
+    s.negZ = (sweep >> 1) & 1;
+    s.signX = s.negX ? -1 : 1;
+    s.signZ = s.negZ ? -1 : 1;
+    s.izShift = s.negZ ? 1 : -1;
+    s.jx0 = 1;
+    s.jz0 = 1;
+    if (initialize)
+    {
+        s.jx0 = s.negX ? max(p.nx - 2 - p.srcCellX, 1) : max(p.srcCellX, 1);
+        s.jz0 = s.negZ ? max(p.nz - 2 - p.srcCellZ, 1) : max(p.srcCellZ, 1);
+    }
+    return s;
+}
+
+// What the factored update and the source cell need, by value: the band
+// kernel keeps it in scalar registers (through the descriptor, every step
+// would load it again).
+struct Source2D
+{
+    double dx, dz;              // dz: dx on a uniform grid
+    double xs, zs, slowness;
+    double dxinv, dzinv, hx2inv, hz2inv, twoOverH, twoOverH2, halfOverH2;
+    int cellX, cellZ, radius;
+    bool uniform;
+};
+
+__device__ __forceinline__ Source2D source2d(const Problem2D &p)
+{
+    return Source2D{p.dx, p.uniform ? p.dx : p.dz, p.srcOffX, p.srcOffZ,
+                    p.srcSlowness, p.dxinv, p.dzinv, p.hx2inv, p.hz2inv,
+                    p.twoOverH, p.twoOverH2, p.halfOverH2, p.srcCellX,
+                    p.srcCellZ, p.radius, p.uniform != 0};
+}
+
+// Distance of node (ix, iz) from the source.
+__device__ __forceinline__ double distance2d(const Source2D &s, int ix, int iz)
+{
+    return distance2d(ix, iz, s.dx, s.dz, s.xs, s.zs);
+}
+
+// finiteDifference near the source: the analytic time factored out, uniform
+// grid (solverUtilities2d.hpp:400-472) and non-uniform (:560-614).  r0..r3:
+// the distances from the source of the node and of its neighbours 1, 2
+// and 3; the
+// quotients of the spacings come from the descriptor.
+__device__ __forceinline__ double factored2d(
+    const Source2D &p, const Sweep2D &w, int ix, int iz, double s0,
+    double s1, double s3, double t1, double t2, double t3, double r0,
+    double r1, double r2, double r3)
+{
+    const double huge = kHuge;
+    const double dx = p.dx, dz = p.dz;
+    const double sourceSlowness = p.slowness;
     double t0x = t1 + dx*fmin(s0, s3);
     double t0z = t3 + dz*fmin(s0, s1);
     double t0Update1 = fmin(t0x, t0z);
     double dTx = t3 - t2;
     double dTz = t1 - t2;
-    double sx = cosTheta*s0;
-    double sz = sinTheta*s0;
     double hxs0 = dx*s0;
     double hzs0 = dz*s0;
-    if (abs(p.srcCellX - ix) > p.radius || abs(p.srcCellZ - iz) > p.radius)
+    double t0Update3 = huge;
+    if (dTx >= 0 && dTz >= 0 && t1 < t3 + hzs0 && t3 < t1 + hxs0)
     {
-        double t0a = huge;
-        double deta = hzs0*hzs0 - dTz*dTz;
-        if (dTz >= 0 && deta >= 0 && dTz <= dz*sz)
+        double dt0dx, dt0dz, t0;
+        analytic_time_deriv2d(ix, iz, dx, dz, p.xs, p.zs,
+                              sourceSlowness, r0, t0, dt0dx, dt0dz);
+        double tau1 = t1 - sourceSlowness*r1;
+        double tau2 = t2 - sourceSlowness*r2;
+        double tau3 = t3 - sourceSlowness*r3;
+        dt0dx = w.signX*dt0dx;
+        dt0dz = w.signZ*dt0dz;
+        double tauX = tau1 - tau3 + tau2;
+        double tauZ = tau3 - tau1 + tau2;
+        const double two = 2, four = 4;
+        double a, b, c;
+        if (p.uniform)
         {
-            t0a = t1 + dx_dz*::sqrt(deta);
+            a = p.hx2inv;
+            b = p.twoOverH*(dt0dx + dt0dz) - p.twoOverH2*tau2;
+            c = p.halfOverH2*(tauX*tauX + tauZ*tauZ)
+              - p.twoOverH*(dt0dx*tauX + dt0dz*tauZ)
+              + two*(sourceSlowness*sourceSlowness - s0*s0);
         }
-        double t0b = huge;
-        double detb = hxs0*hxs0 - dTx*dTx;
-        if (dTx >= 0 && detb >= 0 && dTx <= dx*sx)
+        else
         {
-            t0b = t3 + dz_dx*::sqrt(detb);
+            a = p.hx2inv + p.hz2inv;
+            b = four*(p.dxinv*dt0dx + p.dzinv*dt0dz)
+              - two*(tauX*p.hx2inv + tauZ*p.hz2inv);
+            c = (tauX*tauX)*p.hx2inv + (tauZ*tauZ)*p.hz2inv
+              - four*((dt0dx*tauX)*p.dxinv + (dt0dz*tauZ)*p.dzinv)
+              + four*(sourceSlowness*sourceSlowness - s0*s0);
         }
-        double t0Update2 = fmin(t0a, t0b);
-        double dxdz_dx2_p_dz2 = cosTheta*sinTheta;
-        double tildeTx = t1 - t3 + t2;
-        double tildeTz = t3 - t1 + t2;
-        double dtCross = t1 - t3;
-        double detc = hxs0*hxs0 + hzs0*hzs0 - dtCross*dtCross;
-        double t0Update3 = huge;
-        if (dTx >= 0 && dTz >= 0 && detc > 0 &&
-            t1 < t3 + hzs0 && t3 < t1 + hxs0)
+        double det = b*b - four*a*c;
+        if (det >= 0)
         {
-            t0Update3 = tildeTx*dz_dx + tildeTz*dx_dz + 2*::sqrt(detc);
-            t0Update3 = dxdz_dx2_p_dz2*t0Update3;
+            double tau = (-b + ::sqrt(det))/(two*a);
+            t0Update3 = t0 + tau;
         }
-        if (t0Update3 < 0) { t0Update3 = huge; }
-        tUpd = fmin(fmin(t0Update1, t0Update2), t0Update3);
+        if (t0Update3 < t1 || t0Update3 < t3) { t0Update3 = huge; }
     }
-    else
-    {
-        double t0Update3 = huge;
-        if (dTx >= 0 && dTz >= 0 && t1 < t3 + hzs0 && t3 < t1 + hxs0)
-        {
-            double dt0dx, dt0dz, t0;
-            const double xs = p.srcOffX, zs = p.srcOffZ;
-            analytic_time_deriv2d(ix, iz, dx, dz, xs, zs, sourceSlowness, t0,
-                                  dt0dx, dt0dz);
-            double tau1 = t1 - analytic_time2d(ix + ixShift, iz, dx, dz, xs,
-                                               zs, sourceSlowness);
-            double tau2 = t2 - analytic_time2d(ix + ixShift, iz + izShift, dx,
-                                               dz, xs, zs, sourceSlowness);
-            double tau3 = t3 - analytic_time2d(ix, iz + izShift, dx, dz, xs,
-                                               zs, sourceSlowness);
-            dt0dx = signX*dt0dx;
-            dt0dz = signZ*dt0dz;
-            double tauX = tau1 - tau3 + tau2;
-            double tauZ = tau3 - tau1 + tau2;
-            const double one = 1, two = 2, four = 4;
-            double hx2inv = one/(dx*dx);
-            double hz2inv = one/(dz*dz);
-            double dxinv = one/dx;
-            double dzinv = one/dz;
-            double a = hx2inv + hz2inv;
-            double b = four*(dxinv*dt0dx + dzinv*dt0dz)
-                     - two*(tauX*hx2inv + tauZ*hz2inv);
-            double c = (tauX*tauX)*hx2inv + (tauZ*tauZ)*hz2inv
-                     - four*((dt0dx*tauX)*dxinv + (dt0dz*tauZ)*dzinv)
-                     + four*(sourceSlowness*sourceSlowness - s0*s0);
-            double det = b*b - four*a*c;
-            if (det >= 0)
-            {
-                double tau = (-b + ::sqrt(det))/(two*a);
-                t0Update3 = t0 + tau;
-            }
-            if (t0Update3 < t1 || t0Update3 < t3) { t0Update3 = huge; }
-        }
-        tUpd = fmin(t0Update1, t0Update3);
-    }
-    return tUpd;
+    return fmin(t0Update1, t0Update3);
 }
 
-// One sweep of one problem, levels separated by block barriers.
+__device__ __forceinline__ bool in_factored_box2d(const Source2D &p, int ix,
+                                                  int iz)
+{
+    return !(abs(p.cellX - ix) > p.radius || abs(p.cellZ - iz) > p.radius);
+}
+
+// ---------------------------------------------------------------------------
+// Band kernel: one workgroup solves one problem.  The grid's rows are cut
+// into bands of 64 (grid rows 64 m .. 64 m + 63), one wave each, for the
+// whole solve.  In the sweep's permuted frame lane i owns row i of its band
+// and at step t works on column t - i: its x neighbour is its own previous
+// value, its z neighbour the value that lane i - 1 computed one step
+// earlier, one cross-lane move (wave_shr) away.  A band's last row goes to
+// the next band through a ring in LDS; the next band runs kLag2d groups of
+// kGroup2d steps behind, and one block barrier per group is all the
+// synchronisation there is.  The lags are constant, so every wave derives
+// its start in each sweep from the sizes alone, and a sweep that keeps the
+// z direction follows the one before it without a gap.
+//
+// What bounds it: the chain of nx + nz dependent node updates per sweep, on
+// waves that have a SIMD to themselves (up to 4 bands): such a wave issues
+// one instruction every 4 cycles, scalar ones included, so a step costs its
+// instruction count, not its latency.  Hence the group kinds below (what a
+// group cannot meet costs it nothing), fixed strides (immediate offsets
+// instead of address arithmetic) and stores without a mask.
+//
+// Times between sweeps: step records of 64 values, in the step and lane
+// order of the sweep that reads them, so that every access of the step loop
+// is coalesced.  The x direction reverses with every sweep, so a sweep
+// always writes its records backwards, into the other of two buffers; a
+// lane outside the grid writes a padding element (its column is outside
+// the reader's grid too).  The last sweep writes the natural-order field.
+//
+// 201 x 201, 2 iterations: LDS-level kernel 2.81 ms, this kernel 1.24 ms;
+// 701 x 523, 3 iterations: 31.4 ms (memory-only levels) and 9.4 ms.
+// ---------------------------------------------------------------------------
+constexpr int kBand2d = 64;
+constexpr int kGroup2d = 8;
+// groups between a band and the next: the first column of the band's last
+// row is done at step 63, i.e. within group 8
+constexpr int kLag2d = kBand2d/kGroup2d + 1;
+// columns of a band's last row kept for the next band: written up to 16
+// ahead of the reader
+constexpr int kRing2d = 64;
+
+// Doubles in device memory: through generic pointers the accesses would be
+// FLAT ones, which the waits for LDS also wait for.
+using GlobalDouble = __attribute__((address_space(1))) double;
+
+// lane i's value of lane i - 1; lane 0 takes `first`
+__device__ __forceinline__ double from_previous_lane(double v, double first)
+{
+    constexpr int kWaveShr1 = 0x138;
+    const uint64_t a = __builtin_bit_cast(uint64_t, v);
+    const uint64_t f = __builtin_bit_cast(uint64_t, first);
+    const uint32_t lo = (uint32_t) __builtin_amdgcn_update_dpp(
+        (int) (uint32_t) f, (int) (uint32_t) a, kWaveShr1, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t) __builtin_amdgcn_update_dpp(
+        (int) (f >> 32), (int) (a >> 32), kWaveShr1, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
+}
+
+// LDS accesses done, then the barrier: values exchanged between waves are
+// in LDS, global accesses stay in flight.  The compiler treats both
+// builtins as touching no memory, so empty asm statements keep the accesses
+// on their side.
+__device__ __forceinline__ void group_barrier()
+{
+    __asm__ __volatile__("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();
+    __asm__ __volatile__("" ::: "memory");
+}
+
+// What a group of steps can meet.  kFull: every lane is on a column that
+// the sweep updates, none in the factored box.  kIdle: no lane updates
+// anything.  kAny: lanes enter or leave the columns.  kRare: kAny in the
+// solve's first sweep (old times HUGE and the source cell's corners) or its
+// last one (writes the field), or with lanes in the factored box.
+enum Group2D { kFull, kIdle, kAny, kRare };
+
+// A band's wave within one sweep; AHEAD: steps that a record is loaded
+// ahead.
+template <int AHEAD>
+struct Band2D
+{
+    Source2D src;
+    Sweep2D w;
+    Grid2D grid;
+    int lane, iz, nx;
+    bool row;               // the lane's row is in the grid
+    uint32_t liveSpan;      // columns it updates (from jx0)
+    double floor;           // kFull: above HUGE in lanes that update nothing
+    bool first, last;       // the solve's first or last sweep
+    int boxLo, boxHi;       // steps with lanes in the box
+    int t;                  // first step of the next AHEAD
+    const GlobalDouble *old, *cells;    // records AHEAD steps ahead
+    GlobalDouble *out;
+    double cur, s1Prev, t3Prev, hand;
+    // in the box's steps: distances from the source of the lane's previous
+    // node and of that node's z neighbour
+    double r0, r3;
+    double T0[AHEAD], SA[AHEAD], SB[AHEAD];
+
+    // the records of steps t .. t + AHEAD - 1, which old and cells point at
+    __device__ __forceinline__ void load()
+    {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u)
+        {
+            T0[u] = old[u*kBand2d];
+            SA[u] = cells[u*kCellRecord2d];
+            SB[u] = cells[u*kCellRecord2d + 1];
+        }
+        old += AHEAD*kBand2d;
+        cells += AHEAD*kCellRecord2d;
+    }
+    // the first sweep's old time of the lane's node in column ix
+    __device__ __forceinline__ double start_time(int ix) const
+    {
+        const int ox = ix - src.cellX, oz = iz - src.cellZ;
+        double v = kHuge;
+        if (ox >= 0 && ox <= 1 && oz >= 0 && oz <= 1)
+        {
+            v = analytic_time2d(ix, iz, grid.dx, grid.dz, src.xs, src.zs,
+                                src.slowness);
+        }
+        return v;
+    }
+    template <bool UNIFORM>
+    __device__ __forceinline__ double cartesian(double s0, double s1,
+                                                double s3, double t1,
+                                                double t2, double t3) const
+    {
+        if constexpr (UNIFORM)
+        {
+            return cartesian2d_uniform<true>(grid.dx, s0, s1, s3, t1, t2,
+                                             t3);
+        }
+        else
+        {
+            return cartesian2d_nonuniform<true>(grid, s0, s1, s3, t1, t2,
+                                                t3);
+        }
+    }
+};
+
+// AHEAD steps.  ri: the previous band's last row (column t + u + 1 in
+// ri[u]); hp: where lane 63 leaves this band's.
+template <bool UNIFORM, Group2D KIND, int AHEAD>
+__device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
+                                           double *hp)
+{
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+    {
+        const double t3 = from_previous_lane(b.cur, b.hand);
+        b.hand = ri[u];
+        const double t1 = b.cur, t2 = b.t3Prev;
+        const double s0 = b.s1Prev, s1 = b.SA[u], s3 = b.SB[u];
+        double t0 = b.T0[u];
+        // the record AHEAD steps on, into the freed registers
+        b.T0[u] = b.old[u*kBand2d];
+        b.SA[u] = b.cells[u*kCellRecord2d];
+        b.SB[u] = b.cells[u*kCellRecord2d + 1];
+        b.t3Prev = t3;
+        b.s1Prev = s1;
+        const int jx = b.t + u - b.lane;
+        const int ix = b.w.negX ? b.nx - 1 - jx : jx;
+        if constexpr (KIND == kIdle) { b.cur = t0; }
+        else
+        {
+            double v = b.template cartesian<UNIFORM>(s0, s1, s3, t1, t2, t3);
+            if constexpr (KIND == kFull)
+            {
+                b.cur = fmin(fmax(v, b.floor), t0);
+            }
+            else
+            {
+                const bool live = (uint32_t) (jx - b.w.jx0) < b.liveSpan;
+                if constexpr (KIND == kRare)
+                {
+                    if (b.first) { t0 = b.start_time(ix); }
+                    if (b.t + u >= b.boxLo - 1 && b.t + u <= b.boxHi)
+                    {
+                        // the node's x neighbour is the lane's previous
+                        // node
+                        const double r1 = b.r0, r2 = b.r3;
+                        b.r0 = distance2d(b.src, ix, b.iz);
+                        b.r3 = distance2d(b.src, ix, b.iz + b.w.izShift);
+                        if (live && in_factored_box2d(b.src, ix, b.iz))
+                        {
+                            v = factored2d(b.src, b.w, ix, b.iz, s0, s1, s3,
+                                           t1, t2, t3, b.r0, r1, r2, b.r3);
+                        }
+                    }
+                }
+                b.cur = live && v < t0 ? v : t0;
+            }
+        }
+        hp[u] = b.cur;
+        if (KIND == kRare && b.last)
+        {
+            if (b.row && (uint32_t) jx < (uint32_t) b.nx)
+            {
+                b.out[ix] = b.cur;
+            }
+        }
+        else { b.out[-u*kBand2d] = b.cur; }
+    }
+    b.t += AHEAD;
+    b.old += AHEAD*kBand2d;
+    b.cells += AHEAD*kCellRecord2d;
+    if (!(KIND == kRare && b.last)) { b.out -= AHEAD*kBand2d; }
+}
+
+// One sweep of one band.  old: record of step 0 (this lane's value); cells:
+// the sweep's cell records; out: this lane's result of step 0, the next
+// steps' each one record before it (last: the start of the lane's row in
+// the field).
+template <bool UNIFORM, int AHEAD>
+__device__ __forceinline__ void band_sweep(
+    const Problem2D &p, const Sweep2D &w, int band, int lane, int groups,
+    bool first, bool last, const GlobalDouble *old, const GlobalDouble *cells,
+    GlobalDouble *out, const double *ringIn, double *ringOut, double *sink)
+{
+    const int nx = p.nx, nz = p.nz;
+    const int iz = kBand2d*band + (w.negZ ? kBand2d - 1 - lane : lane);
+    const int jz = w.negZ ? nz - 1 - iz : iz;
+    const bool row = iz < nz;
+    const bool rowLive = row && jz >= w.jz0;
+    const bool anyRow = __builtin_amdgcn_ballot_w64(rowLive) != 0;
+    // the constants of the step loop in registers (the barriers' memory
+    // clobbers would reload them)
+    Band2D<AHEAD> b{source2d(p), w, grid2d(p), lane, iz, nx, row,
+                    rowLive ? (uint32_t) (nx - w.jx0) : 0u,
+                    rowLive ? -kHuge : 4*kHuge, first, last, 1, 0, 0, old,
+                    cells + lane, out, 0, 0, 0, 0, 0, 0, {}, {}, {}};
+    // Runs of groups of one kind: [0, idleEnd) idle, [fullLo, fullHi) full,
+    // [boxLo, boxEnd) with lanes in the box or on the step before it.
+    // (the step before the first live one is not idle: it leaves the box's
+    // distances)
+    const int idleEnd = anyRow ? min((w.jx0 - 1)/kGroup2d, groups) : groups;
+    const int fullLo = (w.jx0 + kBand2d - 2)/kGroup2d + 1;
+    const int fullHi = nx/kGroup2d;
+    int boxGroup = groups, boxEnd = groups;
+    const int zLo = max(p.srcCellZ - p.radius, 0);
+    const int zHi = min(p.srcCellZ + p.radius, nz - 1);
+    if (p.radius >= 0 && zHi >= kBand2d*band && zLo < kBand2d*(band + 1))
+    {
+        const int xLo = max(p.srcCellX - p.radius, 0);
+        const int xHi = min(p.srcCellX + p.radius, nx - 1);
+        // the lanes of the box's rows in this band
+        const int iLo = max(zLo - kBand2d*band, 0);
+        const int iHi = min(zHi - kBand2d*band, kBand2d - 1);
+        b.boxLo = (w.negX ? nx - 1 - xHi : xLo) +
+                  (w.negZ ? kBand2d - 1 - iHi : iLo);
+        b.boxHi = (w.negX ? nx - 1 - xLo : xHi) +
+                  (w.negZ ? kBand2d - 1 - iLo : iHi);
+        boxGroup = max(b.boxLo - 1, 0)/kGroup2d;
+        boxEnd = b.boxHi/kGroup2d + 1;
+    }
+    b.load();
+    // groups [g, end) of one kind; step(ri, hp) runs AHEAD steps.
+    // ri: the previous band's last row at the columns after the step's
+    // (column c in slot c - 1, so that the writer's eight are contiguous),
+    // read one step ahead; hp: lane 63 writes column t - 63 (from the group
+    // that holds column 0 on), the other lanes into a sink.
+    auto run = [&](int g, int end, auto &&step)
+    {
+        for (; g < end; ++g)
+        {
+            const int t = g*kGroup2d;
+            b.hand = ringIn[(t - 1) & (kRing2d - 1)];
+            const double *ri = ringIn + (t & (kRing2d - 1));
+            double *hp = lane == kBand2d - 1 && g >= kLag2d - 2
+                             ? ringOut + (t & (kRing2d - 1)) : sink;
+#pragma unroll 1
+            for (int part = 0; part < kGroup2d; part += AHEAD)
+            {
+                step(ri + part, hp + part);
+            }
+            group_barrier();
+        }
+    };
+    for (int g = 0; g < groups;)
+    {
+        int end = groups;
+        if (g < idleEnd) { end = min(end, idleEnd); }
+        if (g < fullLo) { end = min(end, fullLo); }
+        if (g < fullHi) { end = min(end, fullHi); }
+        if (g < boxGroup) { end = min(end, boxGroup); }
+        if (g < boxEnd) { end = min(end, boxEnd); }
+        if (first || last || (g >= idleEnd && g >= boxGroup && g < boxEnd))
+        {
+            run(g, end, [&](const double *ri, double *hp)
+                { band_steps<UNIFORM, kRare>(b, ri, hp); });
+        }
+        else if (g < idleEnd)
+        {
+            run(g, end, [&](const double *ri, double *hp)
+                { band_steps<UNIFORM, kIdle>(b, ri, hp); });
+        }
+        else if (g >= fullLo && g < fullHi)
+        {
+            run(g, end, [&](const double *ri, double *hp)
+                { band_steps<UNIFORM, kFull>(b, ri, hp); });
+        }
+        else
+        {
+            run(g, end, [&](const double *ri, double *hp)
+                { band_steps<UNIFORM, kAny>(b, ri, hp); });
+        }
+        g = end;
+    }
+}
+
+template <int WAVES, int AHEAD>
+__global__ void __launch_bounds__(kBand2d*WAVES)
+solve2d_bands_kernel(const Problem2D *__restrict__ problems,
+                     double *__restrict__ T, double *work,
+                     const double *__restrict__ cells)
+{
+    // (a group's last read-ahead takes the value after the ring)
+    __shared__ double ring[WAVES][kRing2d + 1];
+    __shared__ double sinks[WAVES][kBand2d + kGroup2d];
+    const Problem2D &p = problems[blockIdx.x];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    const int nx = p.nx, nz = p.nz;
+    const int nb = bands2d(nz);
+    // a wave without a band leaves: barriers count the running waves
+    if (wave >= nb) { return; }
+    // the two buffers of the band's records, at step 0
+    const int64_t perBand = (int64_t) band_records2d(nx)*kBand2d;
+    GlobalDouble *rec[2];
+    rec[0] = (GlobalDouble *) work + p.wOffset + wave*perBand +
+             kBandPad2d*kBand2d;
+    rec[1] = rec[0] + nb*perBand;
+    const GlobalDouble *bandCells = (const GlobalDouble *) cells +
+        p.cOffset + (int64_t) wave*cell_steps2d(nx)*kCellRecord2d;
+    double *sink = &sinks[wave][lane];
+    const int nSweeps = 4*(1 + p.nSweeps);
+    const int groups = (nx + kBand2d - 1 + kGroup2d - 1)/kGroup2d;
+    int now = 0, base = 0;
+    for (int k = 0; k < nSweeps; ++k)
+    {
+        const int sweep = k & 3;
+        const bool last = k == nSweeps - 1;
+        const Sweep2D w = make_sweep2d(p, sweep, k < 4);
+        const bool nextNegZ = (k + 1) & 2;
+        // z reverses with every second sweep: the band that was last is
+        // first, and the others wait for it
+        if (k > 0) { base += groups + ((k & 1) ? 0 : kLag2d*(nb - 1)); }
+        const int pos = w.negZ ? nb - 1 - wave : wave;
+        for (; now < base + kLag2d*pos; ++now) { group_barrier(); }
+        const GlobalDouble *old = ((k & 1) ? rec[1] : rec[0]) + lane;
+        // the result of step t, column jx = t - lane: the next sweep's
+        // lane i' of the same row at its step (nx - 1 - jx) + i'
+        const int i = nextNegZ == (bool) w.negZ ? lane : kBand2d - 1 - lane;
+        GlobalDouble *out = ((k & 1) ? rec[0] : rec[1]) +
+                            (int64_t) (nx - 1 + lane + i)*kBand2d + i;
+        if (last)
+        {
+            const int izl = kBand2d*wave +
+                            (w.negZ ? kBand2d - 1 - lane : lane);
+            out = (GlobalDouble *) T + p.tOffset + (int64_t) izl*nx;
+        }
+        const int upstream = w.negZ ? min(wave + 1, nb - 1)
+                                    : max(wave - 1, 0);
+        const GlobalDouble *sc = bandCells +
+            (int64_t) sweep*nb*cell_steps2d(nx)*kCellRecord2d;
+        if (p.uniform)
+        {
+            band_sweep<true, AHEAD>(p, w, wave, lane, groups, k == 0, last, old, sc,
+                             out, ring[upstream], ring[wave], sink);
+        }
+        else
+        {
+            band_sweep<false, AHEAD>(p, w, wave, lane, groups, k == 0, last, old,
+                              sc, out, ring[upstream], ring[wave], sink);
+        }
+        now += groups;
+        // the next sweep reads this one's records, by other lanes of the
+        // wave: the stores first
+        __asm__ __volatile__("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0);
+        __asm__ __volatile__("" ::: "memory");
+    }
+}
+
+// The skewed cell records of one model for the four sweeps: value i of
+// step t of a band is the cell at permuted column t - i, permuted row
+// (the node row of lane i) - 1, clamped to the model: lane i's own cell
+// row (its cells 0 and 1) in value i, and in value i + 1 the row beyond
+// (its cell 3: column t - i - 1, row + 1).
+__global__ void __launch_bounds__(256)
+skew_cells2d_kernel(int nx, int nz, const double *__restrict__ s,
+                    double *__restrict__ out)
+{
+    const int ncx = nx - 1, ncz = nz - 1;
+    const int nb = bands2d(nz), steps = cell_steps2d(nx);
+    const int64_t perSweep = (int64_t) nb*steps*kCellRecord2d;
+    const int64_t n = 4*perSweep;
+    for (int64_t e = (int64_t) blockIdx.x*blockDim.x + threadIdx.x; e < n;
+         e += (int64_t) gridDim.x*blockDim.x)
+    {
+        const int sweep = (int) (e/perSweep);
+        const int64_t r = e - sweep*perSweep;
+        const int64_t rec = r/kCellRecord2d;
+        const int i = (int) (r - rec*kCellRecord2d);
+        const int band = (int) (rec/steps);
+        const int t = (int) (rec - (int64_t) band*steps);
+        const bool negX = sweep & 1, negZ = sweep & 2;
+        // permuted row of lane 0 of the band
+        const int jzBase = negZ ? nz - kBand2d*(band + 1) : kBand2d*band;
+        const int pcx = min(max(t - i, 0), ncx - 1);
+        const int pcz = min(max(jzBase + i - 1, 0), ncz - 1);
+        const int cx = negX ? ncx - 1 - pcx : pcx;
+        const int cz = negZ ? ncz - 1 - pcz : pcz;
+        out[e] = s[(int64_t) cz*ncx + cx];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Level kernel, for grids that the band kernel does not take: one sweep of
+// one problem in anti-diagonal order (levels jx + jz), levels separated by
+// block barriers, global memory only.
+// ---------------------------------------------------------------------------
 __device__ void sweep2d_block(const Problem2D &p, int sweep, int initialize,
                               double *__restrict__ T,
                               const double *__restrict__ S)
 {
     const int nx = p.nx, nz = p.nz, ncx = nx - 1, ncz = nz - 1;
-    const int negX = sweep & 1, negZ = (sweep >> 1) & 1;
-    const int signX = negX ? -1 : 1, signZ = negZ ? -1 : 1;
-    const int ixShift = negX ? 1 : -1, izShift = negZ ? 1 : -1;
-    int jx0 = 1, jz0 = 1;
-    if (initialize)
-    {
-        // getLoopLimits (init) 2D, solverUtilities2d.hpp:1004-1053
-        jx0 = negX ? max(nx - 2 - p.srcCellX, 1) : max(p.srcCellX, 1);
-        jz0 = negZ ? max(nz - 2 - p.srcCellZ, 1) : max(p.srcCellZ, 1);
-    }
+    const Sweep2D w = make_sweep2d(p, sweep, initialize);
+    const Source2D src = source2d(p);
     const int lastLevel = (nx - 1) + (nz - 1);
-    for (int level = jx0 + jz0; level <= lastLevel; ++level)
+    for (int level = w.jx0 + w.jz0; level <= lastLevel; ++level)
     {
-        const int kLo = max(jz0, level - (nx - 1));
-        const int kHi = min(nz - 1, level - jx0);
+        const int kLo = max(w.jz0, level - (nx - 1));
+        const int kHi = min(nz - 1, level - w.jx0);
         for (int jz = kLo + (int) threadIdx.x; jz <= kHi; jz += blockDim.x)
         {
             const int jx = level - jz;
-            const int ix = negX ? nx - 1 - jx : jx;
-            const int iz = negZ ? nz - 1 - jz : jz;
-            const int ixU = negX ? ix + 1 : ix - 1;
-            const int izU = negZ ? iz + 1 : iz - 1;
+            const int ix = w.negX ? nx - 1 - jx : jx;
+            const int iz = w.negZ ? nz - 1 - jz : jz;
+            const int ixU = w.negX ? ix + 1 : ix - 1;
+            const int izU = w.negZ ? iz + 1 : iz - 1;
             // gridToSurroundingSlowness (solverUtilities2d.hpp:1279-1370)
             // in the permuted frame: home (jx-1, jz-1), offsets clamped.
             const int pcxH = jx - 1, pcxO = min(jx, ncx - 1);
             const int pczH = jz - 1, pczO = min(jz, ncz - 1);
-            const int cxH = negX ? ncx - 1 - pcxH : pcxH;
-            const int cxO = negX ? ncx - 1 - pcxO : pcxO;
-            const int czH = negZ ? ncz - 1 - pczH : pczH;
-            const int czO = negZ ? ncz - 1 - pczO : pczO;
+            const int cxH = w.negX ? ncx - 1 - pcxH : pcxH;
+            const int cxO = w.negX ? ncx - 1 - pcxO : pcxO;
+            const int czH = w.negZ ? ncz - 1 - pczH : pczH;
+            const int czO = w.negZ ? ncz - 1 - pczO : pczO;
             const double s0 = S[czH*ncx + cxH];
             const double s1 = S[czH*ncx + cxO];
             const double s3 = S[czO*ncx + cxH];
@@ -274,158 +762,26 @@ __device__ void sweep2d_block(const Problem2D &p, int sweep, int initialize,
             const double t2 = T[izU*nx + ixU];
             const double t3 = T[izU*nx + ix];
             double tUpd;
-            if (p.uniform)
+            if (in_factored_box2d(src, ix, iz))
             {
-                tUpd = fd2d_uniform(p, ix, iz, signX, signZ, ixShift, izShift,
-                                    s0, s1, s3, t1, t2, t3);
+                tUpd = factored2d(src, w, ix, iz, s0, s1, s3, t1, t2, t3,
+                                  distance2d(src, ix, iz),
+                                  distance2d(src, ixU, iz),
+                                  distance2d(src, ixU, izU),
+                                  distance2d(src, ix, izU));
+            }
+            else if (p.uniform)
+            {
+                tUpd = cartesian2d_uniform<false>(p.dx, s0, s1, s3, t1, t2, t3);
             }
             else
             {
-                tUpd = fd2d_nonuniform(p, ix, iz, signX, signZ, ixShift,
-                                       izShift, s0, s1, s3, t1, t2, t3);
+                tUpd = cartesian2d_nonuniform<false>(grid2d(p), s0, s1, s3,
+                                                     t1, t2, t3);
             }
             if (tUpd < t0) { T[i0] = tUpd; }
         }
         __syncthreads();
-    }
-}
-
-// One sweep of one problem by one 256-thread workgroup with a node per
-// thread and level, for grids of at most kLdsRows2d rows (nz): the three
-// latest levels of the sweep stay in LDS, indexed by the permuted row jz,
-// so that a node's upwind neighbours (levels L - 1 and L - 2) are LDS
-// reads behind a barrier that waits for LDS only, while the node's old
-// time and cells, which no node of the sweep writes before it, are loaded
-// a level ahead (after the level's own store, so that waiting for them
-// waits for nothing newer) and stay in flight across the barrier.  Nodes of a level
-// that the sweep leaves alone (the boundary row and column, the part
-// outside an initialization sweep's range) enter the buffers with their
-// stored times; every access is unconditional and in bounds (threads past
-// the level's last row repeat it and store the same value), so the
-// compiler counts the prefetch loads exactly.
-constexpr int kLdsRows2d = 256;
-
-__device__ void sweep2d_lds(const Problem2D &p, int sweep, int initialize,
-                            double *__restrict__ T,
-                            const double *__restrict__ S,
-                            double (*lev)[kLdsRows2d])
-{
-    const int tid = threadIdx.x;
-    const int nx = p.nx, nz = p.nz, ncx = nx - 1, ncz = nz - 1;
-    const int negX = sweep & 1, negZ = (sweep >> 1) & 1;
-    const int signX = negX ? -1 : 1, signZ = negZ ? -1 : 1;
-    const int ixShift = negX ? 1 : -1, izShift = negZ ? 1 : -1;
-    int jx0 = 1, jz0 = 1;
-    if (initialize)
-    {
-        // getLoopLimits (init) 2D, solverUtilities2d.hpp:1004-1053
-        jx0 = negX ? max(nx - 2 - p.srcCellX, 1) : max(p.srcCellX, 1);
-        jz0 = negZ ? max(nz - 2 - p.srcCellZ, 1) : max(p.srcCellZ, 1);
-    }
-    const int lastLevel = (nx - 1) + (nz - 1);
-    const int firstLevel = max(0, jx0 + jz0 - 2);
-    auto node = [&](int level, int &jx, int &jz)
-    {
-        const int lo = max(0, level - (nx - 1)), hi = min(nz - 1, level);
-        jz = min(lo + tid, hi);
-        jx = level - jz;
-    };
-    auto fetch = [&](int level, double &f0, double &f1, double &f2,
-                     double &f3)
-    {
-        int jx, jz;
-        node(level, jx, jz);
-        const int ix = negX ? nx - 1 - jx : jx;
-        const int iz = negZ ? nz - 1 - jz : jz;
-        f0 = T[iz*nx + ix];
-        // gridToSurroundingSlowness (solverUtilities2d.hpp:1279-1370):
-        // home (jx-1, jz-1), offsets clamped
-        const int pcxH = max(jx - 1, 0), pcxO = min(jx, ncx - 1);
-        const int pczH = max(jz - 1, 0), pczO = min(jz, ncz - 1);
-        const int cxH = negX ? ncx - 1 - pcxH : pcxH;
-        const int cxO = negX ? ncx - 1 - pcxO : pcxO;
-        const int czH = negZ ? ncz - 1 - pczH : pczH;
-        const int czO = negZ ? ncz - 1 - pczO : pczO;
-        f1 = S[czH*ncx + cxH];
-        f2 = S[czH*ncx + cxO];
-        f3 = S[czO*ncx + cxH];
-    };
-    double t0, s0, s1, s3;
-    fetch(firstLevel, t0, s0, s1, s3);
-    for (int level = firstLevel; level <= lastLevel; ++level)
-    {
-        int jx, jz;
-        node(level, jx, jz);
-        const int ix = negX ? nx - 1 - jx : jx;
-        const int iz = negZ ? nz - 1 - jz : jz;
-        const int jzU = max(jz - 1, 0);
-        const double t1 = lev[(level + 2) % 3][jz];     // (jx - 1, jz)
-        const double t3 = lev[(level + 2) % 3][jzU];    // (jx, jz - 1)
-        const double t2 = lev[(level + 1) % 3][jzU];    // (jx - 1, jz - 1)
-        double v = t0;
-        if (jx >= jx0 && jz >= jz0)
-        {
-            const double tUpd = p.uniform
-                ? fd2d_uniform(p, ix, iz, signX, signZ, ixShift, izShift,
-                               s0, s1, s3, t1, t2, t3)
-                : fd2d_nonuniform(p, ix, iz, signX, signZ, ixShift, izShift,
-                                  s0, s1, s3, t1, t2, t3);
-            v = tUpd < v ? tUpd : v;
-        }
-        T[iz*nx + ix] = v;
-        lev[level % 3][jz] = v;
-        // the next level's node, in flight across the barrier (the last
-        // level repeats itself: in bounds, unused)
-        fetch(min(level + 1, lastLevel), t0, s0, s1, s3);
-        // LDS writes done, then the barrier (global accesses stay in
-        // flight: the field is read back only after the sweep).  The
-        // compiler treats both builtins as touching no memory, so empty
-        // asm statements with a memory clobber keep the lev[] store above
-        // and the next level's lev[] loads below them in program order.
-        __asm__ __volatile__("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        __builtin_amdgcn_s_barrier();
-        __asm__ __volatile__("" ::: "memory");
-    }
-    // the next sweep reads this one's stores from memory
-    __syncthreads();
-}
-
-// The whole solve of problem blockIdx.x by one 256-thread workgroup with
-// LDS level buffers (nz <= kLdsRows2d).
-__global__ void __launch_bounds__(256)
-solve2d_lds_kernel(const Problem2D *__restrict__ problems,
-                   double *__restrict__ T, const double *__restrict__ S)
-{
-    __shared__ double lev[3][kLdsRows2d];
-    const Problem2D &p = problems[blockIdx.x];
-    double *Tp = T + p.tOffset;
-    const double *Sp = S + p.sOffset;
-    const int n = p.nx*p.nz;
-    // Solver2DImpl::initializeTravelTimes (src/solver2d.cpp:61-105)
-    for (int i = threadIdx.x; i < n; i += blockDim.x)
-    {
-        int iz = i/p.nx, ix = i - iz*p.nx;
-        int ox = ix - p.srcCellX, oz = iz - p.srcCellZ;
-        double v = kHuge;
-        if (ox >= 0 && ox <= 1 && oz >= 0 && oz <= 1)
-        {
-            v = analytic_time2d(ix, iz, p.dx, p.dz, p.srcOffX, p.srcOffZ,
-                                p.srcSlowness);
-        }
-        Tp[i] = v;
-    }
-    __syncthreads();
-    for (int sweep = 0; sweep < 4; ++sweep)
-    {
-        sweep2d_lds(p, sweep, 1, Tp, Sp, lev);
-    }
-    for (int k = 0; k < p.nSweeps; ++k)
-    {
-        for (int sweep = 0; sweep < 4; ++sweep)
-        {
-            sweep2d_lds(p, sweep, 0, Tp, Sp, lev);
-        }
     }
 }
 
@@ -538,18 +894,45 @@ nodal_to_cell2d(int nx, int nz, const double *__restrict__ v, int ordering,
 
 hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
                           int maxNz, double *T, const double *S,
+                          double *work, const double *cells,
                           hipStream_t stream)
 {
-    if (maxNz <= kLdsRows2d)
+    const dim3 grid((unsigned) nProblems);
+    const int nb = bands2d(maxNz);
+    if (work == nullptr)
     {
-        hipLaunchKernelGGL(solve2d_lds_kernel, dim3((unsigned) nProblems),
-                           dim3(256), 0, stream, dProblems, T, S);
+        hipLaunchKernelGGL(solve2d_kernel, grid, dim3(256), 0, stream,
+                           dProblems, T, S);
+    }
+    // Registers per wave set the read-ahead: 8 steps (223 registers) while
+    // at most 2 waves share a SIMD, 4 steps (168) for 3 waves, 2 for 4 waves
+    // (128).  201 x 41, one band: 266 ns a step with 4 steps, 239 with 8.
+    else if (nb <= 8)
+    {
+        hipLaunchKernelGGL((solve2d_bands_kernel<8, 8>), grid, dim3(64*nb),
+                           0, stream, dProblems, T, work, cells);
+    }
+    else if (nb <= 12)
+    {
+        hipLaunchKernelGGL((solve2d_bands_kernel<12, 4>), grid, dim3(64*nb),
+                           0, stream, dProblems, T, work, cells);
     }
     else
     {
-        hipLaunchKernelGGL(solve2d_kernel, dim3((unsigned) nProblems),
-                           dim3(256), 0, stream, dProblems, T, S);
+        hipLaunchKernelGGL((solve2d_bands_kernel<kMaxBands2d, 2>), grid,
+                           dim3(64*nb), 0, stream, dProblems, T, work, cells);
     }
+    return hipGetLastError();
+}
+
+hipError_t launch_skew_cells2d(int nx, int nz, const double *s, double *out,
+                               hipStream_t stream)
+{
+    const int64_t n = cell_values2d(nx, nz);
+    const int64_t g = (n + 255)/256;
+    hipLaunchKernelGGL(skew_cells2d_kernel,
+                       dim3((unsigned) (g < 4096 ? g : 4096)), dim3(256), 0,
+                       stream, nx, nz, s, out);
     return hipGetLastError();
 }
 
