@@ -25,6 +25,8 @@ namespace
 
 // Blocks of the model-maximum reduction (FIXED32 modes).
 constexpr size_t kMaxPartials = 1024;
+// blocks of the reduction of one model's slowness range
+constexpr int kRangeBlocks = 256;
 // Column z-chunk depths the launch-shape choice considers (0: whole
 // columns), longest first.
 constexpr int kChunkCandidates[] = {0, 96, 64, 48, 32, 24, 16, 12, 8};
@@ -489,7 +491,8 @@ struct Engine3D
     mutable int naturalProblem = -1;
     mutable uint64_t naturalStamp = 0;
     DeviceBuffer<double> partial;
-    std::vector<double> modelSMax;   // largest slowness of each model
+    // smallest and largest slowness of each model
+    std::vector<double> modelSMin, modelSMax;
     DeviceBuffer<Problem3D> dProblems;
     DeviceBuffer<ColumnItem> dItems;
     // Column items ordered by chain, then diagonal bx + by: chain c's items
@@ -664,7 +667,9 @@ struct Engine3D
         // model offsets (cells)
         modelOffset.assign(nModels, -1);
         modelCells.assign(nModels, 0);
+        modelSMin.assign(nModels, 0.0);
         modelSMax.assign(nModels, 0.0);
+        EKX_CHECK(partial.allocate((size_t) nModels*2*kRangeBlocks));
         totalCells = 0;
         for (int i = 0; i < n; ++i)
         {
@@ -692,7 +697,7 @@ struct Engine3D
             p.tiled = tiled ? 1 : 0;
             p.nTX = tiles_of(g.nx);
             p.nTY = tiles_of(g.ny);
-            p.pad = 0;
+            p.scaled = 0;
             const int64_t nTiles = (int64_t) p.nTX*p.nTY;
             const int m = modelOf[i];
             if (modelBrickOffset[m] < 0)
@@ -742,7 +747,6 @@ struct Engine3D
         if (fixed32())
         {
             EKX_CHECK(SQ.allocate((size_t) totalCells));
-            EKX_CHECK(partial.allocate(kMaxPartials));
             EKX_CHECK(TQ.allocate((size_t) totalNodes));
             EKX_HIP(hipMemsetAsync(TQ.ptr, 0, TQ.count*sizeof(uint32_t),
                                    stream));
@@ -1112,8 +1116,48 @@ struct Engine3D
         return EKX_OK;
     }
 
+    // The slowness range of every model, and whether it suits the update
+    // without range tests of its roots (cartesian_uniform3d); scaled
+    // integers decode to zero or to at least sMax / (2^32 - 2), half a step
+    // less before rounding.
+    ekx_status find_ranges()
+    {
+        const size_t per = 2*(size_t) kRangeBlocks;
+        for (size_t m = 0; m < modelCells.size(); ++m)
+        {
+            EKX_HIP(launch_block_range(modelCells[m], S64.ptr + modelOffset[m],
+                                       partial.ptr + m*per, kRangeBlocks,
+                                       stream));
+        }
+        std::vector<double> host(modelCells.size()*per);
+        EKX_HIP(hipMemcpyAsync(host.data(), partial.ptr,
+                               host.size()*sizeof(double),
+                               hipMemcpyDeviceToHost, stream));
+        EKX_HIP(hipStreamSynchronize(stream));
+        for (size_t m = 0; m < modelCells.size(); ++m)
+        {
+            modelSMin[m] = host[m*per];
+            modelSMax[m] = host[m*per + 1];
+            for (size_t k = m*per; k < (m + 1)*per; k += 2)
+            {
+                modelSMin[m] = std::min(modelSMin[m], host[k]);
+                modelSMax[m] = std::max(modelSMax[m], host[k + 1]);
+            }
+        }
+        for (size_t i = 0; i < problems.size(); ++i)
+        {
+            Problem3D &p = problems[i];
+            const double lo = modelSMin[modelOf[i]];
+            const double hi = modelSMax[modelOf[i]];
+            p.scaled = p.dx*std::min(lo, hi*0x1p-33) >= 0x1p-300 &&
+                       p.dx*hi <= 0x1p500 ? 1 : 0;
+        }
+        return EKX_OK;
+    }
+
     ekx_status finish_models()
     {
+        EKX_CHECK(find_ranges());
         if (S32.ptr)
         {
             EKX_HIP(launch_convert(totalCells, S64.ptr, S32.ptr, stream));
@@ -1122,24 +1166,15 @@ struct Engine3D
         {
             // Per model: the largest slowness fixes the code step
             // (s = code * sMax / (2^32 - 2)), then the model is encoded.
-            std::vector<double> host(kMaxPartials);
             for (size_t m = 0; m < modelCells.size(); ++m)
             {
                 const double *sm = S64.ptr + modelOffset[m];
-                EKX_HIP(launch_block_max(modelCells[m], sm, partial.ptr,
-                                         (int) kMaxPartials, stream));
-                EKX_HIP(hipMemcpyAsync(host.data(), partial.ptr,
-                                       kMaxPartials*sizeof(double),
-                                       hipMemcpyDeviceToHost, stream));
-                EKX_HIP(hipStreamSynchronize(stream));
-                double sMax = 0.0;
-                for (double v : host) { sMax = std::max(sMax, v); }
+                const double sMax = modelSMax[m];
                 if (!(sMax > 0.0) || !std::isfinite(sMax))
                 {
                     return fail(EKX_EINVAL, "slowness model must be positive "
                                             "and finite");
                 }
-                modelSMax[m] = sMax;
                 double step = sMax/(double) kTimeMaxCode;
                 EKX_HIP(launch_encode_slowness(modelCells[m], sm, 1.0/step,
                                                SQ.ptr + modelOffset[m],

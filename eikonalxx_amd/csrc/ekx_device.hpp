@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace ekx
 {
 
@@ -67,6 +69,15 @@ template <typename TS> constexpr int ring_slot()
 {
     return sizeof(TS) == 8 ? 88 : 86;
 }
+// Element type of the slowness ring: the arithmetic's.  Scaled-integer cells
+// are decoded as they enter (2 values a lane and step instead of 4 as they
+// are read); the ring's 2.6 KB still leave more waves per CU than the
+// registers of the FP64 arithmetic do.
+template <typename TS>
+using SlownessRing =
+    typename std::conditional<sizeof(TS) == 4 &&
+                                  !std::is_same<TS, float>::value,
+                              double, TS>::type;
 // Largest prefetch depth (planes loaded ahead) of the column kernel.
 constexpr int kMaxPrefetch = 12;
 
@@ -161,7 +172,8 @@ struct Problem3D
     // slowness bricks.
     int tiled;
     int nTX, nTY;
-    int pad;
+    // h s of every cell within [2^-300, 2^500] (cartesian_uniform3d)
+    int scaled;
     int64_t tCount;
     int64_t eOffset;
     int64_t sbOffset;

@@ -96,11 +96,11 @@ hipError_t launch_cell_velocity_to_slowness3d(int nx, int ny, int nz,
                                               const double *v, int ordering,
                                               double *slow,
                                               hipStream_t stream);
-// Scaled-integer storage: block maxima of a model (nPartial blocks), the
-// model's slowness codes round(s * scale), and every problem's travel-time
+// Block minima and maxima of a model (2 nBlocks values).  Scaled-integer
+// storage: the model's slowness codes round(s * scale), and every problem's travel-time
 // codes decoded to FP64.
-hipError_t launch_block_max(int64_t n, const double *v, double *partial,
-                            int nPartial, hipStream_t stream);
+hipError_t launch_block_range(int64_t n, const double *v, double *partial,
+                              int nBlocks, hipStream_t stream);
 hipError_t launch_encode_slowness(int64_t n, const double *in, double scale,
                                   uint32_t *out, hipStream_t stream);
 hipError_t launch_decode_times(const Problem3D *dProblems, int nProblems,

@@ -385,18 +385,21 @@ struct ColumnRun
 // One column chunk (problem pIndex, column (bx, by), chunk bz) of one sweep
 // on one wave; ringT and ringS are the wave's LDS rings of travel-time
 // planes and slowness records.
-// UNIFORM: the problem's grid is uniform (the Cartesian update's branch);
+// GRID: the Cartesian update's branch (uniform or not) and, on uniform
+// grids, whether the model's h s suit the roots without range tests;
 // MONITOR: the largest decrease is kept for the convergence monitor
 // (change != nullptr).  Both are per launch and item, chosen outside the
 // step loop so that the loop carries no test of them.
+enum Grid3D { kNonUniform, kUniform, kUniformScaled };
+
 template <typename TS, int DL, bool FACTORED, bool COHERENT, bool MERGED,
-          bool UNIFORM, bool MONITOR>
+          Grid3D GRID, bool MONITOR>
 __device__ __forceinline__ void run_column(
     const Problem3D *__restrict__ problems, int pIndex, int bx, int by,
     int bz, int sweep, int initialize, int chunk, int boxPhase,
     TS *__restrict__ T, const TS *__restrict__ S,
     unsigned int *__restrict__ change, TS (*ringT)[ring_slot<TS>()],
-    TS (*ringS)[kColumnPlane], int lane)
+    SlownessRing<TS> (*ringS)[kColumnPlane], int lane)
 {
     // the slowness ring's slots are compile-time per unrolled step
     static_assert(DL % kSlownessRing == 0, "prefetch depth");
@@ -462,8 +465,6 @@ __device__ __forceinline__ void run_column(
     const int ix = negX ? nx - 1 - jx : jx;
     const int iy = negY ? ny - 1 - jy : jy;
     const Sweep3D sw = make_sweep3d(sweep);
-    // problem constant of the uniform Cartesian update
-    const double gridH = p.dx;
 
     // LDS plane layout: local coordinate (c, r) of the permuted frame,
     // c = jx - X0 + 1, r = jy - Y0 + 1, both in 0..8, at r*9 + c (the
@@ -485,6 +486,16 @@ __device__ __forceinline__ void run_column(
     };
     using St = Store<TS>;
     using R = typename St::R;
+    // A cell's slowness as it enters the ring: decoded, and times h for the
+    // uniform Cartesian update (2 products a step; 7 in the update).
+    const bool boxWave = FACTORED || (kMerged && boxColumn);
+    const R sScale = boxWave ? (R) 1 : (R) p.dx;
+    auto ringCell = [&](TS v)
+    {
+        const R s = St::slowness(v, p);
+        if constexpr (FACTORED || GRID == kNonUniform) { return s; }
+        else { return sScale*s; }
+    };
     TS *Tp = T + p.tOffset;
     const int64_t tileIndex = (int64_t) my*nTX + mx;
     // Loads per lane and step: tile element `lane`, one halo value (lanes
@@ -622,8 +633,8 @@ __device__ __forceinline__ void run_column(
 #pragma unroll
     for (int m = 0; m < 2; ++m)
     {
-        ringS[m][dstOwn] = pS0[m];
-        ringS[m][dstHalo] = pS1[m];
+        ringS[m][dstOwn] = ringCell(pS0[m]);
+        ringS[m][dstHalo] = ringCell(pS1[m]);
     }
     // Running plane pointers: the next prefetch (plane min(tc + DL,
     // nPlanes - 1), slowness record P0 + tc + DL + 2) and the next
@@ -644,6 +655,7 @@ __device__ __forceinline__ void run_column(
     // z-neighbours (plane q - 1) of the lane's node, decoded
     R pt4 = (R) kHuge, pt5 = (R) kHuge, pt6 = (R) kHuge, pt7 = (R) kHuge;
     R ps00 = 0, ps10 = 0, ps01 = 0, ps11 = 0;
+    R pMin = 0;                           // min(ps00, ps01), uniform grids
     R maxDrop = 0;                        // largest decrease by this lane
     // The node is local (a+1, b+1); oA is (a, b), the xy-1 neighbour.
     constexpr int kB = 1, kC = kColumnHalo, kD = kColumnHalo + 1;
@@ -716,11 +728,11 @@ __device__ __forceinline__ void run_column(
                 const int slot = (tc >= nPlanes && inSlot == lastSlot)
                                      ? nextSlot(inSlot) : inSlot;
                 TS *dT = ringT[slot];
-                TS *dS = ringS[(u + 2) % kSlownessRing];
+                SlownessRing<TS> *dS = ringS[(u + 2) % kSlownessRing];
                 dT[dstOwn] = bT0[u];
-                dS[dstOwn] = bS0[u];
+                dS[dstOwn] = ringCell(bS0[u]);
                 dT[dstHalo] = bT1[u];
-                dS[dstHalo] = bS1[u];
+                dS[dstHalo] = ringCell(bS1[u]);
             }
             inSlot = nextSlot(inSlot);
             // (b) prefetch plane tc + DL into the freed registers (past the
@@ -768,13 +780,13 @@ __device__ __forceinline__ void run_column(
                 const R t1 = St::time(sT[kC], p);
                 const R t2 = St::time(sT[0], p);
                 const R t3 = St::time(sT[kB], p);
-                const TS *s0 = ringS[u % kSlownessRing] + oA;
-                const TS *s1 = ringS[(u + 1) % kSlownessRing] + oA;
-                const TS *s2 = ringS[(u + 2) % kSlownessRing] + oA;
-                const R c00 = St::slowness(s0[0], p);
-                const R c10 = St::slowness(s1[kB], p);
-                const R c01 = St::slowness(s1[kC], p);
-                const R c11 = St::slowness(s2[kD], p);
+                const R *s0 = ringS[u % kSlownessRing] + oA;
+                const R *s1 = ringS[(u + 1) % kSlownessRing] + oA;
+                const R *s2 = ringS[(u + 2) % kSlownessRing] + oA;
+                const R c00 = s0[0];
+                const R c10 = s1[kB];
+                const R c01 = s1[kC];
+                const R c11 = s2[kD];
                 // the wave-uniform choice of operator outside the lanes'
                 // branch, so that it stays a scalar branch; live: upd and
                 // 0 < q < nPlanes, one unsigned compare
@@ -793,7 +805,8 @@ __device__ __forceinline__ void run_column(
                         sT[kD] = c;
                     }
                 };
-                if (FACTORED || (kMerged && boxColumn))
+                R nextMin = Math<R>::min(c00, c01);
+                if (boxWave)
                 {
                     if (live)
                     {
@@ -804,13 +817,34 @@ __device__ __forceinline__ void run_column(
                             c10, c01, t1, t2, t3, pt4, pt5, pt6, pt7));
                     }
                 }
-                else if constexpr (UNIFORM)
+                else if constexpr (GRID != kNonUniform)
                 {
-                    if (live)
+                    // The merged instance runs short launches whose waves
+                    // have their SIMDs nearly to themselves: there every
+                    // branch is a wait (257 x 257 x 193: 49.4 ms with
+                    // them, 46.4 without); in the bulk launches the
+                    // branches skip work (64 tables sources: 615 and
+                    // 648 ms), and with scaled integers, whose decoding
+                    // fills the waits, they are no slower either way.
+                    if constexpr (kMerged && GRID == kUniformScaled &&
+                                  std::is_same<R, TS>::value)
                     {
-                        keep(cartesian_uniform3d<R>(
-                            (R) gridH, ps00, ps10, ps11, ps01, c00, c10, c01,
-                            t1, t2, t3, pt4, pt5, pt6, pt7));
+                        const R v = cartesian_uniform3d_flat<R>(
+                            ps00, ps10, ps11, ps01, c00, c10, c01, pMin,
+                            nextMin, t1, t2, t3, pt4, pt5, pt6, pt7);
+                        const R tNew = live & (v < tOwn) ? v : tOwn;
+                        if constexpr (MONITOR)
+                        {
+                            maxDrop = Math<R>::max(maxDrop, tOwn - tNew);
+                        }
+                        tOwn = tNew;
+                        sT[kD] = tNew;
+                    }
+                    else if (live)
+                    {
+                        keep(cartesian_uniform3d<R, GRID == kUniformScaled>(
+                            ps00, ps10, ps11, ps01, c00, c10, c01, pMin,
+                            nextMin, t1, t2, t3, pt4, pt5, pt6, pt7));
                     }
                 }
                 else if (live)
@@ -827,6 +861,7 @@ __device__ __forceinline__ void run_column(
                 ps10 = c10;
                 ps01 = c01;
                 ps11 = c11;
+                pMin = nextMin;
             }
             {
                 const uint32_t nb = laneB + kSlotB;
@@ -875,6 +910,36 @@ __device__ __forceinline__ void run_column(
     }
 }
 
+__device__ __forceinline__ int grid_kind(const Problem3D &p)
+{
+    return !p.uniform ? kNonUniform : p.scaled ? kUniformScaled : kUniform;
+}
+
+// go(grid, monitor) with both as compile-time constants.
+template <bool UNIFORM, typename F>
+__device__ __forceinline__ void with_grid(int grid, bool monitor, F &&go)
+{
+    auto with = [&](auto g)
+    {
+        if (monitor) { go(g, std::true_type{}); }
+        else { go(g, std::false_type{}); }
+    };
+    if constexpr (UNIFORM)
+    {
+        if (grid == kUniformScaled)
+        {
+            with(std::integral_constant<Grid3D, kUniformScaled>{});
+            return;
+        }
+        if (grid == kUniform)
+        {
+            with(std::integral_constant<Grid3D, kUniform>{});
+            return;
+        }
+    }
+    with(std::integral_constant<Grid3D, kNonUniform>{});
+}
+
 template <typename TS, int WAVES, int DL, bool FACTORED, bool MERGED = false>
 __global__ void __launch_bounds__(64*WAVES)
 sweep_columns3d(const Problem3D *__restrict__ problems,
@@ -884,7 +949,7 @@ sweep_columns3d(const Problem3D *__restrict__ problems,
                 unsigned int *__restrict__ change)
 {
     __shared__ TS ringT[WAVES][kColumnRing][ring_slot<TS>()];
-    __shared__ TS ringS[WAVES][kSlownessRing][kColumnPlane];
+    __shared__ SlownessRing<TS> ringS[WAVES][kSlownessRing][kColumnPlane];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int itemIndex = blockIdx.x*WAVES + wave;
@@ -914,30 +979,19 @@ sweep_columns3d(const Problem3D *__restrict__ problems,
         by = item.by;
         bz = item.bz;
     }
-    // the grid's uniformity (the Cartesian update's branch; the factored
-    // update tests it itself) and the monitor, outside the step loop
-    const bool uniform = !FACTORED &&
-        __builtin_amdgcn_readfirstlane(
-            problems[__builtin_amdgcn_readfirstlane(pIndex)].uniform) != 0;
-    auto go = [&](auto u, auto m)
+    // the Cartesian update's branch (the factored update tests the grid
+    // itself) and the monitor, outside the step loop
+    const int grid = FACTORED ? kNonUniform
+        : __builtin_amdgcn_readfirstlane(grid_kind(
+              problems[__builtin_amdgcn_readfirstlane(pIndex)]));
+    auto go = [&](auto g, auto m)
     {
-        run_column<TS, DL, FACTORED, false, MERGED, decltype(u)::value,
+        run_column<TS, DL, FACTORED, false, MERGED, decltype(g)::value,
                    decltype(m)::value>(
             problems, pIndex, bx, by, bz, sweep, initialize, chunk, boxPhase,
             T, S, change, ringT[wave], ringS[wave], lane);
     };
-    using Yes = std::true_type;
-    using No = std::false_type;
-    if (change != nullptr)
-    {
-        if (uniform) { go(Yes{}, Yes{}); }
-        else { go(No{}, Yes{}); }
-    }
-    else
-    {
-        if (uniform) { go(Yes{}, No{}); }
-        else { go(No{}, No{}); }
-    }
+    with_grid<!FACTORED>(grid, change != nullptr, go);
 }
 
 // ---------------------------------------------------------------------------
@@ -1008,7 +1062,7 @@ sweep_columns3d_queued(const Problem3D *__restrict__ problems,
                        unsigned int *__restrict__ change, ColumnQueue q)
 {
     __shared__ TS ringT[kColumnRing][ring_slot<TS>()];
-    __shared__ TS ringS[kSlownessRing][kColumnPlane];
+    __shared__ SlownessRing<TS> ringS[kSlownessRing][kColumnPlane];
     const int lane = threadIdx.x & 63;
     for (;;)
     {
@@ -1054,24 +1108,15 @@ sweep_columns3d_queued(const Problem3D *__restrict__ problems,
         // follow in program order and the compiler may not hoist them)
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         // the factored-box chunks run in place (MERGED)
-        auto go = [&](auto u, auto m)
+        auto go = [&](auto g, auto m)
         {
-            run_column<TS, DL, false, true, true, decltype(u)::value,
+            run_column<TS, DL, false, true, true, decltype(g)::value,
                        decltype(m)::value>(problems, pIndex, bx, by, bz,
                                            sweep, initialize, chunk, 0, T, S,
                                            change, ringT, ringS, lane);
         };
-        const bool uniform = __builtin_amdgcn_readfirstlane(p.uniform) != 0;
-        if (change != nullptr)
-        {
-            if (uniform) { go(std::true_type{}, std::true_type{}); }
-            else { go(std::false_type{}, std::true_type{}); }
-        }
-        else
-        {
-            if (uniform) { go(std::true_type{}, std::false_type{}); }
-            else { go(std::false_type{}, std::false_type{}); }
-        }
+        with_grid<true>(__builtin_amdgcn_readfirstlane(grid_kind(p)),
+                        change != nullptr, go);
         // publish once every store of the chunk has completed
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
         __builtin_amdgcn_s_waitcnt(0);
@@ -1248,31 +1293,39 @@ convert_kernel(int64_t n, const TSrc *__restrict__ in, TD *__restrict__ out)
 }
 
 // ---------------------------------------------------------------------------
-// Scaled-integer storage: model maximum, slowness codes, decoded fields.
+// Model range; scaled-integer storage: slowness codes, decoded fields.
 // ---------------------------------------------------------------------------
-// Block maxima of v[0..n) into partial[blockIdx.x] (the host reduces them).
+// Block minima and maxima of v[0..n) into partial[2 blockIdx.x] and
+// partial[2 blockIdx.x + 1] (the host reduces them).
 __global__ void __launch_bounds__(256)
-block_max_kernel(int64_t n, const double *__restrict__ v,
-                 double *__restrict__ partial)
+block_range_kernel(int64_t n, const double *__restrict__ v,
+                   double *__restrict__ partial)
 {
-    __shared__ double red[256];
-    double m = 0.0;
+    __shared__ double lo[256], hi[256];
+    double a = v[0], b = a;
     for (int64_t i = (int64_t) blockIdx.x*blockDim.x + threadIdx.x; i < n;
          i += (int64_t) gridDim.x*blockDim.x)
     {
-        m = fmax(m, v[i]);
+        a = fmin(a, v[i]);
+        b = fmax(b, v[i]);
     }
-    red[threadIdx.x] = m;
+    lo[threadIdx.x] = a;
+    hi[threadIdx.x] = b;
     __syncthreads();
     for (int k = 128; k > 0; k >>= 1)
     {
         if ((int) threadIdx.x < k)
         {
-            red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + k]);
+            lo[threadIdx.x] = fmin(lo[threadIdx.x], lo[threadIdx.x + k]);
+            hi[threadIdx.x] = fmax(hi[threadIdx.x], hi[threadIdx.x + k]);
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) { partial[blockIdx.x] = red[0]; }
+    if (threadIdx.x == 0)
+    {
+        partial[2*blockIdx.x] = lo[0];
+        partial[2*blockIdx.x + 1] = hi[0];
+    }
 }
 
 __global__ void __launch_bounds__(256)
@@ -1588,11 +1641,11 @@ hipError_t launch_convert(int64_t n, const float *in, double *out,
     return hipGetLastError();
 }
 
-hipError_t launch_block_max(int64_t n, const double *v, double *partial,
-                            int nPartial, hipStream_t stream)
+hipError_t launch_block_range(int64_t n, const double *v, double *partial,
+                              int nBlocks, hipStream_t stream)
 {
-    hipLaunchKernelGGL(block_max_kernel, dim3((unsigned) nPartial), dim3(256),
-                       0, stream, n, v, partial);
+    hipLaunchKernelGGL(block_range_kernel, dim3((unsigned) nBlocks),
+                       dim3(256), 0, stream, n, v, partial);
     return hipGetLastError();
 }
 

@@ -29,6 +29,8 @@ template <> struct Math<double>
     { return fmin(a, b); }
     static __device__ __forceinline__ double max(double a, double b)
     { return fmax(a, b); }
+    static __device__ __forceinline__ double fma(double a, double b, double c)
+    { return ::fma(a, b, c); }
     static __device__ __forceinline__ double sqrt(double a)
     {
         double r = sqrt_normal_range(a);
@@ -41,6 +43,13 @@ template <> struct Math<double>
         }
         return r;
     }
+    // of an argument known to lie in sqrt_normal_range's range
+    static __device__ __forceinline__ double sqrt_in_range(double a)
+    { return sqrt_normal_range(a); }
+    // the same, or of zero: the root of the clamped argument, 2^-500, minus
+    // itself (which changes no root of an argument in the range)
+    static __device__ __forceinline__ double sqrt_or_zero(double a)
+    { return sqrt_normal_range(fmax(a, 0x1p-1000)) - 0x1p-500; }
 };
 template <> struct Math<float>
 {
@@ -48,10 +57,16 @@ template <> struct Math<float>
     { return fminf(a, b); }
     static __device__ __forceinline__ float max(float a, float b)
     { return fmaxf(a, b); }
+    static __device__ __forceinline__ float fma(float a, float b, float c)
+    { return ::fmaf(a, b, c); }
     // One-ulp hardware square root: the FP32 modes are validated against
     // the FP64 solve at 1e-5 relative, far above this rounding.
     static __device__ __forceinline__ float sqrt(float a)
     { return __builtin_amdgcn_sqrtf(a); }
+    static __device__ __forceinline__ float sqrt_in_range(float a)
+    { return sqrt(a); }
+    static __device__ __forceinline__ float sqrt_or_zero(float a)
+    { return sqrt(a); }
 };
 
 struct Sweep3D
@@ -123,56 +138,69 @@ __device__ __forceinline__ bool in_factored_box(const Problem3D &p, int ix,
              abs(p.srcCellZ - iz) > p.radius);
 }
 
-// Cartesian branch, uniform grid (:281-371) in arithmetic R.  The
-// candidates' minimum is kept in one running value instead of the
+// Cartesian branch, uniform grid (:281-371) in arithmetic R, from the cells'
+// h s (h min(a, b) = min(h a, h b): rounding is monotone).  hs03: the
+// minimum of hs0 and hs3; hs47 returns that of hs4 and hs7, which is the
+// next plane's hs03.
+//
+// The candidates' minimum is kept in one running value instead of the
 // reference's per-candidate HUGE defaults and final minimum: the same
 // minimum over the valid candidates, except when no 2D or 3D candidate is
 // valid and t1d exceeds HUGE, where the reference returns HUGE.  Neither
 // is then below the node's own value (never above HUGE), so the update
 // keeps the node and the field is the same.
-template <typename R>
+//
+// The instruction count bounds the sweeps, so: a pair's two causality tests
+// are one (max <= min + hs: the other holds by itself), and the products by
+// 2 and 1/2, which are exact, are fused into the sum after them (one
+// rounding, the reference's).  SCALED: every hs in [2^-300, 2^500], so a
+// positive 2D determinant 2 hs hs - c c is hs hs-sized or, where its terms
+// cancel, a multiple of their last place, and its root needs no range test.
+template <typename R, bool SCALED>
 __device__ __forceinline__ R cartesian_uniform3d(
-    R h, R s0, R s1, R s2, R s3, R s4, R s5, R s7,
+    R hs0, R hs1, R hs2, R hs3, R hs4, R hs5, R hs7, R hs03, R &hs47,
     R t1, R t2, R t3, R t4, R t5, R t6, R t7)
 {
     using M = Math<R>;
-    R minS0S3 = M::min(s0, s3);
-    R minS0S1 = M::min(s0, s1);
-    R minS0S4 = M::min(s0, s4);
-    R t1d1 = t1 + h*M::min(minS0S3, M::min(s4, s7));
-    R t1d2 = t3 + h*M::min(minS0S4, M::min(s1, s5));
-    R t1d3 = t4 + h*M::min(minS0S1, M::min(s2, s3));
-    R best = M::min(M::min(t1d1, t1d2), t1d3);
-    R hs03 = h*minS0S3;
-    R hs01 = h*minS0S1;
-    R hs04 = h*minS0S4;
-    R dtCrossXZ = t1 - t4;
-    R detXZ = 2*(hs03*hs03) - dtCrossXZ*dtCrossXZ;
-    if (detXZ > 0 && t4 <= t1 + hs03 && t1 <= t4 + hs03)
+    auto root = [](R a)
     {
-        best = M::min(best, t5 + M::sqrt(detXZ));
+        return SCALED ? M::sqrt_in_range(a) : M::sqrt(a);
+    };
+    hs47 = M::min(hs4, hs7);
+    const R hs01 = M::min(hs0, hs1);
+    const R hs04 = M::min(hs0, hs4);
+    R t1d1 = t1 + M::min(hs03, hs47);
+    R t1d2 = t3 + M::min(hs04, M::min(hs1, hs5));
+    R t1d3 = t4 + M::min(hs01, M::min(hs2, hs3));
+    R best = M::min(M::min(t1d1, t1d2), t1d3);
+    const R max14 = M::max(t1, t4);
+    R dtCrossXZ = t1 - t4;
+    R detXZ = M::fma(2, hs03*hs03, -(dtCrossXZ*dtCrossXZ));
+    if ((detXZ > 0) & (max14 <= M::min(t1, t4) + hs03))
+    {
+        best = M::min(best, t5 + root(detXZ));
     }
     R dtCrossYZ = t3 - t4;
-    R detYZ = 2*(hs01*hs01) - dtCrossYZ*dtCrossYZ;
-    if (detYZ > 0 && t3 <= t4 + hs01 && t4 <= t3 + hs01)
+    R detYZ = M::fma(2, hs01*hs01, -(dtCrossYZ*dtCrossYZ));
+    if ((detYZ > 0) & (M::max(t3, t4) <= M::min(t3, t4) + hs01))
     {
-        best = M::min(best, t7 + M::sqrt(detYZ));
+        best = M::min(best, t7 + root(detYZ));
     }
     R dtCrossXY = t1 - t3;
-    R detXY = 2*(hs04*hs04) - dtCrossXY*dtCrossXY;
-    if (detXY > 0 && t3 <= t1 + hs04 && t1 <= t3 + hs04)
+    R detXY = M::fma(2, hs04*hs04, -(dtCrossXY*dtCrossXY));
+    if ((detXY > 0) & (M::max(t1, t3) <= M::min(t1, t3) + hs04))
     {
-        best = M::min(best, t2 + M::sqrt(detXY));
+        best = M::min(best, t2 + root(detXY));
     }
     // min(t1d, t2d) > max(t1, t4, t3) of the reference
-    if (best > M::max(M::max(t1, t4), t3))
+    if (best > M::max(max14, t3))
     {
         const R third = (R) 0.33333333333333333333333;
         const R half = (R) 0.5;
-        R Tx = t1 + half*(-t4 + t5 - t3 + t2) - t7 + t6;
-        R Ty = t3 + half*(-t4 + t7 - t1 + t2) - t5 + t6;
-        R Tz = t4 + half*(-t1 + t5 - t3 + t7) - t2 + t6;
-        R det = 27*(h*s0)*(h*s0)
+        R Tx = M::fma(half, -t4 + t5 - t3 + t2, t1) - t7 + t6;
+        R Ty = M::fma(half, -t4 + t7 - t1 + t2, t3) - t5 + t6;
+        R Tz = M::fma(half, -t1 + t5 - t3 + t7, t4) - t2 + t6;
+        R det = 27*hs0*hs0
               - (Tx - Ty)*(Tx - Ty)
               - (Tx - Tz)*(Tx - Tz)
               - (Ty - Tz)*(Ty - Tz);
@@ -182,6 +210,63 @@ __device__ __forceinline__ R cartesian_uniform3d(
         }
     }
     return best;
+}
+
+// v where valid, else a number above HUGE (HUGE's next high word): one
+// select instead of two, the low word does not matter.
+__device__ __forceinline__ double valid_or_huge(double v, bool valid)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t hi = valid ? (uint32_t) (u >> 32) : 0x4202A060u;
+    return __builtin_bit_cast(double,
+                              ((uint64_t) hi << 32) | (uint32_t) u);
+}
+__device__ __forceinline__ float valid_or_huge(float v, bool valid)
+{
+    return valid ? v : 2*(float) kHuge;
+}
+
+// cartesian_uniform3d<R, true> without branches: every candidate is
+// evaluated, and an invalid one is replaced by a number above HUGE.  For
+// waves that have a SIMD to themselves, where each branch is a wait.
+template <typename R>
+__device__ __forceinline__ R cartesian_uniform3d_flat(
+    R hs0, R hs1, R hs2, R hs3, R hs4, R hs5, R hs7, R hs03, R &hs47,
+    R t1, R t2, R t3, R t4, R t5, R t6, R t7)
+{
+    using M = Math<R>;
+    hs47 = M::min(hs4, hs7);
+    const R hs01 = M::min(hs0, hs1);
+    const R hs04 = M::min(hs0, hs4);
+    R t1d1 = t1 + M::min(hs03, hs47);
+    R t1d2 = t3 + M::min(hs04, M::min(hs1, hs5));
+    R t1d3 = t4 + M::min(hs01, M::min(hs2, hs3));
+    R best = M::min(M::min(t1d1, t1d2), t1d3);
+    const R max14 = M::max(t1, t4);
+    R dtCrossXZ = t1 - t4;
+    R detXZ = M::fma(2, hs03*hs03, -(dtCrossXZ*dtCrossXZ));
+    R dtCrossYZ = t3 - t4;
+    R detYZ = M::fma(2, hs01*hs01, -(dtCrossYZ*dtCrossYZ));
+    R dtCrossXY = t1 - t3;
+    R detXY = M::fma(2, hs04*hs04, -(dtCrossXY*dtCrossXY));
+    const bool cXZ = (detXZ > 0) & (max14 <= M::min(t1, t4) + hs03);
+    const bool cYZ = (detYZ > 0) & (M::max(t3, t4) <= M::min(t3, t4) + hs01);
+    const bool cXY = (detXY > 0) & (M::max(t1, t3) <= M::min(t1, t3) + hs04);
+    best = M::min(best, valid_or_huge(t5 + M::sqrt_in_range(detXZ), cXZ));
+    best = M::min(best, valid_or_huge(t7 + M::sqrt_in_range(detYZ), cYZ));
+    best = M::min(best, valid_or_huge(t2 + M::sqrt_in_range(detXY), cXY));
+    const R third = (R) 0.33333333333333333333333;
+    const R half = (R) 0.5;
+    R Tx = M::fma(half, -t4 + t5 - t3 + t2, t1) - t7 + t6;
+    R Ty = M::fma(half, -t4 + t7 - t1 + t2, t3) - t5 + t6;
+    R Tz = M::fma(half, -t1 + t5 - t3 + t7, t4) - t2 + t6;
+    R det = 27*hs0*hs0
+          - (Tx - Ty)*(Tx - Ty)
+          - (Tx - Tz)*(Tx - Tz)
+          - (Ty - Tz)*(Ty - Tz);
+    const bool c3 = (best > M::max(max14, t3)) & (det >= 0);
+    return M::min(best, valid_or_huge(third*((Tx + Ty + Tz) +
+                                             M::sqrt_or_zero(det)), c3));
 }
 
 // Factored (spherical) branch, uniform grid (:281-294, :372-553); always
@@ -500,8 +585,11 @@ __device__ __forceinline__ R local_update3d(
     {
         if (p.uniform)
         {
-            return cartesian_uniform3d<R>((R) p.dx, s0, s1, s2, s3, s4, s5,
-                                          s7, t1, t2, t3, t4, t5, t6, t7);
+            const R h = (R) p.dx;
+            R hs47;
+            return cartesian_uniform3d<R, false>(
+                h*s0, h*s1, h*s2, h*s3, h*s4, h*s5, h*s7,
+                Math<R>::min(h*s0, h*s3), hs47, t1, t2, t3, t4, t5, t6, t7);
         }
         return cartesian_nonuniform3d<R>(p, s0, s1, s2, s3, s4, s5, s7,
                                          t1, t2, t3, t4, t5, t6, t7);
