@@ -20,8 +20,9 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(HERE, "libeikonalxx_amd.so")
-SOURCES = ["ekx_kernels3d.hip", "ekx_kernels2d.hip", "ekx_fields.hip",
-           "ekx_model3d.hip", "ekx_capi.hip", "ekx_capi2d.hip"]
+SOURCES = ["ekx_kernels3d.hip", "ekx_flow3d.hip", "ekx_kernels2d.hip",
+           "ekx_fields.hip", "ekx_model3d.hip", "ekx_capi.hip",
+           "ekx_capi2d.hip"]
 ARCH = os.environ.get("EKX_OFFLOAD_ARCH", "gfx950")
 
 
@@ -40,12 +41,13 @@ def compile_flags():
             "-I" + os.path.join(ROOT, "include"), "-I" + CSRC]
 
 
-# Per-source flags.  The column and band kernels are scheduled for
+# Per-source flags.  The column, flow and band kernels are scheduled for
 # instruction-level parallelism: their steps are bound by VALU issue and
 # dependency latency at a residency that LDS (3D) or the few waves of a
 # problem (2D) fix, not by registers.
 SOURCE_FLAGS = {
     "ekx_kernels3d.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
+    "ekx_flow3d.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
     "ekx_kernels2d.hip": ["-mllvm", "-amdgpu-sched-strategy=max-ilp"],
 }
 

@@ -7,6 +7,7 @@
 #include "ekx_storage.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -453,6 +454,41 @@ ekx_status scratch_address(Problem3D **out)
 }
 } // namespace
 
+namespace
+{
+// Waves of flow launches in progress per device.  A flow launch needs all
+// its waves resident together, so it takes place only if they fit beside
+// those of the other flow launches of the process (other threads' solvers);
+// otherwise the solve uses the launches per diagonal.
+std::atomic<int> g_flowWaves[kMaxDevices];
+
+struct FlowReservation
+{
+    int device = -1, waves = 0;
+    FlowReservation() = default;
+    FlowReservation(const FlowReservation &) = delete;
+    FlowReservation &operator=(const FlowReservation &) = delete;
+    ~FlowReservation() { release(); }
+    void release()
+    {
+        if (waves > 0) { g_flowWaves[device].fetch_sub(waves); }
+        waves = 0;
+    }
+    bool take(int dev, int n, int capacity)
+    {
+        if (dev < 0 || dev >= kMaxDevices) { return false; }
+        device = dev;
+        if (g_flowWaves[dev].fetch_add(n) + n > capacity)
+        {
+            g_flowWaves[dev].fetch_sub(n);
+            return false;
+        }
+        waves = n;
+        return true;
+    }
+};
+} // namespace
+
 // ===========================================================================
 // Engine3D: a batch of 3D problems and the schedule that solves them.
 // ===========================================================================
@@ -524,6 +560,18 @@ struct Engine3D
     int queueMaxSweeps = 0;
     int queueWaves = 0;          // column waves the device keeps resident
     uint64_t queueWaitTicks = 0; // bound of one dependency wait
+    // Flow launches (a whole solve in one launch, every column resident):
+    // the columns of all problems and, per element type swept, two buffers
+    // of step records and four of mail.  No columns: not for this setup.
+    std::vector<FlowColumn> flowColumns;
+    DeviceBuffer<FlowColumn> dFlowColumns;
+    DeviceBuffer<double> flowRec64, flowMail64;
+    DeviceBuffer<float> flowRec32, flowMail32;
+    DeviceBuffer<unsigned int> flowError;
+    int64_t flowRecCount = 0, flowMailCount = 0;
+    int flowCapacity = 0;        // waves that the device holds together
+    int flowMaxNz = 0;
+    bool flowUniform = false;
     hipStream_t stream = nullptr;
     hipEvent_t evFork = nullptr;
     hipEvent_t evStart = nullptr, evStop = nullptr;
@@ -784,7 +832,181 @@ struct Engine3D
         }
         else { change.release(); }
         EKX_CHECK(build_schedule());
+        EKX_CHECK(setup_flow());
         EKX_HIP(hipStreamSynchronize(stream));
+        return EKX_OK;
+    }
+
+    // Flow launches serve the default launch shape (a caller who names one
+    // gets it) of the completed schedule in FP64 and FP32 arithmetic on
+    // FP64 and FP32 fields (mail keeps its tag in the sign bit, which the
+    // scaled integers use), for as many columns as the device holds at once.
+    // There the sweeps are a chain of dependent steps, which a launch per
+    // diagonal lengthens: 257 x 257 x 193 FP64 46.5 ms by diagonals, 17.8
+    // ms in one launch.  With more columns than that the chip is full, and
+    // the diagonals keep it so.  Memory that the device does not have for
+    // the buffers is no error: the diagonals need none of it.
+    ekx_status setup_flow()
+    {
+        flowColumns.clear();
+        const ekx_solver_options &o = opt;
+        const bool wanted =
+            kernel() == EKX_KERNEL_COLUMN && !fixed32() && !early_exit() &&
+            o.schedule == EKX_SCHEDULE_COMPLETED && o.kernel_timing == 0 &&
+            o.launch_order == EKX_LAUNCH_AUTO && o.chunk_planes == 0 &&
+            o.chains == 0 && o.prefetch_planes == 0;
+        int device = 0, cus = 0;
+        int64_t columns = 0;
+        int uniform = 0;
+        flowMaxNz = 0;
+        for (const Problem3D &p : problems)
+        {
+            columns += (int64_t) p.nTX*p.nTY;
+            uniform += p.uniform;
+            flowMaxNz = std::max(flowMaxNz, p.nz);
+        }
+        flowUniform = uniform > 0;
+        bool fits = wanted &&
+                    (uniform == 0 || uniform == (int) problems.size());
+        if (fits && hipGetDevice(&device) == hipSuccess &&
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount,
+                                  device) == hipSuccess)
+        {
+            int perCU = 1 << 20;
+            if (sweeps_f64() || polish())
+            {
+                perCU = flow_waves_per_cu<double>(flowUniform);
+            }
+            if (!sweeps_f64())
+            {
+                perCU = std::min(perCU, flow_waves_per_cu<float>(flowUniform));
+            }
+            flowCapacity = perCU*cus;
+            fits = columns <= flowCapacity;
+        }
+        else { fits = false; }
+        int64_t rec = 0, mail = 0;
+        std::vector<FlowColumn> list;
+        for (size_t i = 0; fits && i < problems.size(); ++i)
+        {
+            const Problem3D &p = problems[i];
+            for (int my = 0; my < p.nTY; ++my)
+            {
+                for (int mx = 0; mx < p.nTX; ++mx)
+                {
+                    list.push_back(FlowColumn{
+                        (int) i, mx, my, 0, rec + kFlowPad*kTileValues,
+                        mail + kMailPad*kMailValues});
+                    rec += (int64_t) flow_records(p.nz)*kTileValues;
+                    mail += (int64_t) flow_mails(p.nz)*kMailValues;
+                }
+            }
+        }
+        // (byte offsets into a mail buffer are 32 bits)
+        fits = fits && mail*8 < ((int64_t) 1 << 31);
+        flowRecCount = rec;
+        flowMailCount = mail;
+        const bool f64 = fits && (sweeps_f64() || polish());
+        const bool f32 = fits && !sweeps_f64();
+        const bool have =
+            flowRec64.allocate(f64 ? 2*(size_t) rec : 0) == EKX_OK &&
+            flowMail64.allocate(f64 ? kMailBuffers*(size_t) mail : 0) == EKX_OK &&
+            flowRec32.allocate(f32 ? 2*(size_t) rec : 0) == EKX_OK &&
+            flowMail32.allocate(f32 ? kMailBuffers*(size_t) mail : 0) == EKX_OK &&
+            dFlowColumns.allocate(fits ? list.size() : 0) == EKX_OK &&
+            flowError.allocate(fits ? 1 : 0) == EKX_OK;
+        if (!fits || !have)
+        {
+            if (!have) { (void) hipGetLastError(); }
+            release_flow();
+            return EKX_OK;
+        }
+        flowColumns = list;
+        EKX_HIP(hipMemcpyAsync(dFlowColumns.ptr, flowColumns.data(),
+                               list.size()*sizeof(FlowColumn),
+                               hipMemcpyHostToDevice, stream));
+        return EKX_OK;
+    }
+
+    void release_flow()
+    {
+        flowColumns.clear();
+        dFlowColumns.release();
+        flowRec64.release();
+        flowMail64.release();
+        flowRec32.release();
+        flowMail32.release();
+        flowError.release();
+    }
+
+    // Whether this solve can run as flow launches; takes their waves.
+    bool take_flow(FlowReservation &r) const
+    {
+        if (flowColumns.empty()) { return false; }
+        for (const Problem3D &p : problems)
+        {
+            if (!p.scaled) { return false; }
+        }
+        int device = 0;
+        return hipGetDevice(&device) == hipSuccess &&
+               r.take(device, (int) flowColumns.size(), flowCapacity);
+    }
+
+    template <typename TS> DeviceBuffer<TS> &flow_records_buffer()
+    {
+        if constexpr (sizeof(TS) == 8) { return flowRec64; }
+        else { return flowRec32; }
+    }
+    template <typename TS> DeviceBuffer<TS> &flow_mail_buffer()
+    {
+        if constexpr (sizeof(TS) == 8) { return flowMail64; }
+        else { return flowMail32; }
+    }
+
+    // The sweeps of one precision segment in one launch, from the source
+    // initialisation (doInit) or from the tiled field, to the tiled field.
+    template <typename TS>
+    ekx_status run_flow(TS *T, bool doInit, int iterations,
+                        ekx_solve_stats &st)
+    {
+        const int n = (int) flowColumns.size();
+        TS *rec = flow_records_buffer<TS>().ptr;
+        TS *mail = flow_mail_buffer<TS>().ptr;
+        const int nInit = doInit ? 8 : 0;
+        const int nSweeps = nInit + 8*iterations;
+        for (int s = 0; s < nSweeps; ++s)
+        {
+            count_sweep<TS>(s & 7, s < nInit, st);
+        }
+        st.iterations_run += iterations;
+        if (doInit)
+        {
+            EKX_HIP(launch_clear_words(flowError.ptr, 1, stream));
+        }
+        EKX_HIP(launch_clear_words(
+            reinterpret_cast<unsigned int *>(mail),
+            kMailBuffers*flowMailCount*
+                (int64_t) (sizeof(TS)/sizeof(unsigned int)),
+            stream));
+        if (doInit)
+        {
+            EKX_HIP(launch_flow_init<TS>(dProblems.ptr, dFlowColumns.ptr, n,
+                                         flowMaxNz, rec, stream));
+        }
+        else
+        {
+            EKX_HIP(launch_flow_copy<TS>(dProblems.ptr, dFlowColumns.ptr, n,
+                                         flowMaxNz, 0, true, rec, T, stream));
+        }
+        EKX_HIP(launch_flow3d<TS>(
+            dProblems.ptr, dFlowColumns.ptr, n, nInit, nSweeps, rec,
+            flowRecCount, mail, flowMailCount, bricks<TS>(), flowUniform,
+            flowError.ptr, queueWaitTicks, stream));
+        EKX_HIP(launch_flow_copy<TS>(
+            dProblems.ptr, dFlowColumns.ptr, n, flowMaxNz, nSweeps & 7, false,
+            rec + (nSweeps & 1)*flowRecCount, T, stream));
+        st.kernel_launches += 1;
+        if (sizeof(TS) == 8) { st.kernel_launches_fp64 += 1; }
         return EKX_OK;
     }
 
@@ -1030,7 +1252,7 @@ struct Engine3D
         unsigned int err = 0;
         unsigned int *w = queueWords.ptr + queueFlags +
                           (size_t) nChains*queueMaxSweeps;
-        EKX_HIP(hipMemcpy(&err, w, sizeof(err), hipMemcpyDeviceToHost));
+        EKX_CHECK(copy_out(&err, w, sizeof(err)));
         if (err != 0)
         {
             EKX_HIP(hipMemset(w, 0, sizeof(err)));
@@ -1824,6 +2046,26 @@ struct Engine3D
         }
         haveField = false;
         EKX_CHECK(prepare_sources());
+        bool flowFailed = false;
+        {
+            FlowReservation r;
+            if (take_flow(r)) { EKX_CHECK(solve_fields(true, flowFailed)); }
+            else { EKX_CHECK(solve_fields(false, flowFailed)); }
+        }
+        // a wait of the flow launch exceeded its bound (the device was
+        // shared with work that kept columns out): once more by diagonals
+        if (flowFailed) { EKX_CHECK(solve_fields(false, flowFailed)); }
+        haveField = true;
+        solveStamp += 1;
+        if (nStations > 0) { EKX_CHECK(compute_stations()); }
+        return EKX_OK;
+    }
+
+    // The sweeps of a solve, as flow launches or by diagonals; flowFailed: a
+    // flow launch flagged an error and the field is void.
+    ekx_status solve_fields(bool flow, bool &flowFailed)
+    {
+        flowFailed = false;
         ekx_solve_stats st{};
         st.last_iteration_change = -1;
         const int nIt = opt.number_of_sweeps;
@@ -1833,10 +2075,17 @@ struct Engine3D
         EKX_HIP(hipEventRecord(evStart, stream));
         if (sweeps_f64())
         {
-            EKX_HIP(launch_init3d<double>(dProblems.ptr, nProb, totalNodes,
-                                          T64.ptr, stream));
+            if (!flow)
+            {
+                EKX_HIP(launch_init3d<double>(dProblems.ptr, nProb,
+                                              totalNodes, T64.ptr, stream));
+            }
             EKX_HIP(hipEventRecord(evSeg[0], stream));
-            EKX_CHECK(run_primary<double>(T64.ptr, S64.ptr, nIt, st));
+            if (flow) { EKX_CHECK(run_flow<double>(T64.ptr, true, nIt, st)); }
+            else
+            {
+                EKX_CHECK(run_primary<double>(T64.ptr, S64.ptr, nIt, st));
+            }
             EKX_HIP(hipEventRecord(evSeg[1], stream));
         }
         else if (fixed32())
@@ -1849,10 +2098,21 @@ struct Engine3D
         }
         else
         {
-            EKX_HIP(launch_init3d<float>(dProblems.ptr, nProb, totalNodes,
-                                         T32.ptr, stream));
+            if (!flow)
+            {
+                EKX_HIP(launch_init3d<float>(dProblems.ptr, nProb,
+                                             totalNodes, T32.ptr, stream));
+            }
             EKX_HIP(hipEventRecord(evSeg[0], stream));
-            EKX_CHECK(run_primary<float>(T32.ptr, S32.ptr, itPrimary, st));
+            if (flow)
+            {
+                EKX_CHECK(run_flow<float>(T32.ptr, true, itPrimary, st));
+            }
+            else
+            {
+                EKX_CHECK(run_primary<float>(T32.ptr, S32.ptr, itPrimary,
+                                             st));
+            }
             EKX_HIP(hipEventRecord(evSeg[1], stream));
         }
         if (polish())
@@ -1867,8 +2127,12 @@ struct Engine3D
                 EKX_HIP(launch_convert(totalNodes, T32.ptr, T64.ptr, stream));
             }
             EKX_HIP(hipEventRecord(evSeg[2], stream));
-            EKX_CHECK(run_segment<double>(1, T64.ptr, S64.ptr, false, 1,
-                                          st));
+            if (flow) { EKX_CHECK(run_flow<double>(T64.ptr, false, 1, st)); }
+            else
+            {
+                EKX_CHECK(run_segment<double>(1, T64.ptr, S64.ptr, false, 1,
+                                              st));
+            }
             EKX_HIP(hipEventRecord(evSeg[3], stream));
             polished = true;
         }
@@ -1876,6 +2140,13 @@ struct Engine3D
         EKX_HIP(hipEventSynchronize(evStop));
         EKX_HIP(hipGetLastError());
         EKX_CHECK(check_queue_error());
+        if (flow)
+        {
+            unsigned int err = 0;
+            EKX_CHECK(copy_out(&err, flowError.ptr, sizeof(err)));
+            flowFailed = err != 0;
+            if (flowFailed) { return EKX_OK; }
+        }
         float ms = 0;
         EKX_HIP(hipEventElapsedTime(&ms, evStart, evStop));
         st.last_solve_ms = ms;
@@ -1904,9 +2175,16 @@ struct Engine3D
         st.chunk_planes = kernel() == EKX_KERNEL_COLUMN ? chunkH : 0;
         st.chains = nChains;
         stats = st;
-        haveField = true;
-        solveStamp += 1;
-        if (nStations > 0) { EKX_CHECK(compute_stations()); }
+        return EKX_OK;
+    }
+
+    // Device to host on the engine's own stream: a copy on the default
+    // stream fails while another thread's solver captures its graph.
+    ekx_status copy_out(void *dst, const void *src, size_t bytes) const
+    {
+        EKX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
+                               stream));
+        EKX_HIP(hipStreamSynchronize(stream));
         return EKX_OK;
     }
 
@@ -1950,9 +2228,10 @@ struct Engine3D
         {
             EKX_CHECK(dStations.allocate(locs.size()));
             EKX_CHECK(stationOut.allocate(locs.size()));
-            EKX_HIP(hipMemcpy(dStations.ptr, locs.data(),
-                              locs.size()*sizeof(StationLoc3D),
-                              hipMemcpyHostToDevice));
+            EKX_HIP(hipMemcpyAsync(dStations.ptr, locs.data(),
+                                   locs.size()*sizeof(StationLoc3D),
+                                   hipMemcpyHostToDevice, stream));
+            EKX_HIP(hipStreamSynchronize(stream));
         }
         nStations = n;
         if (haveField && n > 0) { EKX_CHECK(compute_stations()); }
@@ -2053,8 +2332,7 @@ struct Engine3D
                                         std::to_string(nOut/3) +
                                         " values");
         }
-        EKX_HIP(hipMemcpy(out, G.ptr, (size_t) n*sizeof(double),
-                          hipMemcpyDeviceToHost));
+        EKX_CHECK(copy_out(out, G.ptr, (size_t) n*sizeof(double)));
         return EKX_OK;
     }
 
@@ -2112,8 +2390,7 @@ struct Engine3D
         {
             const double *src = nullptr;
             EKX_CHECK(natural_field<double>(problem, T64.ptr, &src));
-            EKX_HIP(hipMemcpy(out, src, (size_t) n*sizeof(double),
-                              hipMemcpyDeviceToHost));
+            EKX_CHECK(copy_out(out, src, (size_t) n*sizeof(double)));
         }
         else if (TQ.ptr)
         {
@@ -2121,8 +2398,8 @@ struct Engine3D
             const uint32_t *src = nullptr;
             EKX_CHECK(natural_field<uint32_t>(problem, TQ.ptr, &src));
             std::vector<uint32_t> tmp((size_t) n);
-            EKX_HIP(hipMemcpy(tmp.data(), src, (size_t) n*sizeof(uint32_t),
-                              hipMemcpyDeviceToHost));
+            EKX_CHECK(copy_out(tmp.data(), src,
+                               (size_t) n*sizeof(uint32_t)));
             const double step = problems[problem].tStep;
             for (int64_t i = 0; i < n; ++i)
             {
@@ -2135,8 +2412,8 @@ struct Engine3D
             const float *src = nullptr;
             EKX_CHECK(natural_field<float>(problem, T32.ptr, &src));
             std::vector<float> tmp((size_t) n);
-            EKX_HIP(hipMemcpy(tmp.data(), src, (size_t) n*sizeof(float),
-                              hipMemcpyDeviceToHost));
+            EKX_CHECK(copy_out(tmp.data(), src,
+                               (size_t) n*sizeof(float)));
             for (int64_t i = 0; i < n; ++i) { out[i] = tmp[(size_t) i]; }
         }
         return EKX_OK;
@@ -2629,8 +2906,7 @@ ekx_status ekx_solver3d_get_travel_times_f32(const ekx_solver3d *h,
             }
             const float *src = nullptr;
             EKX_CHECK(e.natural_field<float>(0, e.T32.ptr, &src));
-            EKX_HIP(hipMemcpy(out, src, (size_t) n*sizeof(float),
-                              hipMemcpyDeviceToHost));
+            EKX_CHECK(e.copy_out(out, src, (size_t) n*sizeof(float)));
             return EKX_OK;
         }
         std::vector<double> tmp((size_t) n);

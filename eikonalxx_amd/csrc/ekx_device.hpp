@@ -211,6 +211,43 @@ struct ColumnQueue
     uint64_t waitTicks;
 };
 
+// Flow kernel (a whole solve in one launch): an 8 x 8 column of a problem,
+// its step records (first element of step 0, in either buffer) and its
+// mailbox (first element of record 0, in each buffer).  A problem's
+// columns follow each other in row-major (tile y, tile x) order, and so do
+// their records and mailboxes.
+struct FlowColumn
+{
+    int problem;
+    int mx, my;
+    int pad;
+    int64_t rec;
+    int64_t mail;
+};
+
+// Step records of 64 values: nz + 14 hold nodes; lanes outside the grid's
+// planes, the steps' rounding to groups of 4 and the prefetch use up to 28
+// records before and 36 after them.
+constexpr int kFlowPad = 28;
+__host__ __device__ inline int flow_records(int nz)
+{
+    return nz + kColumnSkew + kFlowPad + 36;
+}
+
+// Mailbox records: 9 values for the x neighbour (in 16), then 8 for the y
+// neighbour.  Record t is read at the reader's
+// step t and written at the writer's step t + 7, from 7 records before the
+// first on; the reader's prefetch and the rounding of the steps run up to 24
+// records past nz.
+constexpr int kMailValues = 24;
+constexpr int kMailBuffers = 4;
+constexpr int kMailY = 16;
+constexpr int kMailPad = 8;
+__host__ __device__ inline int flow_mails(int nz)
+{
+    return kMailPad + nz + 24;
+}
+
 // A receiver located in one problem's grid (Station3D, src/station3d.cpp:
 // 158-291): offset from the model origin and the cell that holds it.
 struct StationLoc3D

@@ -69,6 +69,31 @@ hipError_t launch_queued_columns3d(const Problem3D *dProblems,
                                    const TS *S, unsigned int *change,
                                    const ColumnQueue &q, int waves, int depth,
                                    hipStream_t stream);
+// Flow kernel: resident waves per CU; the first sweep's records; records
+// from (toRecords) or to the tiled fields, in the order of sweep `sweep`;
+// nSweeps sweeps, the first nInit of them initialisation sweeps, from
+// rec (step records of sweep 0 in the first of two buffers of recCount
+// elements) to the buffer nSweeps & 1, in the order of sweep nSweeps & 7.
+// mail: kMailBuffers buffers of mailCount elements, zero before the launch.  Every
+// model's h s must be in range (Problem3D::scaled), every grid uniform or
+// every one not, and all nColumns waves resident together; error is set when a wait exceeded waitTicks.
+template <typename TS> int flow_waves_per_cu(bool uniform);
+template <typename TS>
+hipError_t launch_flow_init(const Problem3D *dProblems,
+                            const FlowColumn *dColumns, int nColumns,
+                            int maxNz, TS *rec, hipStream_t stream);
+template <typename TS>
+hipError_t launch_flow_copy(const Problem3D *dProblems,
+                            const FlowColumn *dColumns, int nColumns,
+                            int maxNz, int sweep, bool toRecords, TS *rec,
+                            TS *T, hipStream_t stream);
+template <typename TS>
+hipError_t launch_flow3d(const Problem3D *dProblems,
+                         const FlowColumn *dColumns, int nColumns, int nInit,
+                         int nSweeps, TS *rec, int64_t recCount, TS *mail,
+                         int64_t mailCount, const TS *bricks, bool uniform,
+                         unsigned int *error, uint64_t waitTicks,
+                         hipStream_t stream);
 // Zeroes n words of device memory (a kernel, so that captured graphs hold
 // no memset node).
 hipError_t launch_clear_words(unsigned int *w, int64_t n, hipStream_t stream);

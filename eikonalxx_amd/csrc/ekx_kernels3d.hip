@@ -10,31 +10,10 @@
 #include "ekx_kernels.hpp"
 #include "ekx_local3d.hpp"
 #include "ekx_storage.hpp"
+#include "ekx_sweep3d.hpp"
 
 namespace ekx
 {
-
-// First node of each permuted axis that a sweep updates: 1 for refinement
-// sweeps (getLoopLimits, solverUtilities3d.hpp:944-1052), the source octant
-// for initialization sweeps (:1075-1184).
-struct Octant
-{
-    int jx0, jy0, jz0;
-};
-
-__device__ __forceinline__ Octant sweep_octant(const Problem3D &p, int sweep,
-                                               int initialize)
-{
-    Octant o{1, 1, 1};
-    if (initialize)
-    {
-        int negX = sweep & 1, negY = (sweep >> 1) & 1, negZ = (sweep >> 2) & 1;
-        o.jx0 = negX ? max(p.nx - 2 - p.srcCellX, 1) : max(1, p.srcCellX);
-        o.jy0 = negY ? max(p.ny - 2 - p.srcCellY, 1) : max(1, p.srcCellY);
-        o.jz0 = negZ ? max(p.nz - 2 - p.srcCellZ, 1) : max(1, p.srcCellZ);
-    }
-    return o;
-}
 
 // Columns (8 x 8 tiles, indexed in the sweep's visiting order) that
 // overlap the factored-eikonal box |i - iSrc| <= radius
@@ -390,8 +369,6 @@ struct ColumnRun
 // MONITOR: the largest decrease is kept for the convergence monitor
 // (change != nullptr).  Both are per launch and item, chosen outside the
 // step loop so that the loop carries no test of them.
-enum Grid3D { kNonUniform, kUniform, kUniformScaled };
-
 template <typename TS, int DL, bool FACTORED, bool COHERENT, bool MERGED,
           Grid3D GRID, bool MONITOR>
 __device__ __forceinline__ void run_column(
@@ -819,28 +796,7 @@ __device__ __forceinline__ void run_column(
                 }
                 else if constexpr (GRID != kNonUniform)
                 {
-                    // The merged instance runs short launches whose waves
-                    // have their SIMDs nearly to themselves: there every
-                    // branch is a wait (257 x 257 x 193: 49.4 ms with
-                    // them, 46.4 without); in the bulk launches the
-                    // branches skip work (64 tables sources: 615 and
-                    // 648 ms), and with scaled integers, whose decoding
-                    // fills the waits, they are no slower either way.
-                    if constexpr (kMerged && GRID == kUniformScaled &&
-                                  std::is_same<R, TS>::value)
-                    {
-                        const R v = cartesian_uniform3d_flat<R>(
-                            ps00, ps10, ps11, ps01, c00, c10, c01, pMin,
-                            nextMin, t1, t2, t3, pt4, pt5, pt6, pt7);
-                        const R tNew = live & (v < tOwn) ? v : tOwn;
-                        if constexpr (MONITOR)
-                        {
-                            maxDrop = Math<R>::max(maxDrop, tOwn - tNew);
-                        }
-                        tOwn = tNew;
-                        sT[kD] = tNew;
-                    }
-                    else if (live)
+                    if (live)
                     {
                         keep(cartesian_uniform3d<R, GRID == kUniformScaled>(
                             ps00, ps10, ps11, ps01, c00, c10, c01, pMin,

@@ -228,7 +228,11 @@ __device__ __forceinline__ float valid_or_huge(float v, bool valid)
 
 // cartesian_uniform3d<R, true> without branches: every candidate is
 // evaluated, and an invalid one is replaced by a number above HUGE.  For
-// waves that have a SIMD to themselves, where each branch is a wait.
+// waves that have a SIMD nearly to themselves, where each branch is a wait
+// (one 257 x 257 x 193 grid by diagonals: 49.4 ms with branches, 46.4
+// without); where the launches fill the chip the branches skip work (64
+// sources on 385 x 385 x 193: 615 and 648 ms, 62 on 206 x 173 x 44: 30 and
+// 32 ms).
 template <typename R>
 __device__ __forceinline__ R cartesian_uniform3d_flat(
     R hs0, R hs1, R hs2, R hs3, R hs4, R hs5, R hs7, R hs03, R &hs47,
@@ -271,7 +275,7 @@ __device__ __forceinline__ R cartesian_uniform3d_flat(
 
 // Factored (spherical) branch, uniform grid (:281-294, :372-553); always
 // evaluated in double.
-__device__ __noinline__ double factored_uniform3d(
+__device__ __forceinline__ double factored_uniform3d(
     const Problem3D &p, const Sweep3D &sw, int ix, int iy, int iz,
     double s0, double s1, double s2, double s3, double s4, double s5,
     double s7, double t1, double t2, double t3, double t4, double t5,
@@ -460,7 +464,7 @@ __device__ __forceinline__ R cartesian_nonuniform3d(
 }
 
 // Factored branch, non-uniform grid (:591-599, :681-821), in double.
-__device__ __noinline__ double factored_nonuniform3d(
+__device__ __forceinline__ double factored_nonuniform3d(
     const Problem3D &p, const Sweep3D &sw, int ix, int iy, int iz,
     double s0, double s1, double s2, double s3, double s4, double s5,
     double s7, double t1, double t2, double t3, double t4, double t5,
@@ -572,6 +576,91 @@ __device__ __noinline__ double factored_nonuniform3d(
     return fmin(t1d, fmin(t2d, t3d));
 }
 
+// The grid constants of the branch-free updates, by value (in registers
+// across a step loop).
+template <typename R>
+struct FlowGrid
+{
+    R dx, dy, dz, dx2Inv, dy2Inv, dz2Inv;
+    R dx_dz, dz_dx, dy_dz, dz_dy, dx_dy, dy_dx;
+    R dx2_p_dz2_inv, dy2_p_dz2_inv, dx2_p_dy2_inv;
+};
+
+template <typename R>
+__device__ __forceinline__ FlowGrid<R> flow_grid(const Problem3D &p)
+{
+    const NonUniform3D &nu = p.nu;
+    return FlowGrid<R>{
+        (R) p.dx, (R) p.dy, (R) p.dz, (R) nu.dx2Inv, (R) nu.dy2Inv,
+        (R) nu.dz2Inv, (R) nu.dx_dz, (R) nu.dz_dx, (R) nu.dy_dz,
+        (R) nu.dz_dy, (R) nu.dx_dy, (R) nu.dy_dx, (R) nu.dx2_p_dz2_inv,
+        (R) nu.dy2_p_dz2_inv, (R) nu.dx2_p_dy2_inv};
+}
+
+// cartesian_nonuniform3d without branches, for models whose h s are in
+// range (as cartesian_uniform3d_flat).
+template <typename R>
+__device__ __forceinline__ R cartesian_nonuniform3d_flat(
+    const FlowGrid<R> &g, R s0, R s1, R s2, R s3, R s4, R s5, R s7,
+    R t1, R t2, R t3, R t4, R t5, R t6, R t7)
+{
+    using M = Math<R>;
+    const R dx = g.dx, dy = g.dy, dz = g.dz;
+    R minS0S3 = M::min(s0, s3);
+    R minS0S1 = M::min(s0, s1);
+    R minS0S4 = M::min(s0, s4);
+    R t1d1 = t1 + dx*M::min(minS0S3, M::min(s4, s7));
+    R t1d2 = t3 + dy*M::min(minS0S4, M::min(s1, s5));
+    R t1d3 = t4 + dz*M::min(minS0S1, M::min(s2, s3));
+    R best = M::min(M::min(t1d1, t1d2), t1d3);
+    // the candidate of the plane of axes u (neighbour tu) and v (tv), corner
+    // tc: same expressions as the branching form
+    auto plane = [](R tu, R tv, R tc, R s, R du, R dv, R du_dv, R dv_du,
+                    R inv)
+    {
+        R dtCross = tu - tv;
+        R det = (du*du + dv*dv)*(s*s) - dtCross*dtCross;
+        const bool c = (det > 0) & (tu < tv + dv*s) & (tv < tu + du*s);
+        R Tu = tu - tv + tc;
+        R Tv = tv - tu + tc;
+        R t = (Tu*dv_du + Tv*du_dv) + 2*M::sqrt_in_range(det);
+        return valid_or_huge(((du*dv)*inv)*t, c);
+    };
+    best = M::min(best, plane(t1, t4, t5, minS0S3, dx, dz, g.dx_dz, g.dz_dx,
+                              g.dx2_p_dz2_inv));
+    best = M::min(best, plane(t3, t4, t7, minS0S1, dy, dz, g.dy_dz, g.dz_dy,
+                              g.dy2_p_dz2_inv));
+    best = M::min(best, plane(t1, t3, t2, minS0S4, dx, dy, g.dx_dy, g.dy_dx,
+                              g.dx2_p_dy2_inv));
+    const R half = (R) 0.5;
+    R Tx = M::fma(half, -t4 + t5 - t3 + t2, t1) - t7 + t6;
+    R Ty = M::fma(half, -t4 + t7 - t1 + t2, t3) - t5 + t6;
+    R Tz = M::fma(half, -t1 + t5 - t3 + t7, t4) - t2 + t6;
+    const R sumInv = g.dx2Inv + g.dy2Inv + g.dz2Inv;
+    R det = 9*(s0*s0)*sumInv
+          - ((Tx - Tz)*(Tx - Tz))*(g.dx2Inv*g.dz2Inv)
+          - ((Ty - Tz)*(Ty - Tz))*(g.dy2Inv*g.dz2Inv)
+          - ((Tx - Ty)*(Tx - Ty))*(g.dx2Inv*g.dy2Inv);
+    const bool c3 = (best > M::max(M::max(t1, t4), t3)) & (det >= 0);
+    R t = (Tx*g.dx2Inv + Ty*g.dy2Inv + Tz*g.dz2Inv + M::sqrt_or_zero(det))/
+          sumInv;
+    return M::min(best, valid_or_huge(t, c3));
+}
+
+// The factored update as a call, for kernels in which it is rare.
+static __device__ __noinline__ double factored3d(
+    const Problem3D &p, const Sweep3D &sw, int ix, int iy, int iz, double s0,
+    double s1, double s2, double s3, double s4, double s5, double s7,
+    double t1, double t2, double t3, double t4, double t5, double t6,
+    double t7)
+{
+    return p.uniform
+        ? factored_uniform3d(p, sw, ix, iy, iz, s0, s1, s2, s3, s4, s5, s7,
+                             t1, t2, t3, t4, t5, t6, t7)
+        : factored_nonuniform3d(p, sw, ix, iy, iz, s0, s1, s2, s3, s4, s5,
+                                s7, t1, t2, t3, t4, t5, t6, t7);
+}
+
 // The complete local update: the factored branch inside the
 // (2 radius + 1)^3 box around the source cell, Cartesian outside
 // (:296-298).  ix, iy, iz are natural grid indices.
@@ -594,18 +683,8 @@ __device__ __forceinline__ R local_update3d(
         return cartesian_nonuniform3d<R>(p, s0, s1, s2, s3, s4, s5, s7,
                                          t1, t2, t3, t4, t5, t6, t7);
     }
-    double r;
-    if (p.uniform)
-    {
-        r = factored_uniform3d(p, sw, ix, iy, iz, s0, s1, s2, s3, s4, s5, s7,
-                               t1, t2, t3, t4, t5, t6, t7);
-    }
-    else
-    {
-        r = factored_nonuniform3d(p, sw, ix, iy, iz, s0, s1, s2, s3, s4, s5,
-                                  s7, t1, t2, t3, t4, t5, t6, t7);
-    }
-    return (R) r;
+    return (R) factored3d(p, sw, ix, iy, iz, s0, s1, s2, s3, s4, s5, s7, t1,
+                          t2, t3, t4, t5, t6, t7);
 }
 
 } // namespace ekx
