@@ -561,13 +561,15 @@ struct Engine3D
     int queueWaves = 0;          // column waves the device keeps resident
     uint64_t queueWaitTicks = 0; // bound of one dependency wait
     // Flow launches (a whole solve in one launch, every column resident):
-    // the columns of all problems and, per element type swept, two buffers
-    // of step records and four of mail.  No columns: not for this setup.
+    // the columns of all problems in launch order and, per element type
+    // swept, two buffers of step records and four of mail; the error word
+    // and each column's XCD.  No columns: not for this setup.
     std::vector<FlowColumn> flowColumns;
     DeviceBuffer<FlowColumn> dFlowColumns;
     DeviceBuffer<double> flowRec64, flowMail64;
     DeviceBuffer<float> flowRec32, flowMail32;
-    DeviceBuffer<unsigned int> flowError;
+    DeviceBuffer<unsigned int> flowWords;
+    int flowWaves = 0;           // columns without the placeholders
     int64_t flowRecCount = 0, flowMailCount = 0;
     int flowCapacity = 0;        // waves that the device holds together
     int flowMaxNz = 0;
@@ -842,7 +844,7 @@ struct Engine3D
     // FP64 and FP32 fields (mail keeps its tag in the sign bit, which the
     // scaled integers use), for as many columns as the device holds at once.
     // There the sweeps are a chain of dependent steps, which a launch per
-    // diagonal lengthens: 257 x 257 x 193 FP64 46.5 ms by diagonals, 17.8
+    // diagonal lengthens: 257 x 257 x 193 FP64 46.5 ms by diagonals, 15.8
     // ms in one launch.  With more columns than that the chip is full, and
     // the diagonals keep it so.  Memory that the device does not have for
     // the buffers is no error: the diagonals need none of it.
@@ -895,13 +897,15 @@ struct Engine3D
                 for (int mx = 0; mx < p.nTX; ++mx)
                 {
                     list.push_back(FlowColumn{
-                        (int) i, mx, my, 0, rec + kFlowPad*kTileValues,
+                        (int) i, mx, my, (int) list.size(), rec + kFlowPad*kTileValues,
                         mail + kMailPad*kMailValues});
                     rec += (int64_t) flow_records(p.nz)*kTileValues;
                     mail += (int64_t) flow_mails(p.nz)*kMailValues;
                 }
             }
         }
+        std::vector<FlowColumn> placed;
+        if (fits) { placed = place_columns(list); }
         // (byte offsets into a mail buffer are 32 bits)
         fits = fits && mail*8 < ((int64_t) 1 << 31);
         flowRecCount = rec;
@@ -913,19 +917,60 @@ struct Engine3D
             flowMail64.allocate(f64 ? kMailBuffers*(size_t) mail : 0) == EKX_OK &&
             flowRec32.allocate(f32 ? 2*(size_t) rec : 0) == EKX_OK &&
             flowMail32.allocate(f32 ? kMailBuffers*(size_t) mail : 0) == EKX_OK &&
-            dFlowColumns.allocate(fits ? list.size() : 0) == EKX_OK &&
-            flowError.allocate(fits ? 1 : 0) == EKX_OK;
+            dFlowColumns.allocate(fits ? placed.size() : 0) == EKX_OK &&
+            flowWords.allocate(fits ? 1 + list.size() : 0) == EKX_OK;
         if (!fits || !have)
         {
             if (!have) { (void) hipGetLastError(); }
             release_flow();
             return EKX_OK;
         }
-        flowColumns = list;
+        flowColumns = placed;
+        flowWaves = (int) list.size();
         EKX_HIP(hipMemcpyAsync(dFlowColumns.ptr, flowColumns.data(),
-                               list.size()*sizeof(FlowColumn),
+                               placed.size()*sizeof(FlowColumn),
                                hipMemcpyHostToDevice, stream));
         return EKX_OK;
+    }
+
+    // The launch order of the columns.  Workgroups (one column each) go to
+    // the 8 XCDs round-robin by index, and on an XCD to one CU after the
+    // other, then to the next SIMD of each.  So: contiguous runs of columns,
+    // one per XCD, so that most neighbours exchange their mail through one
+    // L2; a run of up to a column per CU stays on one XCD (33 x 29 x 25, 20
+    // columns: 0.68 ms per iteration on one XCD, 0.72 on eight), a longer
+    // one is cheaper spread (129^3, 289 columns: 1.62 ms on three, 1.51 on
+    // eight).  Within a run x first: columns that share a CU are then far
+    // apart in x, and seldom busy together (257 x 257 x 193: 3.46 ms; in
+    // rows of y, where they are neighbours on a diagonal, 4.54).  What runs
+    // where changes no result.
+    static std::vector<FlowColumn> place_columns(
+        const std::vector<FlowColumn> &list)
+    {
+        constexpr size_t kXcds = 8, kCusPerXcd = 32;
+        const size_t n = list.size();
+        const size_t per = std::max((n + kXcds - 1)/kXcds,
+                                    std::min(n, kCusPerXcd));
+        const FlowColumn none{-1, 0, 0, 0, 0, 0};
+        std::vector<FlowColumn> placed(kXcds*per, none);
+        for (size_t x = 0; x < kXcds; ++x)
+        {
+            std::vector<FlowColumn> run(list.begin() + std::min(n, x*per),
+                                        list.begin() +
+                                            std::min(n, (x + 1)*per));
+            std::stable_sort(run.begin(), run.end(),
+                             [](const FlowColumn &a, const FlowColumn &b)
+                             {
+                                 return a.problem != b.problem
+                                            ? a.problem < b.problem
+                                            : a.mx < b.mx;
+                             });
+            for (size_t k = 0; k < run.size(); ++k)
+            {
+                placed[k*kXcds + x] = run[k];
+            }
+        }
+        return placed;
     }
 
     void release_flow()
@@ -936,7 +981,7 @@ struct Engine3D
         flowMail64.release();
         flowRec32.release();
         flowMail32.release();
-        flowError.release();
+        flowWords.release();
     }
 
     // Whether this solve can run as flow launches; takes their waves.
@@ -949,7 +994,7 @@ struct Engine3D
         }
         int device = 0;
         return hipGetDevice(&device) == hipSuccess &&
-               r.take(device, (int) flowColumns.size(), flowCapacity);
+               r.take(device, flowWaves, flowCapacity);
     }
 
     template <typename TS> DeviceBuffer<TS> &flow_records_buffer()
@@ -979,10 +1024,8 @@ struct Engine3D
             count_sweep<TS>(s & 7, s < nInit, st);
         }
         st.iterations_run += iterations;
-        if (doInit)
-        {
-            EKX_HIP(launch_clear_words(flowError.ptr, 1, stream));
-        }
+        EKX_HIP(launch_clear_words(flowWords.ptr + (doInit ? 0 : 1),
+                                   flowWaves + (doInit ? 1 : 0), stream));
         EKX_HIP(launch_clear_words(
             reinterpret_cast<unsigned int *>(mail),
             kMailBuffers*flowMailCount*
@@ -1001,7 +1044,7 @@ struct Engine3D
         EKX_HIP(launch_flow3d<TS>(
             dProblems.ptr, dFlowColumns.ptr, n, nInit, nSweeps, rec,
             flowRecCount, mail, flowMailCount, bricks<TS>(), flowUniform,
-            flowError.ptr, queueWaitTicks, stream));
+            flowWords.ptr, flowWords.ptr + 1, queueWaitTicks, stream));
         EKX_HIP(launch_flow_copy<TS>(
             dProblems.ptr, dFlowColumns.ptr, n, flowMaxNz, nSweeps & 7, false,
             rec + (nSweeps & 1)*flowRecCount, T, stream));
@@ -2143,7 +2186,7 @@ struct Engine3D
         if (flow)
         {
             unsigned int err = 0;
-            EKX_CHECK(copy_out(&err, flowError.ptr, sizeof(err)));
+            EKX_CHECK(copy_out(&err, flowWords.ptr, sizeof(err)));
             flowFailed = err != 0;
             if (flowFailed) { return EKX_OK; }
         }

@@ -213,14 +213,15 @@ struct ColumnQueue
 
 // Flow kernel (a whole solve in one launch): an 8 x 8 column of a problem,
 // its step records (first element of step 0, in either buffer) and its
-// mailbox (first element of record 0, in each buffer).  A problem's
-// columns follow each other in row-major (tile y, tile x) order, and so do
-// their records and mailboxes.
+// mailbox (first element of record 0, in each buffer).  Columns are numbered
+// by id, a problem's in row-major (tile y, tile x) order, and their records
+// and mailboxes follow each other in that order; the launch places them in
+// another (placeholders there have problem -1).
 struct FlowColumn
 {
     int problem;
     int mx, my;
-    int pad;
+    int id;
     int64_t rec;
     int64_t mail;
 };
@@ -234,14 +235,15 @@ __host__ __device__ inline int flow_records(int nz)
     return nz + kColumnSkew + kFlowPad + 36;
 }
 
-// Mailbox records: 9 values for the x neighbour (in 16), then 8 for the y
-// neighbour.  Record t is read at the reader's
-// step t and written at the writer's step t + 7, from 7 records before the
-// first on; the reader's prefetch and the rounding of the steps run up to 24
-// records past nz.
-constexpr int kMailValues = 24;
+// Mailbox records: the corner and the 8 nodes for the x neighbour, then
+// those 7 of the y neighbour's 8 nodes that are not among them (the last of
+// the x neighbour's is the y neighbour's last too): one 128 byte line in
+// FP64.  Record t is read at the reader's step t and written at the writer's
+// step t + 7, from 7 records before the first on; the reader's prefetch and
+// the rounding of the steps run up to 24 records past nz.
+constexpr int kMailValues = 16;
 constexpr int kMailBuffers = 4;
-constexpr int kMailY = 16;
+constexpr int kMailY = 9;
 constexpr int kMailPad = 8;
 __host__ __device__ inline int flow_mails(int nz)
 {

@@ -21,8 +21,9 @@ namespace ekx
 // a ring of 4 steps), its z neighbour one step before by itself.
 //
 // Between columns: at step t a column publishes the values its downwind
-// neighbours need at their step t - 7: lanes (7, b) to x, lanes (a, 7) to y,
-// and the corner (7, -1) with x.  They are 17 mailbox values of one record.
+// neighbours need at their step t - 7: lanes (7, b) for x, lanes (a, 7) for
+// y, and the corner (7, -1) for x.  They are 16 mailbox values of one record,
+// one store.
 // Each sweep of four has its own buffer, and each value carries a tag in its
 // sign bit (times are not negative) that alternates with every fourth sweep,
 // so a value is its own arrival flag: the reader loads kMailAhead steps ahead
@@ -40,16 +41,24 @@ namespace ekx
 // order of the next sweep, so no plane is staged through LDS.  A lane
 // outside the grid's planes writes a padding element.
 //
+// Mail is stored to L2, which is where a reader on the same XCD finds it
+// (its loads pass over the L1), and through to memory as well where a reader
+// is on another XCD: columns tell each other at the start where they run.
+// The launch order makes most neighbours share an XCD.  A hop from column to
+// column takes 8 steps and 1.3 us through L2, 2.7 us through memory (64 x 8
+// x 193: 1.22 ms per iteration with all mail through memory, 1.03 now).
+//
 // What bounds it: the chain of dependent steps.  A sweep needs
-// nz + 14 + lag (bx + by) of them, where lag is 8 plus the mail's flight
-// (store to load through memory, since columns are on all XCDs), and the
-// next sweep starts where the last one ended, so only the reversed axes'
+// nz + 14 + lag (bx + by) of them, where lag is 8 plus the mail's flight,
+// and the next sweep starts where the last one ended, so only the reversed axes'
 // lags add up.  A wave has its SIMD nearly to itself, so a step costs its
 // instruction count: branch-free updates, and group kinds for what a group
 // of 4 steps can meet.
 //
 // One 257 x 257 x 193 grid, FP64, 3 iterations: 46.5 ms with one launch per
-// diagonal of 8-plane chunks (89 a sweep), 17.8 ms here.
+// diagonal of 8-plane chunks (89 a sweep), 15.8 ms here.  A step takes 0.46
+// us alone (170 instructions of 5 cycles, and the wait for LDS), more where
+// waves share a CU (4: 0.52 us) or a SIMD (the younger one 0.7 us).
 //
 // Every wave must be resident at once: the host launches it only for as
 // many columns as the device holds and reserves them; each wait is bounded
@@ -57,8 +66,13 @@ namespace ekx
 // which no wave waits any more and the host solves with the diagonals.
 // ---------------------------------------------------------------------------
 constexpr int kFlowAhead = 4;       // steps that records are loaded ahead
-constexpr int kMailAhead = 2;       // steps that mail is loaded ahead
+// Steps that mail is loaded ahead: each one more is one step more a hop
+// (129^3: 1.50 ms per iteration, 1.65 with 2).
+constexpr int kMailAhead = 1;
 constexpr int kFlowRing = 4;
+// The lane that sends the corner: the lanes from here on hold the mail of
+// node (7, -1).
+constexpr int kCornerLane = 2*kColumnTile;
 
 template <typename TS> using Global = __attribute__((address_space(1))) TS;
 
@@ -92,7 +106,8 @@ __device__ __forceinline__ TS tagged(TS v, uint32_t tag)
 
 // A region of device memory as a buffer resource: a 32-bit lane offset and a
 // scalar one, in bytes, so that a step's address work is scalar.  COHERENT
-// accesses (mail) go past the caches that the other XCDs do not see.
+// accesses are mail's: loads that pass over L1, stores that go through L2 to
+// where the other XCDs see them.
 template <typename TS>
 struct FlowBuffer
 {
@@ -127,22 +142,23 @@ struct FlowBuffer
                         rsrc, (int) lane, (int) scalar, kAux));
         }
     }
-    __device__ __forceinline__ void store_coherent(uint32_t lane,
-                                                   uint32_t scalar,
-                                                   TS v) const
+    template <bool COHERENT>
+    __device__ __forceinline__ void store(uint32_t lane, uint32_t scalar,
+                                          TS v) const
     {
+        constexpr int kAux = COHERENT ? kAgent : 0;
         if constexpr (sizeof(TS) == 8)
         {
             using V2 = __attribute__((ext_vector_type(2))) unsigned int;
             __builtin_amdgcn_raw_buffer_store_b64(
                 __builtin_bit_cast(V2, v), rsrc, (int) lane, (int) scalar,
-                kAgent);
+                kAux);
         }
         else
         {
             __builtin_amdgcn_raw_buffer_store_b32(
                 __builtin_bit_cast(unsigned int, v), rsrc, (int) lane,
-                (int) scalar, kAgent);
+                (int) scalar, kAux);
         }
     }
 };
@@ -179,6 +195,7 @@ struct FlowSweep
     // and yOff, which are 7 records back)
     uint32_t oldS, cellS, mailInS, mailOutS;
     int outStep;
+    int remote;             // a reader of this column's mail on another XCD
     uint32_t tag;
     unsigned int *error;
     uint64_t waitTicks;
@@ -186,10 +203,10 @@ struct FlowSweep
     // per lane
     int lane, ab, ix, iy;
     Global<TS> *out;                        // the result of step t
-    uint32_t oldOff, mailOff, xOff, yOff;   // byte offsets
+    uint32_t oldOff, mailOff, sendOff;  // byte offsets
     uint32_t off00, off10, off01, off11;
     bool need;              // the lane's mail has a sender
-    bool xSender, ySender;
+    bool sender;
     uint32_t liveSpan;
     TS floor;
     int haloPos, haloSlot;  // ring position, and steps back of its slot
@@ -366,16 +383,12 @@ __device__ __forceinline__ void flow_step(FlowSweep<TS> &f,
     // (c) the result for the next sweep, and the mail
     *f.out = cur;
     f.out += f.outStep;
-    if (f.xSender)
+    if (f.sender)
     {
-        f.mail.store_coherent(f.xOff + u*kMailBytes<TS>, f.mailOutS,
-                              tagged(cur, f.tag));
-    }
-    if (f.ySender)
-    {
-        f.mail.store_coherent(f.yOff + u*kMailBytes<TS>, f.mailOutS,
-                              tagged(f.lane == kColumnTile - 1 ? t3 : cur,
-                                     f.tag));
+        const TS sent = tagged(f.lane == kCornerLane ? l.h : cur, f.tag);
+        const uint32_t s = f.mailOutS + u*kMailBytes<TS>;
+        f.mail.template store<false>(f.sendOff, s, sent);
+        if (f.remote) { f.mail.template store<true>(f.sendOff, s, sent); }
     }
     f.pt4 = cur;
     f.pt5 = t1;
@@ -506,6 +519,52 @@ __device__ __forceinline__ uint32_t brick_element(int c, int r, int negX,
                             : yl*kColumnTile + xl);
 }
 
+// Publishes the XCD that this column runs on and returns which neighbours
+// run on the same one (bits: +x, -x, +y, -y), for which L2 is coherent.
+__device__ __forceinline__ unsigned int local_neighbours(
+    unsigned int *xcc, int id, bool hasE, bool hasW, bool hasN, bool hasS,
+    int nTX, unsigned int *error, uint64_t waitTicks, bool &need)
+{
+    constexpr int kXccId = 20;              // hardware register XCC_ID
+    const unsigned int mine =
+        1 + __builtin_amdgcn_s_getreg(kXccId | (3 << 11));
+    const int lane = threadIdx.x & 63;
+    if (lane == 0)
+    {
+        __hip_atomic_store(xcc + id, mine, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const bool has = lane == 0 ? hasE : lane == 1 ? hasW
+                   : lane == 2 ? hasN : lane == 3 ? hasS : false;
+    const int other = id + (lane == 0 ? 1 : lane == 1 ? -1
+                            : lane == 2 ? nTX : lane == 3 ? -nTX : 0);
+    const uint64_t t0 = (uint64_t) wall_clock64();
+    for (;;)
+    {
+        unsigned int v = 0;
+        if (has)
+        {
+            v = __hip_atomic_load(xcc + other, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (__builtin_amdgcn_ballot_w64(has && v == 0) == 0)
+        {
+            return (unsigned int) __builtin_amdgcn_ballot_w64(!has ||
+                                                              v == mine);
+        }
+        const bool stop = __builtin_amdgcn_readfirstlane(
+            __hip_atomic_load(error, __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_AGENT)) != 0;
+        if (stop || (uint64_t) wall_clock64() - t0 > waitTicks)
+        {
+            __hip_atomic_fetch_or(error, 1u, __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+            need = false;
+            return 0;
+        }
+    }
+}
+
 // GRID: every problem's grid.  Two waves per SIMD: 2048 columns on 256 CUs.
 template <typename TS, Grid3D GRID>
 __global__ void __launch_bounds__(64)
@@ -514,10 +573,11 @@ sweep_flow3d(const Problem3D *__restrict__ problems,
              const FlowColumn *__restrict__ columns, int nInit, int nSweeps,
              TS *rec, int64_t recCount, TS *mail, int64_t mailCount,
              const TS *__restrict__ bricks, unsigned int *error,
-             uint64_t waitTicks)
+             unsigned int *xcc, uint64_t waitTicks)
 {
     __shared__ TS ring[kFlowRing][ring_slot<TS>()];
     const FlowColumn col = columns[blockIdx.x];
+    if (col.problem < 0) { return; }
     const Problem3D &p = problems[__builtin_amdgcn_readfirstlane(col.problem)];
     const int lane = threadIdx.x & 63;
     const int a = lane & 7, b = lane >> 3;
@@ -531,6 +591,9 @@ sweep_flow3d(const Problem3D *__restrict__ problems,
     // so that the last two groups receive nothing
     const int groups = (nz + kColumnSkew + 1 + kFlowAhead - 1)/kFlowAhead;
     bool need = true;       // false once a wait has failed
+    const unsigned int local = local_neighbours(
+        xcc, col.id, mx + 1 < nTX, mx > 0, my + 1 < nTY, my > 0, nTX, error,
+        waitTicks, need);
     for (int s = 0; s < nSweeps; ++s)
     {
         const int sweep = s & 7;
@@ -589,12 +652,14 @@ sweep_flow3d(const Problem3D *__restrict__ problems,
         auto bytes = [](int64_t v) { return (uint32_t) (v*kSize); };
         f.oldOff = bytes(lane);
         f.mailOff = bytes(fromMail +
-                          (xHalo ? h : kMailY + h - kColumnTile - 1));
-        f.xSender = a == kColumnTile - 1;
-        f.ySender = b == kColumnTile - 1 || lane == kColumnTile - 1;
-        const int64_t back = selfMail - (kColumnTile - 1)*kMailValues;
-        f.xOff = bytes(back + 1 + b);
-        f.yOff = bytes(back + (lane == kColumnTile - 1 ? 0 : kMailY + a));
+                          (xHalo ? h : h == kCornerLane ? kColumnTile
+                                 : kMailY + h - kColumnTile - 1));
+        f.sender = a == kColumnTile - 1 || b == kColumnTile - 1 ||
+                   lane == kCornerLane;
+        f.remote = 1 - (int) ((local >> negX) & (local >> (2 + negY)) & 1);
+        f.sendOff = bytes(selfMail - (kColumnTile - 1)*kMailValues +
+                          (lane == kCornerLane    ? 0
+                           : a == kColumnTile - 1 ? 1 + b : kMailY + a));
         f.off00 = bytes(brick_element(a, b, negX, negY));
         f.off10 = bytes(kBrickValues + brick_element(a + 1, b, negX, negY));
         f.off01 = bytes(kBrickValues + brick_element(a, b + 1, negX, negY));
@@ -703,6 +768,7 @@ flow_init_kernel(const Problem3D *__restrict__ problems,
                  const FlowColumn *__restrict__ columns, TS *__restrict__ rec)
 {
     const FlowColumn c = columns[blockIdx.x];
+    if (c.problem < 0) { return; }
     const Problem3D &p = problems[c.problem];
     const int lane = threadIdx.x & 63;
     const bool source = p.srcCellX + 1 >= kColumnTile*c.mx &&
@@ -739,6 +805,7 @@ flow_copy_kernel(const Problem3D *__restrict__ problems,
                  TS *__restrict__ rec, TS *__restrict__ T)
 {
     const FlowColumn c = columns[blockIdx.x];
+    if (c.problem < 0) { return; }
     const Problem3D &p = problems[c.problem];
     const int lane = threadIdx.x & 63;
     for (int q = blockIdx.y*4 + (threadIdx.x >> 6); q < p.nz;
@@ -794,7 +861,8 @@ hipError_t launch_flow3d(const Problem3D *dProblems,
                          const FlowColumn *dColumns, int nColumns, int nInit,
                          int nSweeps, TS *rec, int64_t recCount, TS *mail,
                          int64_t mailCount, const TS *bricks, bool uniform,
-                         unsigned int *error, uint64_t waitTicks,
+                         unsigned int *error, unsigned int *xcc,
+                         uint64_t waitTicks,
                          hipStream_t stream)
 {
     if (nColumns <= 0 || nSweeps <= 0) { return hipErrorInvalidValue; }
@@ -804,14 +872,14 @@ hipError_t launch_flow3d(const Problem3D *dProblems,
         hipLaunchKernelGGL((sweep_flow3d<TS, kUniformScaled>), grid, dim3(64),
                            0, stream, dProblems, dColumns, nInit, nSweeps,
                            rec, recCount, mail, mailCount, bricks, error,
-                           waitTicks);
+                           xcc, waitTicks);
     }
     else
     {
         hipLaunchKernelGGL((sweep_flow3d<TS, kNonUniform>), grid, dim3(64), 0,
                            stream, dProblems, dColumns, nInit, nSweeps, rec,
                            recCount, mail, mailCount, bricks, error,
-                           waitTicks);
+                           xcc, waitTicks);
     }
     return hipGetLastError();
 }
@@ -840,7 +908,8 @@ template <typename TS> int flow_waves_per_cu(bool uniform)
                                           const FlowColumn *, int, int, int, \
                                           TS *, int64_t, TS *, int64_t,      \
                                           const TS *, bool, unsigned int *,  \
-                                          uint64_t, hipStream_t);
+                                          unsigned int *, uint64_t,          \
+                                          hipStream_t);
 EKX_FLOW(double)
 EKX_FLOW(float)
 #undef EKX_FLOW

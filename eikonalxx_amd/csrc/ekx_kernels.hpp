@@ -92,8 +92,8 @@ hipError_t launch_flow3d(const Problem3D *dProblems,
                          const FlowColumn *dColumns, int nColumns, int nInit,
                          int nSweeps, TS *rec, int64_t recCount, TS *mail,
                          int64_t mailCount, const TS *bricks, bool uniform,
-                         unsigned int *error, uint64_t waitTicks,
-                         hipStream_t stream);
+                         unsigned int *error, unsigned int *xcc,
+                         uint64_t waitTicks, hipStream_t stream);
 // Zeroes n words of device memory (a kernel, so that captured graphs hold
 // no memset node).
 hipError_t launch_clear_words(unsigned int *w, int64_t n, hipStream_t stream);

@@ -64,6 +64,26 @@ def test_equals_the_diagonals(ekx, precision, sweeps):
         assert getattr(flow, name) == getattr(diagonals, name)
 
 
+@pytest.mark.parametrize("precision", ["FP64", "FP32"])
+@pytest.mark.parametrize("dims", [(64, 32, 9), (72, 32, 9), (130, 70, 9),
+                                  (70, 261, 12)])
+def test_runs_of_columns(ekx, dims, precision):
+    """One XCD just full (32 columns), one column more, and runs that end
+    within a row of columns on several XCDs."""
+    slow, src, _ = _inputs(*dims, (10.0,) * 3, 5)
+    print("case", dims, precision, flush=True)
+    out = []
+    for chunk in (0, 8):
+        s = _solver(ekx, dims, (10.0,) * 3, slow, number_of_sweeps=2,
+                    factored_radius=2, chunk_planes=chunk,
+                    precision=getattr(ekx.Precision, precision))
+        s.set_source(src)
+        s.solve()
+        assert (s.get_stats().kernel_launches == 1) == (chunk == 0)
+        out.append(s.get_travel_time_field())
+    assert np.array_equal(*out)
+
+
 def test_batch_of_uneven_grids(ekx, oracle):
     rng = np.random.default_rng(11)
     problems, refs = [], []
