@@ -14,6 +14,7 @@
 #include <limits>
 #include <map>
 #include <mutex>
+#include <numeric>
 #include <string>
 #include <tuple>
 #include <type_traits>
@@ -842,12 +843,32 @@ struct Engine3D
     // Flow launches serve the default launch shape (a caller who names one
     // gets it) of the completed schedule in FP64 and FP32 arithmetic on
     // FP64 and FP32 fields (mail keeps its tag in the sign bit, which the
-    // scaled integers use), for as many columns as the device holds at once.
-    // There the sweeps are a chain of dependent steps, which a launch per
-    // diagonal lengthens: 257 x 257 x 193 FP64 46.5 ms by diagonals, 15.8
-    // ms in one launch.  With more columns than that the chip is full, and
-    // the diagonals keep it so.  Memory that the device does not have for
-    // the buffers is no error: the diagonals need none of it.
+    // scaled integers use), for problems that each fit the device's resident
+    // waves.  There the sweeps are a chain of dependent steps, which a launch
+    // per diagonal lengthens: 257 x 257 x 193 FP64 46.5 ms by diagonals, 15.7
+    // ms in one launch.
+    // With more columns than waves the problems follow each other through
+    // the device, the longest chains first: a column waits only for columns
+    // of its own problem, and workgroups of an XCD start in launch order, so
+    // the first unfinished problem always becomes resident as a whole (the
+    // bound on waits holds all the same).  That is faster than the diagonals
+    // until these have enough columns to fill the chip: measured on FP64
+    // grids of 64 to 200 nodes a side, by the ratio of all the waves' steps
+    // to what the device runs in the longest chain: 1.2 27.5 -> 15.3 ms, 2.0
+    // 61.4 -> 33.0, 2.6 69.9 -> 63.6, 3.3 37.1 -> 32.4, 3.75 27.3 -> 26.0,
+    // 4.0 67.3 -> 72.7, 5.0 38.7 -> 45.0.  So up to 7/2.
+    // Memory that the device does not have for the buffers is no error: the
+    // diagonals need none of it.
+    static constexpr int64_t kFlowLoad2 = 7;
+
+    // Twice the steps that a wave of problem p spends in a sweep, waits for
+    // the hops to its columns included (a hop is 10.6 steps; x reverses in
+    // every sweep, y in every second).
+    static int64_t flow_chain(const Problem3D &p)
+    {
+        return 2*(p.nz + kColumnSkew) + 21*(p.nTX - 1) + 11*(p.nTY - 1);
+    }
+
     ekx_status setup_flow()
     {
         flowColumns.clear();
@@ -858,12 +879,16 @@ struct Engine3D
             o.launch_order == EKX_LAUNCH_AUTO && o.chunk_planes == 0 &&
             o.chains == 0 && o.prefetch_planes == 0;
         int device = 0, cus = 0;
-        int64_t columns = 0;
+        int64_t most = 0;               // columns of one problem
+        int64_t steps = 0, chain = 0;   // of all waves, of the longest wave
         int uniform = 0;
         flowMaxNz = 0;
         for (const Problem3D &p : problems)
         {
-            columns += (int64_t) p.nTX*p.nTY;
+            const int64_t columns = (int64_t) p.nTX*p.nTY;
+            most = std::max(most, columns);
+            steps += columns*flow_chain(p);
+            chain = std::max(chain, flow_chain(p));
             uniform += p.uniform;
             flowMaxNz = std::max(flowMaxNz, p.nz);
         }
@@ -884,7 +909,8 @@ struct Engine3D
                 perCU = std::min(perCU, flow_waves_per_cu<float>(flowUniform));
             }
             flowCapacity = perCU*cus;
-            fits = columns <= flowCapacity;
+            fits = most <= flowCapacity &&
+                   2*steps <= kFlowLoad2*flowCapacity*chain;
         }
         else { fits = false; }
         int64_t rec = 0, mail = 0;
@@ -935,39 +961,61 @@ struct Engine3D
 
     // The launch order of the columns.  Workgroups (one column each) go to
     // the 8 XCDs round-robin by index, and on an XCD to one CU after the
-    // other, then to the next SIMD of each.  So: contiguous runs of columns,
-    // one per XCD, so that most neighbours exchange their mail through one
-    // L2; a run of up to a column per CU stays on one XCD (33 x 29 x 25, 20
-    // columns: 0.68 ms per iteration on one XCD, 0.72 on eight), a longer
-    // one is cheaper spread (129^3, 289 columns: 1.62 ms on three, 1.51 on
-    // eight).  Within a run x first: columns that share a CU are then far
-    // apart in x, and seldom busy together (257 x 257 x 193: 3.46 ms; in
-    // rows of y, where they are neighbours on a diagonal, 4.54).  What runs
-    // where changes no result.
-    static std::vector<FlowColumn> place_columns(
-        const std::vector<FlowColumn> &list)
+    // other, then to the next SIMD of each.  So a problem's columns are cut
+    // into contiguous runs, one per XCD, so that most neighbours exchange
+    // their mail through one L2; a run of up to a column per CU stays on one
+    // XCD (33 x 29 x 25, 20 columns: 0.68 ms per iteration on one XCD, 0.72
+    // on eight), a longer one is cheaper spread (129^3, 289 columns: 1.62 ms
+    // on three, 1.51 on eight).  Within a run x first: columns that share a
+    // CU are then far apart in x, and seldom busy together (257 x 257 x 193:
+    // 3.46 ms; in rows of y, where they are neighbours on a diagonal, 4.54).
+    // What runs where changes no result.
+    std::vector<FlowColumn> place_columns(
+        const std::vector<FlowColumn> &list) const
     {
         constexpr size_t kXcds = 8, kCusPerXcd = 32;
-        const size_t n = list.size();
-        const size_t per = std::max((n + kXcds - 1)/kXcds,
-                                    std::min(n, kCusPerXcd));
-        const FlowColumn none{-1, 0, 0, 0, 0, 0};
-        std::vector<FlowColumn> placed(kXcds*per, none);
+        // each problem's columns, the longest chain first
+        std::vector<size_t> begin(problems.size() + 1, 0);
+        for (const FlowColumn &c : list) { ++begin[c.problem + 1]; }
+        std::partial_sum(begin.begin(), begin.end(), begin.begin());
+        std::vector<int> byChain(problems.size());
+        std::iota(byChain.begin(), byChain.end(), 0);
+        std::stable_sort(byChain.begin(), byChain.end(), [&](int a, int b)
+                         { return flow_chain(problems[a]) >
+                                  flow_chain(problems[b]); });
+        std::vector<FlowColumn> onXcd[kXcds];
+        for (int i : byChain)
+        {
+            size_t first = begin[i];
+            const size_t end = begin[i + 1], n = end - first;
+            const size_t per = std::max((n + kXcds - 1)/kXcds,
+                                        std::min(n, kCusPerXcd));
+            // the least loaded XCDs first
+            size_t order[kXcds];
+            for (size_t x = 0; x < kXcds; ++x) { order[x] = x; }
+            std::stable_sort(order, order + kXcds, [&](size_t a, size_t b)
+                             { return onXcd[a].size() < onXcd[b].size(); });
+            for (size_t x = 0; first < end; ++x)
+            {
+                const size_t m = std::min(per, end - first);
+                std::vector<FlowColumn> &to = onXcd[order[x]];
+                to.insert(to.end(), list.begin() + first,
+                          list.begin() + first + m);
+                std::stable_sort(to.end() - m, to.end(),
+                                 [](const FlowColumn &a, const FlowColumn &b)
+                                 { return a.mx < b.mx; });
+                first += m;
+            }
+        }
+        size_t longest = 0;
+        for (const auto &l : onXcd) { longest = std::max(longest, l.size()); }
+        std::vector<FlowColumn> placed(kXcds*longest,
+                                       FlowColumn{-1, 0, 0, 0, 0, 0});
         for (size_t x = 0; x < kXcds; ++x)
         {
-            std::vector<FlowColumn> run(list.begin() + std::min(n, x*per),
-                                        list.begin() +
-                                            std::min(n, (x + 1)*per));
-            std::stable_sort(run.begin(), run.end(),
-                             [](const FlowColumn &a, const FlowColumn &b)
-                             {
-                                 return a.problem != b.problem
-                                            ? a.problem < b.problem
-                                            : a.mx < b.mx;
-                             });
-            for (size_t k = 0; k < run.size(); ++k)
+            for (size_t k = 0; k < onXcd[x].size(); ++k)
             {
-                placed[k*kXcds + x] = run[k];
+                placed[k*kXcds + x] = onXcd[x][k];
             }
         }
         return placed;
@@ -984,7 +1032,9 @@ struct Engine3D
         flowWords.release();
     }
 
-    // Whether this solve can run as flow launches; takes their waves.
+    // Whether this solve can run as flow launches; takes their waves: as if
+    // every XCD had as many as the one with most, so that the columns of
+    // launches that run together are resident on each.
     bool take_flow(FlowReservation &r) const
     {
         if (flowColumns.empty()) { return false; }
@@ -994,7 +1044,8 @@ struct Engine3D
         }
         int device = 0;
         return hipGetDevice(&device) == hipSuccess &&
-               r.take(device, flowWaves, flowCapacity);
+               r.take(device, std::min((int) flowColumns.size(), flowCapacity),
+                      flowCapacity);
     }
 
     template <typename TS> DeviceBuffer<TS> &flow_records_buffer()

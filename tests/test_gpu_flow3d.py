@@ -84,6 +84,38 @@ def test_runs_of_columns(ekx, dims, precision):
     assert np.array_equal(*out)
 
 
+@pytest.mark.parametrize("precision", ["FP64", "FP32_POLISH"])
+@pytest.mark.parametrize("shared", [False, True])
+def test_batch_beyond_the_device(ekx, precision, shared):
+    """More columns than the device holds: problems follow each other through
+    it, each as the diagonals solve it."""
+    rng = np.random.default_rng(3)
+    d, problems = (10.0,) * 3, []
+    slow = None
+    for k in range(66):
+        dims = (64, 49, 6) if shared else \
+            tuple(int(v) for v in (*rng.integers(40, 73, 2),
+                                   rng.integers(4, 12)))
+        new, src, _ = _inputs(*dims, d, k)
+        slow = new if not shared or slow is None else slow
+        problems.append((ekx.Geometry3D(*dims, *d), slow, src))
+    columns = sum(((g.nx + 7) // 8) * ((g.ny + 7) // 8)
+                  for g, _, _ in problems)
+    assert columns > 2048
+    print("case", precision, shared, columns, flush=True)
+    out = []
+    for chunk in (0, 8):
+        b = ekx.Batch3D()
+        b.initialize(ekx.SolverOptions(
+            number_of_sweeps=1, factored_radius=2, chunk_planes=chunk,
+            precision=getattr(ekx.Precision, precision)), problems)
+        for _ in range(2):
+            b.solve()
+        assert (b.get_stats().kernel_launches <= 2) == (chunk == 0)
+        out.append([b.get_travel_time_field(k) for k in range(len(problems))])
+    assert all(np.array_equal(x, y) for x, y in zip(*out))
+
+
 def test_batch_of_uneven_grids(ekx, oracle):
     rng = np.random.default_rng(11)
     problems, refs = [], []
