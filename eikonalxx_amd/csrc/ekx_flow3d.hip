@@ -56,7 +56,7 @@ namespace ekx
 // of 4 steps can meet.
 //
 // One 257 x 257 x 193 grid, FP64, 3 iterations: 46.5 ms with one launch per
-// diagonal of 8-plane chunks (89 a sweep), 15.8 ms here.  A step takes 0.46
+// diagonal of 8-plane chunks (89 a sweep), 14.9 ms here.  A step takes 0.46
 // us alone (170 instructions of 5 cycles, and the wait for LDS), more where
 // waves share a CU (4: 0.52 us) or a SIMD (the younger one 0.7 us).
 //
@@ -215,8 +215,26 @@ struct FlowSweep
     TS T0[kFlowAhead], C00[kFlowAhead], C10[kFlowAhead], C01[kFlowAhead],
         C11[kFlowAhead], H[kFlowRing];
     TS pt4, pt5, pt6, pt7, ps00, ps10, ps01, ps11, pMin;
+    FactoredGrid fg;
+    FactoredDistances dist;                 // of the step before, in the box
     bool failed;
 };
+
+// The natural indices of the lane's node in plane q.
+struct FlowPlace
+{
+    int ix, iy, iz;
+};
+
+template <typename TS>
+__device__ __forceinline__ FlowPlace flow_place(const FlowSweep<TS> &f, int q)
+{
+    FlowPlace n{f.ix, f.iy, f.negZ ? f.nz - 1 - q : q};
+    // opaque, so that what the factored update derives from them is not
+    // kept in registers across all the loops
+    __asm__ __volatile__("" : "+v"(n.ix), "+v"(n.iy));
+    return n;
+}
 
 // The lane's mail of the record at byte offset m, once every lane's has the
 // sweep's tag.
@@ -350,30 +368,36 @@ __device__ __forceinline__ void flow_step(FlowSweep<TS> &f,
             const bool live = (uint32_t) (q - f.jz0) < f.liveSpan;
             if constexpr (KIND == kFlowBox)
             {
-                const int iz = f.negZ ? f.nz - 1 - q : q;
-                // opaque, so that what the factored update derives from
-                // them is not kept in registers across all the loops
-                int ix = f.ix, iy = f.iy;
-                __asm__ __volatile__("" : "+v"(ix), "+v"(iy));
-                if (live && in_factored_box(f.p, ix, iy, iz))
+                const FlowPlace n = flow_place(f, q);
+                const Sweep3D sw =
+                    make_sweep3d(f.negX + 2*f.negY + 4*f.negZ);
+                const FactoredDistances d =
+                    factored_distances(f.fg, sw, n.ix, n.iy, n.iz);
+                const bool in = live &&
+                    in_factored_box(f.p, n.ix, n.iy, n.iz);
+                if (__builtin_amdgcn_ballot_w64(in) != 0)
                 {
-                    const Sweep3D sw =
-                        make_sweep3d(f.negX + 2*f.negY + 4*f.negZ);
+                    double w;
                     if constexpr (GRID == kNonUniform)
                     {
-                        v = (TS) factored_nonuniform3d(
-                            f.p, sw, ix, iy, iz, f.ps00, f.ps10, f.ps11,
-                            f.ps01, c00, c10, c01, t1, t2, t3, f.pt4, f.pt5,
-                            f.pt6, f.pt7);
+                        w = factored_nonuniform3d_flat(
+                            f.fg, sw, d, f.dist, n.ix, n.iy, n.iz, f.ps00,
+                            f.ps10, f.ps11, f.ps01, c00, c10, c01, t1, t2,
+                            t3, f.pt4, f.pt5, f.pt6, f.pt7);
                     }
                     else
                     {
-                        v = (TS) factored_uniform3d(
-                            f.p, sw, ix, iy, iz, f.ps00, f.ps10, f.ps11,
-                            f.ps01, c00, c10, c01, t1, t2, t3, f.pt4, f.pt5,
-                            f.pt6, f.pt7);
+                        const double h = sizeof(TS) == 8 ? (double) g.dx
+                                                         : f.fg.dx;
+                        w = factored_uniform3d_flat(
+                            f.fg, sw, d, f.dist, n.ix, n.iy, n.iz, f.ps00,
+                            h*f.ps00, h*f.ps10, h*f.ps11, h*f.ps01, h*c00,
+                            h*c10, h*c01, t1, t2, t3, f.pt4, f.pt5, f.pt6,
+                            f.pt7);
                     }
+                    v = in ? (TS) w : v;
                 }
+                f.dist = d;
             }
             cur = live & (v < t0) ? v : t0;
         }
@@ -401,37 +425,16 @@ __device__ __forceinline__ void flow_step(FlowSweep<TS> &f,
     f.pMin = nextMin;
 }
 
-// One group of steps.  Groups with lanes in the factored box run one copy of
-// the step's code in a loop (the registers loaded ahead are picked by a
-// uniform branch), the others are unrolled.
+// One group of steps.
 template <typename TS, Grid3D GRID, bool BOX, FlowGroup KIND, bool WAIT>
 __device__ __forceinline__ void flow_steps(FlowSweep<TS> &f,
                                            const FlowGrid<TS> &g)
 {
-    if constexpr (KIND == kFlowBox)
-    {
-#pragma unroll 1
-        for (int u = 0; u < kFlowAhead; ++u)
-        {
-            FlowLoads<TS> l;
-            switch (u)
-            {
-            case 0: l = take_loads(f, 0); break;
-            case 1: l = take_loads(f, 1); break;
-            case 2: l = take_loads(f, 2); break;
-            default: l = take_loads(f, 3); break;
-            }
-            flow_step<TS, GRID, BOX, KIND, WAIT>(f, g, u, l);
-        }
-    }
-    else
-    {
 #pragma unroll
-        for (int u = 0; u < kFlowAhead; ++u)
-        {
-            const FlowLoads<TS> l = take_loads(f, u);
-            flow_step<TS, GRID, BOX, KIND, WAIT>(f, g, u, l);
-        }
+    for (int u = 0; u < kFlowAhead; ++u)
+    {
+        const FlowLoads<TS> l = take_loads(f, u);
+        flow_step<TS, GRID, BOX, KIND, WAIT>(f, g, u, l);
     }
     f.t += kFlowAhead;
     f.oldS += kFlowAhead*kRecordBytes<TS>;
@@ -446,6 +449,13 @@ __device__ __forceinline__ void flow_run(FlowSweep<TS> &f,
                                          const FlowGrid<TS> &g, int from,
                                          int to)
 {
+    if constexpr (KIND == kFlowBox)
+    {
+        const FlowPlace n = flow_place(f, f.t - 1 - f.ab);
+        f.dist = factored_distances(
+            f.fg, make_sweep3d(f.negX + 2*f.negY + 4*f.negZ), n.ix, n.iy,
+            n.iz);
+    }
 #pragma unroll 1
     for (int i = from; i < to; ++i)
     {
@@ -719,6 +729,7 @@ sweep_flow3d(const Problem3D *__restrict__ problems,
         const bool box = boxLo <= boxHi && anyRow;
         if (box)
         {
+            f.fg = factored_grid<GRID != kNonUniform>(p);
             flow_column<TS, GRID, true>(f, grid, groups, anyRow, boxLo,
                                         boxHi);
         }

@@ -647,6 +647,278 @@ __device__ __forceinline__ R cartesian_nonuniform3d_flat(
     return M::min(best, valid_or_huge(t, c3));
 }
 
+// The source and the grid constants of the branch-free factored updates, by
+// value; on a uniform grid opaque too, so that no step loads them again and
+// waits (33 x 29 x 25: 1.55 -> 1.53 ms; the 13 values of the other grids are
+// more than the scalar registers hold).
+struct FactoredGrid
+{
+    double dx, dy, dz, x, y, z, slowness2;
+    double dxInv, dyInv, dzInv, dx2Inv, dy2Inv, dz2Inv;
+};
+
+template <bool UNIFORM>
+__device__ __forceinline__ FactoredGrid factored_grid(const Problem3D &p)
+{
+    auto opaque = [](double v)
+    {
+        if (!UNIFORM) { return v; }
+        uint64_t u = __builtin_bit_cast(uint64_t, v);
+        uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t) u);
+        uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t) (u >> 32));
+        __asm__ __volatile__("" : "+s"(lo), "+s"(hi));
+        return __builtin_bit_cast(double, ((uint64_t) hi << 32) | lo);
+    };
+    const NonUniform3D &nu = p.nu;
+    FactoredGrid g;
+    g.dx = g.dy = g.dz = opaque(p.dx);
+    g.dxInv = g.dyInv = g.dzInv = opaque(nu.dxInv);
+    g.dx2Inv = g.dy2Inv = g.dz2Inv = opaque(nu.dx2Inv);
+    g.x = opaque(p.srcOffX);
+    g.y = opaque(p.srcOffY);
+    g.z = opaque(p.srcOffZ);
+    g.slowness2 = opaque(p.srcSlowness*p.srcSlowness);
+    if (!UNIFORM)
+    {
+        g.dy = opaque(p.dy);
+        g.dz = opaque(p.dz);
+        g.dyInv = opaque(nu.dyInv);
+        g.dzInv = opaque(nu.dzInv);
+        g.dy2Inv = opaque(nu.dy2Inv);
+        g.dz2Inv = opaque(nu.dz2Inv);
+    }
+    return g;
+}
+
+// What the branch-free factored update keeps from step to step: the
+// distances from the source to the node and its three neighbours in the
+// plane (x-1, (x-1, y-1), y-1), which are the next plane's neighbours in z.
+struct FactoredDistances
+{
+    double d0, d1, d2, d3;
+};
+
+// The distances at a node (natural indices).
+__device__ __forceinline__ FactoredDistances factored_distances(
+    const FactoredGrid &k, const Sweep3D &sw, int ix, int iy, int iz)
+{
+    const double x = ix*k.dx - k.x;
+    const double x1 = (ix + sw.ixShift)*k.dx - k.x;
+    const double y = iy*k.dy - k.y;
+    const double y1 = (iy + sw.iyShift)*k.dy - k.y;
+    const double z = iz*k.dz - k.z;
+    const double xx = x*x, xx1 = x1*x1, yy = y*y, yy1 = y1*y1, zz = z*z;
+    const double a0 = xx + yy + zz, a1 = xx1 + yy + zz;
+    const double a2 = xx1 + yy1 + zz, a3 = xx + yy1 + zz;
+    FactoredDistances d{sqrt_normal_range(a0), sqrt_normal_range(a1),
+                        sqrt_normal_range(a2), sqrt_normal_range(a3)};
+    const bool normal = fmin(fmin(a0, a1), fmin(a2, a3)) >= 0x1p-767;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!normal) != 0, 0))
+    {
+        d = FactoredDistances{::sqrt(a0), ::sqrt(a1), ::sqrt(a2),
+                              ::sqrt(a3)};
+    }
+    return d;
+}
+
+// The roots of the determinants of a node's valid candidates (1 for the
+// others): one test for arguments under sqrt_normal_range's range.
+struct FactoredRoots
+{
+    double xz, yz, xy, xyz;
+};
+
+__device__ __forceinline__ double valid_or_one(double v, bool valid)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, v);
+    const uint32_t hi = valid ? (uint32_t) (u >> 32) : 0x3FF00000u;
+    return __builtin_bit_cast(double,
+                              ((uint64_t) hi << 32) | (uint32_t) u);
+}
+
+__device__ __forceinline__ FactoredRoots factored_roots(double xz, double yz,
+                                                        double xy, double xyz)
+{
+    FactoredRoots r{sqrt_normal_range(xz), sqrt_normal_range(yz),
+                    sqrt_normal_range(xy), sqrt_normal_range(xyz)};
+    const bool normal = fmin(fmin(xz, yz), fmin(xy, xyz)) >= 0x1p-767;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!normal) != 0, 0))
+    {
+        r = FactoredRoots{::sqrt(xz), ::sqrt(yz), ::sqrt(xy), ::sqrt(xyz)};
+    }
+    return r;
+}
+
+// The factored update without branches, from the distances at the node's
+// plane (d) and at the plane before (e): same values as factored_uniform3d
+// (the causality test of a pair, the exact products by 2 and 1/2 and h s as
+// in cartesian_uniform3d; an invalid candidate is above HUGE).  For the flow
+// kernel, whose lone waves wait at each branch and pay for each instruction:
+// half of a node's eight distances are those of the plane before, and the
+// quotients that depend on the grid alone come with the problem.  8 x 8 x 33
+// with radius 3, 8 sweeps: 497 us with the branching form and its eight
+// distances, 383 now (about 200 without a box).
+__device__ __forceinline__ double factored_uniform3d_flat(
+    const FactoredGrid &k, const Sweep3D &sw, const FactoredDistances &d,
+    const FactoredDistances &e, int ix, int iy, int iz, double s0, double hs0,
+    double hs1, double hs2, double hs3, double hs4, double hs5, double hs7,
+    double t1, double t2, double t3, double t4, double t5, double t6,
+    double t7)
+{
+    const double h = k.dx, hInv = k.dxInv, h2Inv = k.dx2Inv;
+    const double hs03 = fmin(hs0, hs3), hs01 = fmin(hs0, hs1);
+    const double hs04 = fmin(hs0, hs4);
+    const double t1d =
+        fmin(fmin(t1 + fmin(hs03, fmin(hs4, hs7)),
+                  t3 + fmin(hs04, fmin(hs1, hs5))),
+             t4 + fmin(hs01, fmin(hs2, hs3)));
+    const double t0 = s0*d.d0;
+    const bool off = d.d0 > 0;
+    auto slope = [&](int i, double source, int sign)
+    {
+        const double q = (s0*(sign*(i*h - source)))/d.d0;
+        return off ? q : 0.0;
+    };
+    const double gx = slope(ix, k.x, sw.signX);
+    const double gy = slope(iy, k.y, sw.signY);
+    const double gz = slope(iz, k.z, sw.signZ);
+    const double tau1 = t1 - s0*d.d1, tau2 = t2 - s0*d.d2;
+    const double tau3 = t3 - s0*d.d3, tau4 = t4 - s0*e.d0;
+    const double tau5 = t5 - s0*e.d1, tau6 = t6 - s0*e.d2;
+    const double tau7 = t7 - s0*e.d3;
+    const double excess = k.slowness2 - s0*s0;
+    const double h2Half = 0.5*h2Inv, hTwice = 2*hInv, h2Twice = 2*h2Inv;
+    double b[3], det[3];
+    // the pair (u, v), its corner's tau and the third axis' slope
+    auto pair = [&](int m, double tauU, double tauV, double tauC, double gu,
+                    double gv, double gw)
+    {
+        const double Tu = tauU - tauV + tauC, Tv = tauV - tauU + tauC;
+        b[m] = hTwice*(gu + gv) - h2Twice*tauC;
+        const double c = fma(2.0, excess + gw*gw,
+                             h2Half*(Tu*Tu + Tv*Tv) -
+                                 hTwice*(gu*Tu + gv*Tv));
+        det[m] = b[m]*b[m] - (4*h2Inv)*c;
+    };
+    pair(0, tau1, tau4, tau5, gx, gz, gy);
+    pair(1, tau3, tau4, tau7, gy, gz, gx);
+    pair(2, tau1, tau3, tau2, gx, gy, gz);
+    const double taux = fma(0.5, -tau4 + tau5 - tau3 + tau2, tau1) - tau7 +
+                        tau6;
+    const double tauy = fma(0.5, -tau4 + tau7 - tau1 + tau2, tau3) - tau5 +
+                        tau6;
+    const double tauz = fma(0.5, -tau1 + tau5 - tau3 + tau7, tau4) - tau2 +
+                        tau6;
+    const double a3 = 3*h2Inv, h6 = 6*hInv;
+    const double b3 = -2*h2Inv*(taux + tauy + tauz) + h6*(gx + gy + gz);
+    const double c3 = h2Inv*(taux*taux + tauy*tauy + tauz*tauz) -
+                      h6*(gx*taux + gy*tauy + gz*tauz) + 9*excess;
+    const double det3 = b3*b3 - (4*a3)*c3;
+    const double max14 = fmax(t1, t4), max34 = fmax(t3, t4);
+    const double max13 = fmax(t1, t3);
+    const bool cXZ = (det[0] > 0) & (max14 <= fmin(t1, t4) + hs03);
+    const bool cYZ = (det[1] >= 0) & (max34 <= fmin(t3, t4) + hs01);
+    const bool cXY = (det[2] >= 0) & (max13 <= fmin(t1, t3) + hs04);
+    const bool cXYZ = det3 >= 0;
+    const FactoredRoots r = factored_roots(
+        valid_or_one(det[0], cXZ), valid_or_one(det[1], cYZ),
+        valid_or_one(det[2], cXY), valid_or_one(det3, cXYZ));
+    auto candidate = [&](bool c, double bm, double root, double a2,
+                         double upwind)
+    {
+        const double t = t0 + (-bm + root)/a2;
+        return valid_or_huge(t, c & (t >= upwind));
+    };
+    double t2d = candidate(cXZ, b[0], r.xz, h2Twice, max14);
+    t2d = fmin(t2d, candidate(cYZ, b[1], r.yz, h2Twice, max34));
+    t2d = fmin(t2d, candidate(cXY, b[2], r.xy, h2Twice, max13));
+    const double best = fmin(t1d, t2d), max134 = fmax(max14, t3);
+    return fmin(best, candidate(cXYZ & (best > max134), b3, r.xyz, 2*a3,
+                                max134));
+}
+
+// The same for factored_nonuniform3d.
+__device__ __forceinline__ double factored_nonuniform3d_flat(
+    const FactoredGrid &k, const Sweep3D &sw, const FactoredDistances &d,
+    const FactoredDistances &e, int ix, int iy, int iz, double s0, double s1,
+    double s2, double s3, double s4, double s5, double s7, double t1,
+    double t2, double t3, double t4, double t5, double t6, double t7)
+{
+    const double dx = k.dx, dy = k.dy, dz = k.dz;
+    const double dxInv = k.dxInv, dyInv = k.dyInv, dzInv = k.dzInv;
+    const double dx2Inv = k.dx2Inv, dy2Inv = k.dy2Inv, dz2Inv = k.dz2Inv;
+    const double s03 = fmin(s0, s3), s01 = fmin(s0, s1), s04 = fmin(s0, s4);
+    const double t1d = fmin(fmin(t1 + dx*fmin(s03, fmin(s4, s7)),
+                                 t3 + dy*fmin(s04, fmin(s1, s5))),
+                            t4 + dz*fmin(s01, fmin(s2, s3)));
+    const double t0 = s0*d.d0;
+    const bool off = d.d0 > 0;
+    auto slope = [&](int i, double h, double source, int sign)
+    {
+        const double q = (s0*(sign*(i*h - source)))/d.d0;
+        return off ? q : 0.0;
+    };
+    const double gx = slope(ix, dx, k.x, sw.signX);
+    const double gy = slope(iy, dy, k.y, sw.signY);
+    const double gz = slope(iz, dz, k.z, sw.signZ);
+    const double tau1 = t1 - s0*d.d1, tau2 = t2 - s0*d.d2;
+    const double tau3 = t3 - s0*d.d3, tau4 = t4 - s0*e.d0;
+    const double tau5 = t5 - s0*e.d1, tau6 = t6 - s0*e.d2;
+    const double tau7 = t7 - s0*e.d3;
+    const double excess = k.slowness2 - s0*s0;
+    double b[3], det[3];
+    auto pair = [&](int m, double tauU, double tauV, double tauC, double gu,
+                    double gv, double gw, double uInv, double vInv,
+                    double u2Inv, double v2Inv)
+    {
+        const double Tu = tauU - tauV + tauC, Tv = tauV - tauU + tauC;
+        b[m] = 4*(uInv*gu + vInv*gv) - 2*(Tu*u2Inv + Tv*v2Inv);
+        const double c = fma(4.0, excess + gw*gw,
+                             (Tu*Tu)*u2Inv + (Tv*Tv)*v2Inv -
+                                 4*((gu*Tu)*uInv + (gv*Tv)*vInv));
+        det[m] = b[m]*b[m] - 4*(u2Inv + v2Inv)*c;
+    };
+    pair(0, tau1, tau4, tau5, gx, gz, gy, dxInv, dzInv, dx2Inv, dz2Inv);
+    pair(1, tau3, tau4, tau7, gy, gz, gx, dyInv, dzInv, dy2Inv, dz2Inv);
+    pair(2, tau1, tau3, tau2, gx, gy, gz, dxInv, dyInv, dx2Inv, dy2Inv);
+    const double taux = fma(0.5, -tau4 + tau5 - tau3 + tau2, tau1) - tau7 +
+                        tau6;
+    const double tauy = fma(0.5, -tau4 + tau7 - tau1 + tau2, tau3) - tau5 +
+                        tau6;
+    const double tauz = fma(0.5, -tau1 + tau5 - tau3 + tau7, tau4) - tau2 +
+                        tau6;
+    const double a3 = dx2Inv + dy2Inv + dz2Inv;
+    const double b3 = -2*(taux*dx2Inv + tauy*dy2Inv + tauz*dz2Inv) +
+                      6*(dxInv*gx + dyInv*gy + dzInv*gz);
+    const double c3 = (taux*taux)*dx2Inv + (tauy*tauy)*dy2Inv +
+                      (tauz*tauz)*dz2Inv -
+                      6*(gx*taux*dxInv + gy*tauy*dyInv + gz*tauz*dzInv) +
+                      9*excess;
+    const double det3 = b3*b3 - 4*a3*c3;
+    const bool cXZ = (det[0] > 0) & (t1 < t4 + dz*s03) & (t4 < t1 + dx*s03);
+    const bool cYZ = (det[1] > 0) & (t3 < t4 + dz*s01) & (t4 < t3 + dy*s01);
+    const bool cXY = (det[2] > 0) & (t3 < t1 + dx*s04) & (t1 < t3 + dy*s04);
+    const bool cXYZ = det3 >= 0;
+    const FactoredRoots r = factored_roots(
+        valid_or_one(det[0], cXZ), valid_or_one(det[1], cYZ),
+        valid_or_one(det[2], cXY), valid_or_one(det3, cXYZ));
+    auto candidate = [&](bool c, double bm, double root, double a,
+                         double upwind)
+    {
+        const double t = t0 + (-bm + root)/(2*a);
+        return valid_or_huge(t, c & (t >= upwind));
+    };
+    const double max14 = fmax(t1, t4);
+    double t2d = candidate(cXZ, b[0], r.xz, dx2Inv + dz2Inv, max14);
+    t2d = fmin(t2d, candidate(cYZ, b[1], r.yz, dy2Inv + dz2Inv,
+                              fmax(t3, t4)));
+    t2d = fmin(t2d, candidate(cXY, b[2], r.xy, dx2Inv + dy2Inv,
+                              fmax(t1, t3)));
+    const double best = fmin(t1d, t2d), max134 = fmax(max14, t3);
+    return fmin(best, candidate(cXYZ & (best > max134), b3, r.xyz, a3,
+                                max134));
+}
+
 // The factored update as a call, for kernels in which it is rare.
 static __device__ __noinline__ double factored3d(
     const Problem3D &p, const Sweep3D &sw, int ix, int iy, int iz, double s0,
