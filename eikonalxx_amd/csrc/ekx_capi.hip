@@ -1551,10 +1551,13 @@ struct Engine3D
                                    stream));
         }
         EKX_HIP(hipStreamSynchronize(stream));
+        bool moved = false;
         for (int i = 0; i < n; ++i)
         {
             Problem3D &p = problems[i];
             const SourceInfo &s = sources[i];
+            moved = moved || p.srcCellX != s.cell[0] ||
+                    p.srcCellY != s.cell[1] || p.srcCellZ != s.cell[2];
             p.srcCellX = s.cell[0];
             p.srcCellY = s.cell[1];
             p.srcCellZ = s.cell[2];
@@ -1564,6 +1567,8 @@ struct Engine3D
             p.srcSlowness = sSrc[i];
             if (SQ.ptr) { set_fixed32_steps(i); }
         }
+        // the diagonals that get factored launches are in captured graphs
+        if (moved && !mergedSmall) { drop_graph(); }
         EKX_HIP(hipMemcpyAsync(dProblems.ptr, problems.data(),
                                problems.size()*sizeof(Problem3D),
                                hipMemcpyHostToDevice, stream));
