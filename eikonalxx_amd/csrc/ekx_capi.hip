@@ -31,7 +31,7 @@ constexpr size_t kMaxPartials = 1024;
 constexpr int kRangeBlocks = 256;
 // Column z-chunk depths the launch-shape choice considers (0: whole
 // columns), longest first.
-constexpr int kChunkCandidates[] = {0, 96, 64, 48, 32, 24, 16, 12, 8};
+constexpr int kChunkCandidates[] = {0, 128, 96, 64, 48, 32, 24, 16, 12, 8};
 // Independent launch chains of a batch (one stream each).
 constexpr int kMaxChains = 16;
 
@@ -1204,8 +1204,7 @@ struct Engine3D
         // counts.  The chunk depth is chosen for that instance's
         // occupancy and kept when the separate instances take over: asked
         // again at their higher occupancy the size-class rule would pick
-        // shorter chunks, which measured slower (the FP32 tables: 96-plane
-        // chunks 1106 ms per solve, whole columns 866 ms).
+        // shorter chunks, which measured slower.
         chunkH = o.chunk_planes > 0 ? std::min(o.chunk_planes, maxNz)
                                     : even_chunk(auto_chunk(geoms, maxNz),
                                                  maxNz);
@@ -1387,15 +1386,16 @@ struct Engine3D
     }
 
     // Planes per z-chunk when the caller leaves the choice
-    // (chunk_planes = 0), by size class: the longest of whole columns, 96,
-    // 64, 48, 32, 24, 16, 12 or 8 planes whose column diagonals hold on
-    // average at least 1.5 times the column waves the device keeps
+    // (chunk_planes = 0), by size class: the longest of whole columns (up to
+    // 128 planes), 128, 96, 64, 48, 32, 24, 16, 12 or 8 planes whose column
+    // diagonals hold on average at least 1.5 times the column waves the device keeps
     // resident of the bulk instance that also runs the box chunks.
     // Shorter chunks put more column-chunks on each diagonal (a sweep's
     // dependency chain is nbx + nby + nbz - 2 launches) at the price of
     // the 15-step lane skew at both ends of every chunk.  Measured on the
-    // MI355X: the 256-source 385 x 385 x 193 tables run fastest with whole
-    // columns, a 64-problem batch of 96..320-point grids with 32 planes, a
+    // MI355X: the 256-source 385 x 385 x 193 tables run fastest with two
+    // chunks of 97 planes (1 iteration: whole columns 475 ms, 97 460, 65 471,
+    // 49 547; FP32 283, 270, 270, 394), a 64-problem batch of 96..320-point grids with 32 planes, a
     // single 257 x 257 x 193 or 129^3 grid with 8 (4.5x and 3x faster than
     // whole columns); every choice gives the same field.
     int auto_chunk(const std::vector<ekx_geometry3d> &geoms, int maxNz) const
@@ -1420,6 +1420,7 @@ struct Engine3D
         const double want = 1.5*cus*perCU;
         for (int c : kChunkCandidates)
         {
+            if (c == 0 && maxNz > 128) { continue; }
             const int h = c == 0 ? maxNz : std::min(c, maxNz);
             double items = 0;
             int diags = 1;

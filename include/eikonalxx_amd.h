@@ -139,7 +139,7 @@ typedef struct
                                       a column (chunks run on diagonals
                                       bx+by+bz, shortening the dependency
                                       chain of a sweep); 0 (default): chosen
-                                      by size class (whole columns for
+                                      by size class (up to 128 planes for
                                       large batches, down to 8 planes for
                                       one grid); results do not depend on
                                       it                                   */
@@ -149,8 +149,14 @@ typedef struct
                                       take the chunks from a work queue in
                                       diagonal order and start each once
                                       its upwind chunks are done; 0
-                                      (default) chooses.  Results do not
-                                      depend on it                         */
+                                      (default) chooses: with chunk_planes,
+                                      chains and prefetch_planes 0 too,
+                                      COMPLETED solves in FP64, FP32 and
+                                      FP32_POLISH run as one launch (a
+                                      resident wave per column) unless the
+                                      diagonals would fill the device;
+                                      else one launch per diagonal.
+                                      Results do not depend on it          */
 } ekx_solver_options;
 
 /* Geometry3D (include/eikonalxx/geometry3d.hpp:50-160). */
