@@ -543,6 +543,7 @@ struct Engine3D
     // kMergedMaxChunk planes)
     bool mergedSmall = false;
     static constexpr int kMergedMaxChunk = 64;
+    static constexpr int kMergedMaxChunk64 = 80;    // FP64, default shapes
     std::vector<int> chainBegin;
     std::vector<hipStream_t> chainStreams;
     std::vector<hipEvent_t> chainEvents;
@@ -1208,7 +1209,11 @@ struct Engine3D
         chunkH = o.chunk_planes > 0 ? std::min(o.chunk_planes, maxNz)
                                     : even_chunk(auto_chunk(geoms, maxNz),
                                                  maxNz);
-        mergedSmall = chunkH < kMergedMaxChunk;
+        // (64 FP64 sources on 385 x 385 x 193, chunks of 65: 164 ms with
+        // launches of their own for the box, 154 without; FP32 108 and 115)
+        mergedSmall = chunkH < kMergedMaxChunk ||
+                      (sweeps_f64() && o.chunk_planes == 0 &&
+                       o.prefetch_planes == 0 && chunkH < kMergedMaxChunk64);
         nDiag = 0;
         for (int i = 0; i < n; ++i)
         {
@@ -1431,7 +1436,9 @@ struct Engine3D
                 items += (double) nbx*nby*nbz;
                 diags = std::max(diags, nbx + nby + nbz - 2);
             }
-            if (items/diags >= want) { return h; }
+            // (64 sources on 385 x 385 x 193: chunks of 97 planes 171 ms, 65
+            // 164; 128 sources 263 and 262; 256 sources 460 and 471)
+            if (items/diags >= (h > 96 ? 2*want : want)) { return h; }
         }
         return std::min(8, maxNz);
     }
