@@ -1391,17 +1391,18 @@ struct Engine3D
     }
 
     // Planes per z-chunk when the caller leaves the choice
-    // (chunk_planes = 0), by size class: the longest of whole columns (up to
-    // 128 planes), 128, 96, 64, 48, 32, 24, 16, 12 or 8 planes whose column
-    // diagonals hold on average at least 1.5 times the column waves the device keeps
-    // resident of the bulk instance that also runs the box chunks.
+    // (chunk_planes = 0), by size class: the longest of whole
+    // columns, 128, 96, 64, 48, 32, 24, 16, 12 or 8 planes whose column
+    // diagonals hold on average at least 1.5 times (above 96 planes, 3 times)
+    // the column waves the device keeps resident of the bulk instance that
+    // also runs the box chunks.
     // Shorter chunks put more column-chunks on each diagonal (a sweep's
     // dependency chain is nbx + nby + nbz - 2 launches) at the price of
     // the 15-step lane skew at both ends of every chunk.  Measured on the
-    // MI355X: the 256-source 385 x 385 x 193 tables run fastest with two
-    // chunks of 97 planes (1 iteration: whole columns 475 ms, 97 460, 65 471,
-    // 49 547; FP32 283, 270, 270, 394), a 64-problem batch of 96..320-point grids with 32 planes, a
-    // single 257 x 257 x 193 or 129^3 grid with 8 (4.5x and 3x faster than
+    // MI355X: the 256-source 385 x 385 x 193 tables run fastest with whole
+    // columns (FP64, 4 iterations: 1570 ms, chunks of 97 planes 1613), 128
+    // sources with 97 planes (1 iteration: 297 and 263 ms), a 64-problem
+    // batch of 96..320-point grids with 32 planes, a single 257 x 257 x 193 or 129^3 grid with 8 (4.5x and 3x faster than
     // whole columns); every choice gives the same field.
     int auto_chunk(const std::vector<ekx_geometry3d> &geoms, int maxNz) const
     {
@@ -1425,7 +1426,6 @@ struct Engine3D
         const double want = 1.5*cus*perCU;
         for (int c : kChunkCandidates)
         {
-            if (c == 0 && maxNz > 128) { continue; }
             const int h = c == 0 ? maxNz : std::min(c, maxNz);
             double items = 0;
             int diags = 1;
@@ -1437,7 +1437,7 @@ struct Engine3D
                 diags = std::max(diags, nbx + nby + nbz - 2);
             }
             // (64 sources on 385 x 385 x 193: chunks of 97 planes 171 ms, 65
-            // 164; 128 sources 263 and 262; 256 sources 460 and 471)
+            // 164; 128 sources: whole columns 297 ms, 97 planes 263)
             if (items/diags >= (h > 96 ? 2*want : want)) { return h; }
         }
         return std::min(8, maxNz);

@@ -139,7 +139,7 @@ typedef struct
                                       a column (chunks run on diagonals
                                       bx+by+bz, shortening the dependency
                                       chain of a sweep); 0 (default): chosen
-                                      by size class (up to 128 planes for
+                                      by size class (whole columns for
                                       large batches, down to 8 planes for
                                       one grid); results do not depend on
                                       it                                   */
