@@ -1588,8 +1588,12 @@ struct Engine3D
             p.srcSlowness = sSrc[i];
             if (SQ.ptr) { set_fixed32_steps(i); }
         }
-        // the diagonals that get factored launches are in captured graphs
-        if (moved && !mergedSmall) { drop_graph(); }
+        // captured graphs hold the diagonals that get factored launches, and
+        // the hyperplane kernel's levels and their sizes
+        if (moved && (!mergedSmall || kernel() == EKX_KERNEL_HYPERPLANE))
+        {
+            drop_graph();
+        }
         EKX_HIP(hipMemcpyAsync(dProblems.ptr, problems.data(),
                                problems.size()*sizeof(Problem3D),
                                hipMemcpyHostToDevice, stream));

@@ -131,7 +131,7 @@ sweep_hyperplane3d(const Problem3D *__restrict__ problems, int problem,
     const int jz = kLo + pid/nyRange;
     const int jy = o.jy0 + pid%nyRange;
     const int jx = level - jy - jz;
-    if (jx < o.jx0 || jx > p.nx - 1) { return; }
+    if (jx < o.jx0 || jx > p.nx - 1 || jz > p.nz - 1) { return; }
     const int negX = sweep & 1, negY = (sweep >> 1) & 1, negZ = (sweep >> 2) & 1;
     const int nx = p.nx, ny = p.ny, nz = p.nz;
     const int ncx = nx - 1, ncy = ny - 1, ncz = nz - 1;
