@@ -562,6 +562,7 @@ struct Engine3D
     int queueMaxSweeps = 0;
     int queueWaves = 0;          // column waves the device keeps resident
     uint64_t queueWaitTicks = 0; // bound of one dependency wait
+    int clockKHz = 0;            // rate of the device's wall clock
     // Flow launches (a whole solve in one launch, every column resident):
     // the columns of all problems in launch order and, per element type
     // swept, two buffers of step records and four of mail; the error word
@@ -575,6 +576,8 @@ struct Engine3D
     int64_t flowRecCount = 0, flowMailCount = 0;
     int flowCapacity = 0;        // waves that the device holds together
     int flowMaxNz = 0;
+    int64_t flowSteps = 0;       // flow_chain of all waves
+    int64_t flowChain = 0;       // and of the longest
     bool flowUniform = false;
     hipStream_t stream = nullptr;
     hipEvent_t evFork = nullptr;
@@ -851,8 +854,8 @@ struct Engine3D
     // With more columns than waves the problems follow each other through
     // the device, the longest chains first: a column waits only for columns
     // of its own problem, and workgroups of an XCD start in launch order, so
-    // the first unfinished problem always becomes resident as a whole (the
-    // bound on waits holds all the same).  That is faster than the diagonals
+    // the first unfinished problem always becomes resident as a whole.  That
+    // is faster than the diagonals
     // until these have enough columns to fill the chip: measured on FP64
     // grids of 64 to 200 nodes a side, by the ratio of all the waves' steps
     // to what the device runs in the longest chain: 1.2 27.5 -> 15.3 ms, 2.0
@@ -861,6 +864,25 @@ struct Engine3D
     // Memory that the device does not have for the buffers is no error: the
     // diagonals need none of it.
     static constexpr int64_t kFlowLoad2 = 7;
+
+    // The bound of one wait in a flow launch of nSweeps sweeps, in the
+    // device's wall clock.  With every column resident a wait lasts a few
+    // traversals of a problem at most; otherwise a column may wait until the
+    // problems before its own have done all their sweeps, which is the
+    // launch's whole time.  At 4 us a step (0.5 to 1.5 measured), 4 traversals,
+    // and at least 250 ms, so that a device shared with other work does not
+    // trip it.
+    uint64_t flow_wait_ticks(int nSweeps) const
+    {
+        constexpr double kStepMs = 4e-3;
+        const double chain = 0.5*(double) flowChain;
+        double steps = 4*chain;
+        if (flowWaves > flowCapacity)
+        {
+            steps += nSweeps*(0.5*(double) flowSteps/flowCapacity + chain);
+        }
+        return (uint64_t) (clockKHz*std::max(250.0, kStepMs*steps));
+    }
 
     // Twice the steps that a wave of problem p spends in a sweep, waits for
     // the hops to its columns included (a hop is 10.6 steps; x reverses in
@@ -881,15 +903,15 @@ struct Engine3D
             o.chains == 0 && o.prefetch_planes == 0;
         int device = 0, cus = 0;
         int64_t most = 0;               // columns of one problem
-        int64_t steps = 0, chain = 0;   // of all waves, of the longest wave
         int uniform = 0;
         flowMaxNz = 0;
+        flowSteps = flowChain = 0;
         for (const Problem3D &p : problems)
         {
             const int64_t columns = (int64_t) p.nTX*p.nTY;
             most = std::max(most, columns);
-            steps += columns*flow_chain(p);
-            chain = std::max(chain, flow_chain(p));
+            flowSteps += columns*flow_chain(p);
+            flowChain = std::max(flowChain, flow_chain(p));
             uniform += p.uniform;
             flowMaxNz = std::max(flowMaxNz, p.nz);
         }
@@ -911,7 +933,7 @@ struct Engine3D
             }
             flowCapacity = perCU*cus;
             fits = most <= flowCapacity &&
-                   2*steps <= kFlowLoad2*flowCapacity*chain;
+                   2*flowSteps <= kFlowLoad2*flowCapacity*flowChain;
         }
         else { fits = false; }
         int64_t rec = 0, mail = 0;
@@ -1096,7 +1118,8 @@ struct Engine3D
         EKX_HIP(launch_flow3d<TS>(
             dProblems.ptr, dFlowColumns.ptr, n, nInit, nSweeps, rec,
             flowRecCount, mail, flowMailCount, bricks<TS>(), flowUniform,
-            flowWords.ptr, flowWords.ptr + 1, queueWaitTicks, stream));
+            flowWords.ptr, flowWords.ptr + 1, flow_wait_ticks(nSweeps),
+            stream));
         EKX_HIP(launch_flow_copy<TS>(
             dProblems.ptr, dFlowColumns.ptr, n, flowMaxNz, nSweeps & 7, false,
             rec + (nSweeps & 1)*flowRecCount, T, stream));
@@ -1319,11 +1342,11 @@ struct Engine3D
             // the sweeps run at 1e10 and more), so that a device shared
             // with other work does not trip it.  A wait past the bound
             // makes the solve fail with EKX_EHIP and its field is void.
-            int kHz = 0;
-            if (hipDeviceGetAttribute(&kHz, hipDeviceAttributeWallClockRate,
-                                      device) != hipSuccess || kHz <= 0)
+            if (hipDeviceGetAttribute(&clockKHz,
+                                      hipDeviceAttributeWallClockRate,
+                                      device) != hipSuccess || clockKHz <= 0)
             {
-                kHz = 100000;
+                clockKHz = 100000;
             }
             int64_t chainNodes = 0;
             for (int c = 0; c < nChains; ++c)
@@ -1337,7 +1360,7 @@ struct Engine3D
                 chainNodes = std::max(chainNodes, nodes);
             }
             const double ms = std::max(250.0, 4.0e-6*(double) chainNodes);
-            queueWaitTicks = (uint64_t) ((double) kHz*ms);
+            queueWaitTicks = (uint64_t) ((double) clockKHz*ms);
         }
         return EKX_OK;
     }
