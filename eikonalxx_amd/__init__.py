@@ -183,6 +183,7 @@ EXPORTED_SYMBOLS = [
     "ekx_solver2d_get_travel_time_gradient_field",
     "ekx_model3d_layered_gaussian", "ekx_solver3d_set_layered_gaussian_model",
     "ekx_solver3d_autotune", "ekx_batch3d_autotune",
+    "ekx_solver3d_set_wait_bound", "ekx_batch3d_set_wait_bound",
     "ekx_batch2d_create", "ekx_batch2d_destroy", "ekx_batch2d_initialize",
     "ekx_batch2d_solve", "ekx_batch2d_get_travel_times",
     "ekx_batch2d_get_stats",
@@ -291,6 +292,8 @@ def _declare(L):
     L.ekx_solver2d_compute_travel_time_gradient_field.argtypes = [_P]
     L.ekx_solver2d_have_travel_time_gradient_field.argtypes = [_P]
     L.ekx_solver2d_get_travel_time_gradient_field.argtypes = [_P, _I64, _PD]
+    for name in ("ekx_solver3d_set_wait_bound", "ekx_batch3d_set_wait_bound"):
+        getattr(L, name).argtypes = [_P, _D]
     for name in ("ekx_solver3d_autotune", "ekx_batch3d_autotune"):
         getattr(L, name).argtypes = [_P, ctypes.POINTER(_I),
                                      ctypes.POINTER(_I)]
@@ -548,6 +551,12 @@ class Solver3D:
                                              ctypes.byref(n)))
         return c.value, n.value
 
+    def set_wait_bound(self, ms):
+        """Longest wait (ms) of a solve in one launch before it is repeated
+        by launches per diagonal, as are all later solves until the next
+        initialize; negative: the default."""
+        _check(self._L.ekx_solver3d_set_wait_bound(self._h, float(ms)))
+
     def have_travel_time_field(self):
         return bool(self._L.ekx_solver3d_have_travel_time_field(self._h))
 
@@ -686,6 +695,10 @@ class Batch3D:
         _check(self._L.ekx_batch3d_autotune(self._h, ctypes.byref(c),
                                             ctypes.byref(n)))
         return c.value, n.value
+
+    def set_wait_bound(self, ms):
+        """As Solver3D.set_wait_bound."""
+        _check(self._L.ekx_batch3d_set_wait_bound(self._h, float(ms)))
 
     def get_travel_time_field(self, problem):
         n = self._geoms[problem].n_grid

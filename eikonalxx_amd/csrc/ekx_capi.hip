@@ -578,6 +578,7 @@ struct Engine3D
     int flowMaxNz = 0;
     int64_t flowSteps = 0;       // flow_chain of all waves
     int64_t flowChain = 0;       // and of the longest
+    double flowWaitMs = -1;      // a caller's bound of one wait
     bool flowUniform = false;
     hipStream_t stream = nullptr;
     hipEvent_t evFork = nullptr;
@@ -874,6 +875,7 @@ struct Engine3D
     // trip it.
     uint64_t flow_wait_ticks(int nSweeps) const
     {
+        if (flowWaitMs >= 0) { return (uint64_t) (clockKHz*flowWaitMs); }
         constexpr double kStepMs = 4e-3;
         const double chain = 0.5*(double) flowChain;
         double steps = 4*chain;
@@ -882,6 +884,16 @@ struct Engine3D
             steps += nSweeps*(0.5*(double) flowSteps/flowCapacity + chain);
         }
         return (uint64_t) (clockKHz*std::max(250.0, kStepMs*steps));
+    }
+
+    ekx_status set_wait_bound(double ms)
+    {
+        if (ms > 1e9)
+        {
+            return fail(EKX_EINVAL, "wait bound must be at most 1e9 ms");
+        }
+        flowWaitMs = ms;
+        return EKX_OK;
     }
 
     // Twice the steps that a wave of problem p spends in a sweep, waits for
@@ -895,6 +907,7 @@ struct Engine3D
     ekx_status setup_flow()
     {
         flowColumns.clear();
+        flowWaitMs = -1;
         const ekx_solver_options &o = opt;
         const bool wanted =
             kernel() == EKX_KERNEL_COLUMN && !fixed32() && !early_exit() &&
@@ -2200,9 +2213,15 @@ struct Engine3D
             if (take_flow(r)) { EKX_CHECK(solve_fields(true, flowFailed)); }
             else { EKX_CHECK(solve_fields(false, flowFailed)); }
         }
-        // a wait of the flow launch exceeded its bound (the device was
-        // shared with work that kept columns out): once more by diagonals
-        if (flowFailed) { EKX_CHECK(solve_fields(false, flowFailed)); }
+        // A wait of the flow launch exceeded its bound (the device is shared
+        // with work that keeps columns out): once more by diagonals, and so
+        // every later solve of this setup, which would wait out the bound
+        // again otherwise.
+        if (flowFailed)
+        {
+            release_flow();
+            EKX_CHECK(solve_fields(false, flowFailed));
+        }
         haveField = true;
         solveStamp += 1;
         if (nStations > 0) { EKX_CHECK(compute_stations()); }
@@ -3006,6 +3025,15 @@ ekx_status ekx_solver3d_solve(ekx_solver3d *h)
     });
 }
 
+ekx_status ekx_solver3d_set_wait_bound(ekx_solver3d *h, double ms)
+{
+    return guarded([&]() -> ekx_status
+    {
+        EKX_CHECK(require_initialized(h));
+        return h->engine.set_wait_bound(ms);
+    });
+}
+
 ekx_status ekx_solver3d_autotune(ekx_solver3d *h, int *chunk_planes,
                                  int *chains)
 {
@@ -3325,6 +3353,15 @@ ekx_status ekx_batch3d_solve(ekx_batch3d *h)
     {
         EKX_CHECK(require_batch(h));
         return h->engine.solve();
+    });
+}
+
+ekx_status ekx_batch3d_set_wait_bound(ekx_batch3d *h, double ms)
+{
+    return guarded([&]() -> ekx_status
+    {
+        EKX_CHECK(require_batch(h));
+        return h->engine.set_wait_bound(ms);
     });
 }
 

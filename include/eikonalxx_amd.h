@@ -278,6 +278,14 @@ EKX_API ekx_status ekx_solver3d_solve(ekx_solver3d *solver);
  * chains (each may be NULL) receive the choice. */
 EKX_API ekx_status ekx_solver3d_autotune(ekx_solver3d *solver,
                                          int *chunk_planes, int *chains);
+/* No reference counterpart.  Longest time (ms) that a wave of a solve in one
+ * launch (launch_order 0) waits for another: past it the solve is repeated
+ * by launches per diagonal, as are all later solves until the next
+ * initialize, which also restores the default.  Negative: the default, at
+ * least 250 ms and more where problems wait for others to finish.  For
+ * devices shared with other processes, where columns can be kept out. */
+EKX_API ekx_status ekx_solver3d_set_wait_bound(ekx_solver3d *solver,
+                                               double ms);
 /* Solver3D::haveTravelTimeField (src/solver3d.cpp:510-514). */
 EKX_API int ekx_solver3d_have_travel_time_field(const ekx_solver3d *solver);
 /* Solver3D::getTravelTimeField (solver3d.hpp:137, src/solver3d.cpp:
@@ -401,6 +409,8 @@ EKX_API ekx_status ekx_batch3d_solve(ekx_batch3d *batch);
  * batch; the fastest is kept. */
 EKX_API ekx_status ekx_batch3d_autotune(ekx_batch3d *batch,
                                         int *chunk_planes, int *chains);
+/* As ekx_solver3d_set_wait_bound. */
+EKX_API ekx_status ekx_batch3d_set_wait_bound(ekx_batch3d *batch, double ms);
 EKX_API ekx_status ekx_batch3d_get_travel_times(const ekx_batch3d *batch,
                                                 int problem, int64_t n,
                                                 double *out);

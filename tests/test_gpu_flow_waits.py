@@ -1,5 +1,6 @@
 """Waits of the one-launch solves: their bound follows the number of sweeps
-where problems wait for others to finish."""
+where problems wait for others to finish, and past the bound the solve, and
+those after it, go by diagonals."""
 import numpy as np
 import pytest
 
@@ -31,3 +32,54 @@ def test_a_problem_waits_for_another_to_finish(ekx):
         assert s.get_stats().kernel_launches == 1
         assert np.array_equal(s.get_travel_time_field(),
                               b.get_travel_time_field(k)), k
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FP32_POLISH"])
+@pytest.mark.parametrize("batch", [False, True])
+def test_past_the_bound_by_diagonals(ekx, oracle, precision, batch):
+    """A bound that no wait meets: every wave gives up and ends, and the
+    field is the diagonals'."""
+    dims, h = (129, 73, 21), 10.0
+    rng = np.random.default_rng(12)
+    slow = 1.0 / rng.uniform(1800.0, 5200.0, 128 * 72 * 20)
+    g = ekx.Geometry3D(*dims, h)
+    src = (700.0, 310.0, 95.0)
+    print("case", precision, batch, flush=True)
+
+    def make(chunk):
+        o = ekx.SolverOptions(number_of_sweeps=2, factored_radius=2,
+                              chunk_planes=chunk,
+                              precision=getattr(ekx.Precision, precision))
+        s = ekx.Batch3D() if batch else ekx.Solver3D()
+        if batch:
+            s.initialize(o, [(g, slow, src)] * 2)
+            return s, lambda: s.get_travel_time_field(1)
+        s.initialize(o, g)
+        s.set_slowness(slow)
+        s.set_source(src)
+        return s, s.get_travel_time_field
+
+    by_diagonals, field = make(8)
+    by_diagonals.solve()
+    ref = field()
+    if precision == "FP64":
+        assert np.array_equal(ref, oracle.solve3d(
+            oracle.geometry3d(*dims, h), slow, src, 2, 2))
+    one = 1 if precision == "FP64" else 2
+    s, field = make(0)
+    s.set_wait_bound(0.0)
+    s.solve()
+    assert s.get_stats().kernel_launches > one
+    assert np.array_equal(field(), ref)
+    # the device stays shared: no second try
+    s.set_wait_bound(-1.0)
+    s.solve()
+    assert s.get_stats().kernel_launches > one
+    assert np.array_equal(field(), ref)
+    # a new setup tries again
+    s, field = make(0)
+    s.solve()
+    assert s.get_stats().kernel_launches == one
+    assert np.array_equal(field(), ref)
+    with pytest.raises(ValueError):
+        s.set_wait_bound(1e10)
