@@ -600,6 +600,7 @@ struct Engine3D
         hipGraphExec_t exec = nullptr;
         bool valid = false;
         ekx_solve_stats st{};
+        uint64_t sourceStamp = 0;       // the sources that st counts for
         void release()
         {
             if (exec) { (void) hipGraphExecDestroy(exec); }
@@ -619,6 +620,7 @@ struct Engine3D
     // Count of completed solves: derived results record the solve they
     // were computed from.
     uint64_t solveStamp = 0;
+    uint64_t sourceStamp = 0;    // count of moves of a source cell
     // Receivers: nStations per problem, located in every problem's grid
     // (dStations is [problem][station]); their travel times after the
     // solve numbered stationStamp.
@@ -1637,6 +1639,7 @@ struct Engine3D
             p.srcSlowness = sSrc[i];
             if (SQ.ptr) { set_fixed32_steps(i); }
         }
+        if (moved) { sourceStamp += 1; }
         if (moved && captures_source()) { drop_graph(); }
         EKX_HIP(hipMemcpyAsync(dProblems.ptr, problems.data(),
                                problems.size()*sizeof(Problem3D),
@@ -1712,7 +1715,6 @@ struct Engine3D
     ekx_status enqueue_sweep(int sweep, bool initialize, TS *T, const TS *S,
                              unsigned int epoch, ekx_solve_stats &st)
     {
-        count_sweep<TS>(sweep, initialize, st);
         int64_t launches = 0;
         ekx_status rc = enqueue_sweep_launches<TS>(sweep, initialize, T, S,
                                                    epoch, launches);
@@ -1906,9 +1908,10 @@ struct Engine3D
         return EKX_OK;
     }
 
-    template <typename TS>
-    ekx_status enqueue_phase_sweeps(TS *T, const TS *S, bool doInit,
-                                    int iterations, ekx_solve_stats &st)
+    // The sweeps of one precision segment (sweep, initialisation sweep) and
+    // the refinement iterations among them.
+    std::vector<std::pair<int, bool>> sweep_list(bool doInit,
+                                                 int &iterations) const
     {
         std::vector<std::pair<int, bool>> list;
         if (doInit)
@@ -1931,6 +1934,25 @@ struct Engine3D
         {
             for (int s = 0; s < 8; ++s) { list.push_back({s, false}); }
         }
+        return list;
+    }
+
+    template <typename TS>
+    void count_segment(bool doInit, int iterations, ekx_solve_stats &st) const
+    {
+        for (const auto &sw : sweep_list(doInit, iterations))
+        {
+            count_sweep<TS>(sw.first, sw.second, st);
+        }
+    }
+
+    template <typename TS>
+    ekx_status enqueue_phase_sweeps(TS *T, const TS *S, bool doInit,
+                                    int iterations, ekx_solve_stats &st)
+    {
+        count_segment<TS>(doInit, iterations, st);
+        const std::vector<std::pair<int, bool>> list =
+            sweep_list(doInit, iterations);
         if (queued<TS>())
         {
             // a new sequence of work-queue sweeps: flags and counters back
@@ -1953,10 +1975,6 @@ struct Engine3D
         {
             // Chains run their whole sweep list independently: fork from
             // the main stream, join back at the end.
-            for (const auto &sw : list)
-            {
-                count_sweep<TS>(sw.first, sw.second, st);
-            }
             int64_t launches = 0;
             EKX_HIP(hipEventRecord(evFork, stream));
             for (int c = 0; c < nChains; ++c)
@@ -2013,7 +2031,17 @@ struct Engine3D
                                                 nullptr, 0));
                 }
                 g.st = local;
+                g.sourceStamp = sourceStamp;
                 g.valid = true;
+            }
+            else if (g.sourceStamp != sourceStamp)
+            {
+                // the octants and the box moved with the sources
+                count_segment<TS>(doInit, iterations, local);
+                g.st.updates = local.updates;
+                g.st.updates_fp64 = local.updates_fp64;
+                g.st.updates_factored = local.updates_factored;
+                g.sourceStamp = sourceStamp;
             }
             local = g.st;
             if (g.exec) { EKX_HIP(hipGraphLaunch(g.exec, stream)); }

@@ -1,0 +1,35 @@
+"""Work counts after a source has moved: those of a solver that starts there,
+also where a captured graph is replayed."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("precision", ["FP64", "FIXED32", "FP32_POLISH"])
+@pytest.mark.parametrize("chunk", [0, 8, 70])
+def test_counts_follow_the_source(ekx, precision, chunk):
+    dims, h = (40, 24, 70), 10.0
+    slow = np.full(39 * 23 * 69, 1.0 / 3000.0)
+    sources = [(25.0, 31.0, 44.0), (371.0, 202.0, 655.0), (201.0, 99.0, 8.0)]
+
+    def make():
+        s = ekx.Solver3D()
+        s.initialize(ekx.SolverOptions(
+            number_of_sweeps=2, factored_radius=3, chunk_planes=chunk,
+            precision=getattr(ekx.Precision, precision),
+            launch_order=ekx.LaunchOrder.DIAGONALS),
+            ekx.Geometry3D(*dims, h))
+        s.set_slowness(slow)
+        return s
+    moving = make()
+    for src in sources:
+        counts = []
+        for s in (moving, make()):
+            s.set_source(src)
+            s.solve()
+            st = s.get_stats()
+            counts.append((st.updates, st.updates_fp64, st.updates_factored,
+                           st.iterations_run, st.kernel_launches))
+        print("case", precision, chunk, src, counts, flush=True)
+        assert counts[0] == counts[1]
