@@ -544,6 +544,8 @@ struct Engine3D
     bool mergedSmall = false;
     static constexpr int kMergedMaxChunk = 64;
     static constexpr int kMergedMaxChunk64 = 80;    // FP64, default shapes
+    // the autotuner's choice (0: none)
+    int tunedChunk = 0, tunedChains = 0;
     std::vector<int> chainBegin;
     std::vector<hipStream_t> chainStreams;
     std::vector<hipEvent_t> chainEvents;
@@ -716,6 +718,7 @@ struct Engine3D
         nStations = 0;
         stationTimes.clear();
         gradientProblem = -1;
+        tunedChunk = tunedChains = 0;
         if (!stream)
         {
             EKX_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
@@ -1192,6 +1195,13 @@ struct Engine3D
         while (!out.empty() && out.back().problem < 0) { out.pop_back(); }
     }
 
+    int default_chains() const
+    {
+        const int n = (int) geometry.size();
+        return opt.chains > 0 ? std::min(opt.chains, n)
+                              : (n >= 16 ? std::min(4, n) : 1);
+    }
+
     // The launch schedule of the current options: chains, the z-chunk
     // depth and the column-chunk work lists by chain and diagonal.
     ekx_status build_schedule()
@@ -1207,8 +1217,8 @@ struct Engine3D
         {
             naturalNodes += (int64_t) g.nx*g.ny*g.nz;
         }
-        nChains = o.chains > 0 ? std::min(o.chains, n)
-                               : (n >= 16 ? std::min(4, n) : 1);
+        nChains = tunedChains > 0 ? std::min(tunedChains, n)
+                                  : default_chains();
         if (kernel() != EKX_KERNEL_COLUMN) { nChains = 1; }
         chainBegin.assign(1, 0);
         {
@@ -1247,9 +1257,10 @@ struct Engine3D
         // occupancy and kept when the separate instances take over: asked
         // again at their higher occupancy the size-class rule would pick
         // shorter chunks, which measured slower.
-        chunkH = o.chunk_planes > 0 ? std::min(o.chunk_planes, maxNz)
-                                    : even_chunk(auto_chunk(geoms, maxNz),
-                                                 maxNz);
+        chunkH = tunedChunk > 0       ? std::min(tunedChunk, maxNz)
+                 : o.chunk_planes > 0 ? std::min(o.chunk_planes, maxNz)
+                                      : even_chunk(auto_chunk(geoms, maxNz),
+                                                   maxNz);
         // (64 FP64 sources on 385 x 385 x 193, chunks of 65: 164 ms with
         // launches of their own for the box, 154 without; FP32 108 and 115)
         mergedSmall = chunkH < kMergedMaxChunk ||
@@ -2099,10 +2110,11 @@ struct Engine3D
     }
 
     // One short solve for the autotuner: the initialisation sweeps and one
-    // refinement iteration, run as later solves run (the captured graph,
-    // unless use_graph is off): once to capture, then timed; device ms.
+    // refinement iteration, run as later solves run (in one launch, or the
+    // captured graph, unless use_graph is off): once to capture, then timed;
+    // device ms.
     template <typename TS>
-    ekx_status trial_run(TS *T, const TS *S, float &ms)
+    ekx_status trial_run(TS *T, const TS *S, bool flow, float &ms)
     {
         const int nProb = (int) problems.size();
         ekx_solve_stats st{};
@@ -2110,9 +2122,14 @@ struct Engine3D
         for (int pass = 0; pass < 2; ++pass)
         {
             EKX_HIP(hipEventRecord(evStart, stream));
-            EKX_HIP(launch_init3d<TS>(dProblems.ptr, nProb, totalNodes, T,
-                                      stream));
-            EKX_CHECK(run_segment<TS>(0, T, S, true, 1, st));
+            if constexpr (std::is_same<TS, uint32_t>::value) { flow = false; }
+            else if (flow) { EKX_CHECK(run_flow<TS>(T, true, 1, st)); }
+            if (!flow)
+            {
+                EKX_HIP(launch_init3d<TS>(dProblems.ptr, nProb, totalNodes, T,
+                                          stream));
+                EKX_CHECK(run_segment<TS>(0, T, S, true, 1, st));
+            }
             EKX_HIP(hipEventRecord(evStop, stream));
             EKX_HIP(hipEventSynchronize(evStop));
             EKX_CHECK(check_queue_error());
@@ -2121,19 +2138,53 @@ struct Engine3D
         return EKX_OK;
     }
 
-    ekx_status trial_ms(float &ms)
+    ekx_status trial_ms(bool flow, float &ms)
     {
         EKX_CHECK(prepare_sources());
-        if (sweeps_f64()) { return trial_run<double>(T64.ptr, S64.ptr, ms); }
-        if (fixed32()) { return trial_run<uint32_t>(TQ.ptr, SQ.ptr, ms); }
-        return trial_run<float>(T32.ptr, S32.ptr, ms);
+        if (sweeps_f64())
+        {
+            return trial_run<double>(T64.ptr, S64.ptr, flow, ms);
+        }
+        if (fixed32())
+        {
+            return trial_run<uint32_t>(TQ.ptr, SQ.ptr, flow, ms);
+        }
+        return trial_run<float>(T32.ptr, S32.ptr, flow, ms);
+    }
+
+    // Time of the solve in one launch; ms < 0: this setup has none, or it
+    // gave up (and is given up for later solves too).
+    ekx_status trial_flow(float &ms)
+    {
+        ms = -1;
+        FlowReservation r;
+        if (!take_flow(r)) { return EKX_OK; }
+        EKX_CHECK(trial_ms(true, ms));
+        unsigned int err = 0;
+        EKX_CHECK(copy_out(&err, flowWords.ptr, sizeof(err)));
+        if (err != 0)
+        {
+            release_flow();
+            ms = -1;
+        }
+        return EKX_OK;
+    }
+
+    // The schedule of a launch shape (0, 0: the default).
+    ekx_status use_shape(int chunk, int chains)
+    {
+        tunedChunk = chunk;
+        tunedChains = chains;
+        drop_graph();
+        return build_schedule();
     }
 
     // Measured choice of the launch shape (no reference counterpart): times
     // a short solve for z-chunk depths around the size-class default (the
     // default and its neighbours in auto_chunk's list) and 1, 2 or 4
-    // chains, and keeps the fastest for later solves.  Fields do not
-    // depend on the choice; the field of the last solve is discarded.
+    // chains, and the solve in one launch where the setup has it, and keeps
+    // the fastest for later solves.  Fields do not depend on the choice; the
+    // field of the last solve is discarded.
     ekx_status autotune(int &chunkOut, int &chainsOut)
     {
         if (!haveModel)
@@ -2176,14 +2227,12 @@ struct Engine3D
             {
                 if (c <= n) { tryChains.push_back(c); }
             }
-            const ekx_solver_options saved = opt;
             float best = 0;
             int bestDepth = h0, bestChains = 1;
             bool first = true;
             // the default shape first; another replaces the best only when
             // it is more than 3% faster (trial times vary by about that)
-            const int c0 = saved.chains > 0 ? std::min(saved.chains, n)
-                                            : (n >= 16 ? std::min(4, n) : 1);
+            const int c0 = default_chains();
             std::vector<std::pair<int, int>> shapes{{h0, c0}};
             for (int d : tryDepth)
             {
@@ -2192,34 +2241,29 @@ struct Engine3D
                     if (d != h0 || c != c0) { shapes.push_back({d, c}); }
                 }
             }
+            const int chunkBefore = tunedChunk, chainsBefore = tunedChains;
             for (const auto &shape : shapes)
             {
-                const int d = shape.first, c = shape.second;
-                opt.chunk_planes = d;
-                opt.chains = c;
-                drop_graph();
-                ekx_status rc = build_schedule();
+                ekx_status rc = use_shape(shape.first, shape.second);
                 float ms = 0;
-                if (rc == EKX_OK) { rc = trial_ms(ms); }
+                if (rc == EKX_OK) { rc = trial_ms(false, ms); }
                 if (rc != EKX_OK)
                 {
-                    opt = saved;
-                    drop_graph();
-                    (void) build_schedule();
+                    (void) use_shape(chunkBefore, chainsBefore);
                     return rc;
                 }
                 if (first || ms < 0.97f*best)
                 {
                     best = ms;
-                    bestDepth = d;
-                    bestChains = c;
+                    bestDepth = shape.first;
+                    bestChains = shape.second;
                     first = false;
                 }
             }
-            opt.chunk_planes = bestDepth;
-            opt.chains = bestChains;
-            drop_graph();
-            EKX_CHECK(build_schedule());
+            EKX_CHECK(use_shape(bestDepth, bestChains));
+            float flowMs = -1;
+            EKX_CHECK(trial_flow(flowMs));
+            if (flowMs > 0 && best < 0.97f*flowMs) { release_flow(); }
         }
         haveField = false;
         chunkOut = chunkH;

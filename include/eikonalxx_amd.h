@@ -194,9 +194,12 @@ typedef struct
                                      layout (device copies in natural
                                      order are made on request)           */
     int32_t chunk_planes;         /* column kernel: z-planes per column
-                                     chunk used (the size-class choice when
-                                     the option is 0)                     */
-    int32_t chains;               /* launch chains used                    */
+                                     chunk (the size-class choice when the
+                                     option is 0) of the launches per
+                                     diagonal; a solve in one launch
+                                     (kernel_launches 1, with polish 2) has
+                                     them ready and uses none             */
+    int32_t chains;               /* their launch chains                   */
     double timed_kernel_ms;       /* summed durations of the timed launches */
     double last_iteration_change; /* early_exit: largest decrease of one
                                      update in the last refinement
@@ -272,10 +275,12 @@ EKX_API ekx_status ekx_solver3d_solve(ekx_solver3d *solver);
 /* No reference counterpart; for callers that solve many times on one
  * setup.  Times short trial solves (the initialisation sweeps and one
  * refinement iteration) for column z-chunk depths around the size-class
- * default and for 1, 2 or 4 launch chains, and keeps the fastest launch
- * shape for later solves.  Fields do not depend on the shape.  Needs the
- * model and the source set; discards the current field.  chunk_planes and
- * chains (each may be NULL) receive the choice. */
+ * default and for 1, 2 or 4 launch chains, and for the solve in one launch
+ * where the options allow it, and keeps the fastest for later solves.
+ * Fields do not depend on the shape.  Needs the model and the source set;
+ * discards the current field.  chunk_planes and chains (each may be NULL)
+ * receive the choice for launches per diagonal, which a solve in one launch
+ * does not use. */
 EKX_API ekx_status ekx_solver3d_autotune(ekx_solver3d *solver,
                                          int *chunk_planes, int *chains);
 /* No reference counterpart.  Longest time (ms) that a wave of a solve in one
