@@ -1536,10 +1536,15 @@ struct Engine3D
         for (size_t i = 0; i < problems.size(); ++i)
         {
             Problem3D &p = problems[i];
-            const double lo = modelSMin[modelOf[i]];
             const double hi = modelSMax[modelOf[i]];
-            p.scaled = p.dx*std::min(lo, hi*0x1p-33) >= 0x1p-300 &&
-                       p.dx*hi <= 0x1p500 ? 1 : 0;
+            const double lo = std::min(modelSMin[modelOf[i]], hi*0x1p-33);
+            // unequal spacings: the planes' determinants are of the size of
+            // (h s)^2 for their larger spacing, the 3D one of (s / h)^2
+            const double least = std::min(p.dx, std::min(p.dy, p.dz));
+            const double most = std::max(p.dx, std::max(p.dy, p.dz));
+            p.scaled = least*lo >= 0x1p-300 && most*hi <= 0x1p500 &&
+                       (p.uniform || (lo >= most*0x1p-340 &&
+                                      hi <= least*0x1p500)) ? 1 : 0;
         }
         return EKX_OK;
     }
