@@ -486,9 +486,12 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         EKX2_HIP(hipMemcpyAsync(h->dProblem.ptr, &p, sizeof(Problem2D),
                                 hipMemcpyHostToDevice, h->stream));
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
-        EKX2_HIP(launch_solve2d(h->dProblem.ptr, 1, h->geometry.nz, h->T.ptr,
-                                h->S.ptr, h->scaled ? h->W.ptr : nullptr,
-                                h->C.ptr, h->stream));
+        EKX2_HIP(launch_solve2d(h->dProblem.ptr, 1, h->geometry.nz,
+                                bands2d(h->geometry.nz),
+                                band_bytes2d(h->geometry.nx, h->geometry.nz),
+                                h->T.ptr, h->S.ptr,
+                                h->scaled ? h->W.ptr : nullptr, h->C.ptr,
+                                h->stream));
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         const int ns = (int) h->stations.size();
         if (ns > 0)
@@ -643,6 +646,7 @@ struct ekx_batch2d
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     int maxNz = 0;
+    int64_t totalBands = 0, recordBytes = 0;
     bool initialized = false, haveField = false;
     ekx_solve_stats stats{};
     ~ekx_batch2d()
@@ -710,6 +714,7 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
         int64_t tTotal = 0, sTotal = 0, wTotal = 0, cTotal = 0;
         bool bands = true;
         h->maxNz = 0;
+        h->totalBands = h->recordBytes = 0;
         for (int i = 0; i < n; ++i)
         {
             const ekx_geometry2d &g = in[i].geometry;
@@ -777,6 +782,8 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
             h->geoms[i] = g;
             h->problems[i] = p;
             h->maxNz = std::max(h->maxNz, g.nz);
+            h->totalBands += bands2d(g.nz);
+            h->recordBytes += band_bytes2d(g.nx, g.nz);
         }
         EKX2_CHECK(h->S.allocate((size_t) sTotal));
         EKX2_CHECK(h->T.allocate((size_t) tTotal));
@@ -821,8 +828,9 @@ ekx_status ekx_batch2d_solve(ekx_batch2d *h)
         EKX2_CHECK(require_batch2d(h));
         const int n = (int) h->problems.size();
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
-        EKX2_HIP(launch_solve2d(h->dProblems.ptr, n, h->maxNz, h->T.ptr,
-                                h->S.ptr, h->W.ptr, h->C.ptr, h->stream));
+        EKX2_HIP(launch_solve2d(h->dProblems.ptr, n, h->maxNz, h->totalBands,
+                                h->recordBytes, h->T.ptr, h->S.ptr, h->W.ptr,
+                                h->C.ptr, h->stream));
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         EKX2_HIP(hipEventSynchronize(h->ev1));
         float ms = 0;

@@ -305,6 +305,12 @@ __host__ __device__ inline int64_t band_values2d(int nx, int nz)
     return 2*(int64_t) bands2d(nz)*band_records2d(nx)*64;
 }
 
+// bytes of it that a solve touches: both buffers, the lanes with a row
+__host__ __device__ inline int64_t band_bytes2d(int nx, int nz)
+{
+    return 2*(int64_t) nz*(nx + 63)*(int64_t) sizeof(double);
+}
+
 // cell records of one band and sweep direction: the steps rounded up to
 // whole groups of 8, and the group that the prefetch runs ahead
 __host__ __device__ inline int cell_steps2d(int nx)

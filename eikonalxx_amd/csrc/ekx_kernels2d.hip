@@ -14,6 +14,7 @@
 #include "ekx_kernels.hpp"
 #include "ekx_sqrt.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace ekx
@@ -395,6 +396,13 @@ struct Band2D
     int t;                  // first step of the next AHEAD
     const GlobalDouble *old, *cells;    // records AHEAD steps ahead
     GlobalDouble *out;
+    // From AHEAD steps to the next.  Lanes whose whole 128 byte line has no
+    // row stay in their first records, which costs nothing and takes their
+    // values out of a traffic that bounds batches (256 problems of 201 x 201,
+    // 55 lanes of the last band without a row: 1.87 ms, 1.76 so; 4096: 29.4
+    // and 28.0; lines written in part are slower than whole ones: 1024
+    // problems of 120 x 60 1.04 ms, 1.13 with their four lanes left out too).
+    uint32_t recordStep, cellStep;
     double cur, s1Prev, t3Prev, hand;
     // in the box's steps: distances from the source of the lane's previous
     // node and of that node's z neighbour
@@ -411,8 +419,8 @@ struct Band2D
             SA[u] = cells[u*kCellRecord2d];
             SB[u] = cells[u*kCellRecord2d + 1];
         }
-        old += AHEAD*kBand2d;
-        cells += AHEAD*kCellRecord2d;
+        old += recordStep;
+        cells += cellStep;
     }
     // the first sweep's old time of the lane's node in column ix
     __device__ __forceinline__ double start_time(int ix) const
@@ -508,9 +516,9 @@ __device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
         else { b.out[-u*kBand2d] = b.cur; }
     }
     b.t += AHEAD;
-    b.old += AHEAD*kBand2d;
-    b.cells += AHEAD*kCellRecord2d;
-    if (!(KIND == kRare && b.last)) { b.out -= AHEAD*kBand2d; }
+    b.old += b.recordStep;
+    b.cells += b.cellStep;
+    if (!(KIND == kRare && b.last)) { b.out -= b.recordStep; }
 }
 
 // One sweep of one band.  old: record of step 0 (this lane's value); cells:
@@ -529,12 +537,17 @@ __device__ __forceinline__ void band_sweep(
     const bool row = iz < nz;
     const bool rowLive = row && jz >= w.jz0;
     const bool anyRow = __builtin_amdgcn_ballot_w64(rowLive) != 0;
+    const int line = kBand2d*band +
+                     (w.negZ ? kBand2d - 1 - (lane | 15) : lane & ~15);
+    const bool stream = line < nz;
     // the constants of the step loop in registers (the barriers' memory
     // clobbers would reload them)
     Band2D<AHEAD> b{source2d(p), w, grid2d(p), lane, iz, nx, row,
                     rowLive ? (uint32_t) (nx - w.jx0) : 0u,
                     rowLive ? -kHuge : 4*kHuge, first, last, 1, 0, 0, old,
-                    cells + lane, out, 0, 0, 0, 0, 0, 0, {}, {}, {}};
+                    cells + lane, out, stream ? AHEAD*kBand2d : 0u,
+                    stream ? AHEAD*kCellRecord2d : 0u, 0, 0, 0, 0, 0, 0, {}, {},
+                    {}};
     // Runs of groups of one kind: [0, idleEnd) idle, [fullLo, fullHi) full,
     // [boxLo, boxEnd) with lanes in the box or on the step before it.
     // (the step before the first live one is not idle: it leaves the box's
@@ -892,10 +905,50 @@ nodal_to_cell2d(int nx, int nz, const double *__restrict__ v, int ordering,
     }
 }
 
+// LDS that a band workgroup asks for beyond its own, to bound how many a CU
+// holds: as many as keep the records of all resident problems in 200 of the
+// Infinity Cache's 256 MB, up to a wave a SIMD or two workgroups.  More only
+// spill: half of the sweeps write lane i's value two records from lane
+// i - 1's, so lines leave L2 partly written (4096 problems of 201 x 201 with
+// two workgroups a CU, 424 MB: 61 GB written for 27 GB of records).  ms with 1,
+// 2, 3, 4 and 8 a CU: 4096 of 201 x 201 (212 MB each) 28.0 31.8 - - -; 4096 of
+// 60 x 200 (98 MB) 13.7 13.1 - - -; of 120 x 128 (94 MB) 12.2 8.5 10.5 11.7 -;
+// of 300 x 60 (87 MB) 17.8 9.6 9.8 10.8 13.3; 8192 of 51 x 41 (19 MB) 13.9 7.5
+// 6.1 6.1 8.8.
+static size_t band_residency_lds(int nProblems, int64_t totalBands,
+                                 int64_t recordBytes, size_t own)
+{
+    constexpr size_t kLdsPerCU = 160*1024;
+    constexpr int64_t kCUs = 256, kResidentBytes = (int64_t) 200 << 20;
+    const int64_t waves = 4*(int64_t) nProblems/std::max<int64_t>(totalBands,
+                                                                  1);
+    const int64_t cached = kResidentBytes*nProblems/
+                           std::max<int64_t>(kCUs*recordBytes, 1);
+    const int64_t groups = std::max<int64_t>(
+        1, std::min(std::max<int64_t>(2, waves), cached));
+    // (a margin of 2 KB for the allocation's granules)
+    const size_t share = kLdsPerCU/(size_t) groups/1024*1024 - 2048;
+    return share > own ? share - own : 0;
+}
+
+template <int WAVES, int AHEAD>
+static void launch_bands2d(const Problem2D *dProblems, int nProblems, int nb,
+                           int64_t totalBands, int64_t recordBytes,
+                           double *T, double *work,
+                           const double *cells, hipStream_t stream)
+{
+    constexpr size_t kOwn =
+        WAVES*(kRing2d + 1 + kBand2d + kGroup2d)*sizeof(double);
+    hipLaunchKernelGGL((solve2d_bands_kernel<WAVES, AHEAD>),
+                       dim3((unsigned) nProblems), dim3(64*nb),
+                       band_residency_lds(nProblems, totalBands, recordBytes,
+                                          kOwn), stream, dProblems, T, work, cells);
+}
+
 hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
-                          int maxNz, double *T, const double *S,
-                          double *work, const double *cells,
-                          hipStream_t stream)
+                          int maxNz, int64_t totalBands, int64_t recordBytes,
+                          double *T, const double *S, double *work,
+                          const double *cells, hipStream_t stream)
 {
     const dim3 grid((unsigned) nProblems);
     const int nb = bands2d(maxNz);
@@ -909,18 +962,18 @@ hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
     // (128).  201 x 41, one band: 266 ns a step with 4 steps, 239 with 8.
     else if (nb <= 8)
     {
-        hipLaunchKernelGGL((solve2d_bands_kernel<8, 8>), grid, dim3(64*nb),
-                           0, stream, dProblems, T, work, cells);
+        launch_bands2d<8, 8>(dProblems, nProblems, nb, totalBands, recordBytes,
+                             T, work, cells, stream);
     }
     else if (nb <= 12)
     {
-        hipLaunchKernelGGL((solve2d_bands_kernel<12, 4>), grid, dim3(64*nb),
-                           0, stream, dProblems, T, work, cells);
+        launch_bands2d<12, 4>(dProblems, nProblems, nb, totalBands,
+                              recordBytes, T, work, cells, stream);
     }
     else
     {
-        hipLaunchKernelGGL((solve2d_bands_kernel<kMaxBands2d, 2>), grid,
-                           dim3(64*nb), 0, stream, dProblems, T, work, cells);
+        launch_bands2d<kMaxBands2d, 2>(dProblems, nProblems, nb, totalBands,
+                                       recordBytes, T, work, cells, stream);
     }
     return hipGetLastError();
 }
