@@ -527,19 +527,19 @@ __device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
 // the field).
 template <bool UNIFORM, int AHEAD>
 __device__ __forceinline__ void band_sweep(
-    const Problem2D &p, const Sweep2D &w, int band, int lane, int groups,
-    bool first, bool last, const GlobalDouble *old, const GlobalDouble *cells,
+    const Problem2D &p, const Sweep2D &w, int band, int height, int lane,
+    int groups, bool first, bool last, const GlobalDouble *old, const GlobalDouble *cells,
     GlobalDouble *out, const double *ringIn, double *ringOut, double *sink)
 {
     const int nx = p.nx, nz = p.nz;
-    const int iz = kBand2d*band + (w.negZ ? kBand2d - 1 - lane : lane);
+    const int iz = kBand2d*band + (w.negZ ? height - 1 - lane : lane);
     const int jz = w.negZ ? nz - 1 - iz : iz;
-    const bool row = iz < nz;
+    const bool row = lane < height && iz < nz;
     const bool rowLive = row && jz >= w.jz0;
     const bool anyRow = __builtin_amdgcn_ballot_w64(rowLive) != 0;
     const int line = kBand2d*band +
-                     (w.negZ ? kBand2d - 1 - (lane | 15) : lane & ~15);
-    const bool stream = line < nz;
+                     (w.negZ ? height - 1 - (lane | 15) : lane & ~15);
+    const bool stream = (lane & ~15) < height && line < nz;
     // the constants of the step loop in registers (the barriers' memory
     // clobbers would reload them)
     Band2D<AHEAD> b{source2d(p), w, grid2d(p), lane, iz, nx, row,
@@ -553,7 +553,7 @@ __device__ __forceinline__ void band_sweep(
     // (the step before the first live one is not idle: it leaves the box's
     // distances)
     const int idleEnd = anyRow ? min((w.jx0 - 1)/kGroup2d, groups) : groups;
-    const int fullLo = (w.jx0 + kBand2d - 2)/kGroup2d + 1;
+    const int fullLo = (w.jx0 + height - 2)/kGroup2d + 1;
     const int fullHi = nx/kGroup2d;
     int boxGroup = groups, boxEnd = groups;
     const int zLo = max(p.srcCellZ - p.radius, 0);
@@ -564,11 +564,11 @@ __device__ __forceinline__ void band_sweep(
         const int xHi = min(p.srcCellX + p.radius, nx - 1);
         // the lanes of the box's rows in this band
         const int iLo = max(zLo - kBand2d*band, 0);
-        const int iHi = min(zHi - kBand2d*band, kBand2d - 1);
+        const int iHi = min(zHi - kBand2d*band, height - 1);
         b.boxLo = (w.negX ? nx - 1 - xHi : xLo) +
-                  (w.negZ ? kBand2d - 1 - iHi : iLo);
+                  (w.negZ ? height - 1 - iHi : iLo);
         b.boxHi = (w.negX ? nx - 1 - xLo : xHi) +
-                  (w.negZ ? kBand2d - 1 - iLo : iHi);
+                  (w.negZ ? height - 1 - iLo : iHi);
         boxGroup = max(b.boxLo - 1, 0)/kGroup2d;
         boxEnd = b.boxHi/kGroup2d + 1;
     }
@@ -653,7 +653,10 @@ solve2d_bands_kernel(const Problem2D *__restrict__ problems,
         p.cOffset + (int64_t) wave*cell_steps2d(nx)*kCellRecord2d;
     double *sink = &sinks[wave][lane];
     const int nSweeps = 4*(1 + p.nSweeps);
-    const int groups = (nx + kBand2d - 1 + kGroup2d - 1)/kGroup2d;
+    // the last lane with rows ends the band's steps: a band alone is as high
+    // as the grid (10 x 10, 12 sweeps: 0.31 ms with all 64 lanes, 0.14)
+    const int height = nb == 1 ? nz : kBand2d;
+    const int groups = (nx + height - 1 + kGroup2d - 1)/kGroup2d;
     int now = 0, base = 0;
     for (int k = 0; k < nSweeps; ++k)
     {
@@ -669,13 +672,15 @@ solve2d_bands_kernel(const Problem2D *__restrict__ problems,
         const GlobalDouble *old = ((k & 1) ? rec[1] : rec[0]) + lane;
         // the result of step t, column jx = t - lane: the next sweep's
         // lane i' of the same row at its step (nx - 1 - jx) + i'
-        const int i = nextNegZ == (bool) w.negZ ? lane : kBand2d - 1 - lane;
+        // (a lane without a row writes a slot of its own)
+        const int i = nextNegZ == (bool) w.negZ || lane >= height
+                          ? lane : height - 1 - lane;
         GlobalDouble *out = ((k & 1) ? rec[0] : rec[1]) +
                             (int64_t) (nx - 1 + lane + i)*kBand2d + i;
         if (last)
         {
             const int izl = kBand2d*wave +
-                            (w.negZ ? kBand2d - 1 - lane : lane);
+                            (w.negZ ? height - 1 - lane : lane);
             out = (GlobalDouble *) T + p.tOffset + (int64_t) izl*nx;
         }
         const int upstream = w.negZ ? min(wave + 1, nb - 1)
@@ -684,13 +689,15 @@ solve2d_bands_kernel(const Problem2D *__restrict__ problems,
             (int64_t) sweep*nb*cell_steps2d(nx)*kCellRecord2d;
         if (p.uniform)
         {
-            band_sweep<true, AHEAD>(p, w, wave, lane, groups, k == 0, last, old, sc,
-                             out, ring[upstream], ring[wave], sink);
+            band_sweep<true, AHEAD>(p, w, wave, height, lane, groups, k == 0,
+                                    last, old, sc, out, ring[upstream],
+                                    ring[wave], sink);
         }
         else
         {
-            band_sweep<false, AHEAD>(p, w, wave, lane, groups, k == 0, last, old,
-                              sc, out, ring[upstream], ring[wave], sink);
+            band_sweep<false, AHEAD>(p, w, wave, height, lane, groups, k == 0,
+                                     last, old, sc, out, ring[upstream],
+                                     ring[wave], sink);
         }
         now += groups;
         // the next sweep reads this one's records, by other lanes of the
@@ -724,8 +731,10 @@ skew_cells2d_kernel(int nx, int nz, const double *__restrict__ s,
         const int band = (int) (rec/steps);
         const int t = (int) (rec - (int64_t) band*steps);
         const bool negX = sweep & 1, negZ = sweep & 2;
-        // permuted row of lane 0 of the band
-        const int jzBase = negZ ? nz - kBand2d*(band + 1) : kBand2d*band;
+        // permuted row of lane 0 of the band (a band alone: as high as the
+        // grid)
+        const int jzBase = nb == 1 ? 0
+                           : negZ ? nz - kBand2d*(band + 1) : kBand2d*band;
         const int pcx = min(max(t - i, 0), ncx - 1);
         const int pcz = min(max(jzBase + i - 1, 0), ncz - 1);
         const int cx = negX ? ncx - 1 - pcx : pcx;

@@ -1,0 +1,54 @@
+"""Grids of few rows: their band ends at its last row, not at 64 lanes.  Against
+the oracle, and no slower for their rows: 12 sweeps of 10 x 10 take less than
+0.6 of those of 10 x 64 (24 steps of 80; with all 64 lanes passed through they
+took as long)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(ekx, nx, nz, dz, src, sweeps, radius, slow):
+    s = ekx.Solver2D()
+    s.initialize(ekx.SolverOptions(number_of_sweeps=sweeps,
+                                   factored_radius=radius),
+                 ekx.Geometry2D(nx, nz, 10.0, dz))
+    s.set_slowness(slow)
+    s.set_source(src)
+    return s
+
+
+@pytest.mark.parametrize("nx,nz", [(3, 4), (4, 3), (7, 8), (8, 15), (16, 16),
+                                   (10, 17), (9, 31), (25, 32), (6, 33),
+                                   (40, 47), (12, 48), (5, 62), (90, 5)])
+@pytest.mark.parametrize("dz", [10.0, 12.5])
+def test_few_rows(ekx, oracle, nx, nz, dz):
+    rng = np.random.default_rng(nx * 131 + nz)
+    slow = 1.0 / rng.uniform(1500.0, 5500.0, (nx - 1) * (nz - 1))
+    ext = ((nx - 1) * 10.0, (nz - 1) * dz)
+    for k, src in enumerate([(0.0, 0.0), ext, (0.0, ext[1]), (ext[0], 0.0),
+                             (0.37 * ext[0], 0.61 * ext[1])]):
+        print("case", nx, nz, dz, k, flush=True)
+        for radius, sweeps in ((3, 1), (-1, 2), (0, 0)):
+            s = _solver(ekx, nx, nz, dz, src, sweeps, radius, slow)
+            ref = oracle.solve2d(oracle.geometry2d(nx, nz, 10.0, dz), slow,
+                                 src, sweeps, radius)
+            for _ in range(2):          # a second solve on the used buffers
+                s.solve()
+                got = s.get_travel_time_field()
+                # hypot's ulp in the box: the 2D solver's bar
+                rel = np.abs(got - ref) / np.maximum(ref, slow.min() * 10.0)
+                assert rel.max() <= 1e-12
+
+
+def test_time_follows_the_rows(ekx):
+    times = {}
+    for nz in (10, 64):
+        s = _solver(ekx, 10, nz, 10.0, (31.0, 42.0), 2, 3,
+                    np.full(9 * (nz - 1), 2e-4))
+        for _ in range(20):
+            s.solve()
+            ms = s.get_stats().last_solve_ms
+            times[nz] = min(times.get(nz, ms), ms)
+    print("tuned", times, flush=True)
+    assert times[10] <= 0.6 * times[64]
