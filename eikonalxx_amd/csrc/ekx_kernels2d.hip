@@ -402,7 +402,14 @@ struct Band2D
     // 55 lanes of the last band without a row: 1.87 ms, 1.76 so; 4096: 29.4
     // and 28.0; lines written in part are slower than whole ones: 1024
     // problems of 120 x 60 1.04 ms, 1.13 with their four lanes left out too).
-    uint32_t recordStep, cellStep;
+    // Not in the instances of more than 8 bands, where one lane in 9 at most
+    // has no row and the two registers are spilled.
+    static constexpr bool kStays = AHEAD == kGroup2d;
+    uint32_t steps[2];
+    __device__ __forceinline__ uint32_t record_step() const
+    { return kStays ? steps[0] : (uint32_t) (AHEAD*kBand2d); }
+    __device__ __forceinline__ uint32_t cell_step() const
+    { return kStays ? steps[1] : (uint32_t) (AHEAD*kCellRecord2d); }
     double cur, s1Prev, t3Prev, hand;
     // in the box's steps: distances from the source of the lane's previous
     // node and of that node's z neighbour
@@ -419,8 +426,8 @@ struct Band2D
             SA[u] = cells[u*kCellRecord2d];
             SB[u] = cells[u*kCellRecord2d + 1];
         }
-        old += recordStep;
-        cells += cellStep;
+        old += record_step();
+        cells += cell_step();
     }
     // the first sweep's old time of the lane's node in column ix
     __device__ __forceinline__ double start_time(int ix) const
@@ -516,9 +523,9 @@ __device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
         else { b.out[-u*kBand2d] = b.cur; }
     }
     b.t += AHEAD;
-    b.old += b.recordStep;
-    b.cells += b.cellStep;
-    if (!(KIND == kRare && b.last)) { b.out -= b.recordStep; }
+    b.old += b.record_step();
+    b.cells += b.cell_step();
+    if (!(KIND == kRare && b.last)) { b.out -= b.record_step(); }
 }
 
 // One sweep of one band.  old: record of step 0 (this lane's value); cells:
@@ -545,8 +552,9 @@ __device__ __forceinline__ void band_sweep(
     Band2D<AHEAD> b{source2d(p), w, grid2d(p), lane, iz, nx, row,
                     rowLive ? (uint32_t) (nx - w.jx0) : 0u,
                     rowLive ? -kHuge : 4*kHuge, first, last, 1, 0, 0, old,
-                    cells + lane, out, stream ? AHEAD*kBand2d : 0u,
-                    stream ? AHEAD*kCellRecord2d : 0u, 0, 0, 0, 0, 0, 0, {}, {},
+                    cells + lane, out,
+                    {stream ? AHEAD*kBand2d : 0u,
+                     stream ? AHEAD*kCellRecord2d : 0u}, 0, 0, 0, 0, 0, 0, {}, {},
                     {}};
     // Runs of groups of one kind: [0, idleEnd) idle, [fullLo, fullHi) full,
     // [boxLo, boxEnd) with lanes in the box or on the step before it.
