@@ -1542,7 +1542,10 @@ struct Engine3D
             // (h s)^2 for their larger spacing, the 3D one of (s / h)^2
             const double least = std::min(p.dx, std::min(p.dy, p.dz));
             const double most = std::max(p.dx, std::max(p.dy, p.dz));
-            p.scaled = least*lo >= 0x1p-300 && most*hi <= 0x1p500 &&
+            // (and no time at the source cell's corners above HUGE, which an
+            // invalid candidate of the branch-free updates would lower)
+            p.scaled = least*lo >= 0x1p-300 &&
+                       (p.dx + p.dy + p.dz)*hi <= kHuge &&
                        (p.uniform || (lo >= most*0x1p-340 &&
                                       hi <= least*0x1p500)) ? 1 : 0;
         }

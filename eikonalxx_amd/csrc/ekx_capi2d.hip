@@ -93,8 +93,8 @@ bool allocate_bands(Buf<double> &work, int64_t workValues,
 }
 
 // Slowness range of a model, and whether the band kernel's unscaled square
-// roots cover it on a grid: h s within [2^-345, 2^500] (2^-700 <= hs0 hs0,
-// and no determinant overflows).
+// roots cover it on a grid: h s at least 2^-345 (2^-700 <= hs0 hs0), and
+// no time at the source cell's corners above HUGE.
 struct Range2D
 {
     double lo = std::numeric_limits<double>::infinity(), hi = 0;
@@ -106,7 +106,7 @@ struct Range2D
     bool scaled(const ekx_geometry2d &g) const
     {
         return std::min(g.dx, g.dz)*lo >= 0x1p-345 &&
-               std::max(g.dx, g.dz)*hi <= 0x1p500;
+               (g.dx + g.dz)*hi <= kHuge;
     }
 };
 

@@ -172,7 +172,8 @@ struct Problem3D
     // slowness bricks.
     int tiled;
     int nTX, nTY;
-    // h s of every cell within [2^-300, 2^500] (cartesian_uniform3d)
+    // h s of every cell at least 2^-300, no time above HUGE
+    // (cartesian_uniform3d, Engine3D::find_ranges)
     int scaled;
     int64_t tCount;
     int64_t eOffset;

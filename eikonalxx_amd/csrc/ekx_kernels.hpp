@@ -172,7 +172,7 @@ hipError_t launch_layered_velocity(int nx, int ny, int nz, int nLayers,
 // The whole 2D solve, one workgroup per problem.  work and cells: the band
 // kernel's buffers (Problem2D::wOffset, cOffset; every grid within
 // fits_bands2d, at most maxNz rows, totalBands bands and recordBytes bytes of
-// records (band_bytes2d) in all, and h s within [2^-345, 2^500]); work null:
+// records (band_bytes2d) in all, and models in range (Range2D)); work null:
 // the level kernel.
 hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
                           int maxNz, int64_t totalBands, int64_t recordBytes,

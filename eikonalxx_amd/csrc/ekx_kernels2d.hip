@@ -60,10 +60,13 @@ __device__ __forceinline__ void analytic_time_deriv2d(
 
 constexpr double kSqrt1_2 = 0.70710678118654752440;
 
-// v where valid, else a number above HUGE (HUGE's next high word): one
-// select instead of two, the low word does not matter.
+// v where valid, else HUGE or (SCALED: no time is above HUGE) a number above
+// it, HUGE's next high word: one select instead of two, the low word does
+// not matter.
+template <bool SCALED>
 __device__ __forceinline__ double valid_or_huge(double v, bool valid)
 {
+    if (!SCALED) { return valid ? v : kHuge; }
     const uint64_t u = __builtin_bit_cast(uint64_t, v);
     const uint32_t hi = valid ? (uint32_t) (u >> 32) : 0x4202A060u;
     return __builtin_bit_cast(double,
@@ -79,7 +82,7 @@ __device__ __forceinline__ double valid_or_huge(double v, bool valid)
 // h s0 / sqrt 2), so their own tests are left out; 2 (hs0 hs0) is exact, so
 // the fused form of detc rounds once like the reference's subtraction.
 //
-// SCALED (the models the band kernel gets): 2^-700 <= hs0 hs0 in every cell, so every valid
+// SCALED (models in range): 2^-700 <= hs0 hs0 in every cell, so every valid
 // determinant is in the range of sqrt_normal_range: deta and detb are at
 // least about half of hs0 hs0, and a positive detc = 2 q - c c is q-sized
 // or, where the terms cancel, a multiple of their last place, 2^-53 q.
@@ -115,9 +118,9 @@ __device__ __forceinline__ double cartesian2d_uniform(
         rb = ::sqrt(cb ? detb : q);
         rc = ::sqrt(cc ? detc : q);
     }
-    best = fmin(best, valid_or_huge(t1 + h*ra, ca));
-    best = fmin(best, valid_or_huge(t3 + h*rb, cb));
-    return fmin(best, valid_or_huge(t2 + rc, cc));
+    best = fmin(best, valid_or_huge<SCALED>(t1 + h*ra, ca));
+    best = fmin(best, valid_or_huge<SCALED>(t3 + h*rb, cb));
+    return fmin(best, valid_or_huge<SCALED>(t2 + rc, cc));
 }
 
 // The spacings and ratios of the Cartesian updates.
@@ -173,12 +176,12 @@ __device__ __forceinline__ double cartesian2d_nonuniform(
         rb = ::sqrt(cb ? detb : 1.0);
         rc = ::sqrt(cc ? detc : 1.0);
     }
-    best = fmin(best, valid_or_huge(t1 + dx_dz*ra, ca));
-    best = fmin(best, valid_or_huge(t3 + dz_dx*rb, cb));
+    best = fmin(best, valid_or_huge<SCALED>(t1 + dx_dz*ra, ca));
+    best = fmin(best, valid_or_huge<SCALED>(t3 + dz_dx*rb, cb));
     double tc = tildeTx*dz_dx + tildeTz*dx_dz + 2*rc;
     tc = (cosTheta*sinTheta)*tc;
     // a negative candidate is dropped (t0Update3 < 0 of the reference)
-    return fmin(best, valid_or_huge(tc, cc && !(tc < 0)));
+    return fmin(best, valid_or_huge<SCALED>(tc, cc && !(tc < 0)));
 }
 
 // A sweep's directions (bit 0: x decreasing, bit 1: z decreasing) and the

@@ -153,7 +153,7 @@ __device__ __forceinline__ bool in_factored_box(const Problem3D &p, int ix,
 // The instruction count bounds the sweeps, so: a pair's two causality tests
 // are one (max <= min + hs: the other holds by itself), and the products by
 // 2 and 1/2, which are exact, are fused into the sum after them (one
-// rounding, the reference's).  SCALED: every hs in [2^-300, 2^500], so a
+// rounding, the reference's).  SCALED: every hs at least 2^-300, so a
 // positive 2D determinant 2 hs hs - c c is hs hs-sized or, where its terms
 // cancel, a multiple of their last place, and its root needs no range test.
 template <typename R, bool SCALED>
