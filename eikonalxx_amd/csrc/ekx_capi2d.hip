@@ -92,9 +92,9 @@ bool allocate_bands(Buf<double> &work, int64_t workValues,
     return false;
 }
 
-// Slowness range of a model, and whether the band kernel's unscaled square
-// roots cover it on a grid: h s at least 2^-345 (2^-700 <= hs0 hs0), and
-// no time at the source cell's corners above HUGE.
+// Slowness range of a model, and whether the band kernel's square roots
+// without range tests cover it on a grid: h s at least 2^-345 (2^-700 <= hs0
+// hs0), and no time at the source cell's corners above HUGE.
 struct Range2D
 {
     double lo = std::numeric_limits<double>::infinity(), hi = 0;
@@ -109,6 +109,13 @@ struct Range2D
                (g.dx + g.dz)*hi <= kHuge;
     }
 };
+
+// (201 x 201, out of range: 2.8 ms by levels in LDS, 3.1 by levels in
+// memory, 1.5 by bands with range tests, 1.2 without)
+int route2d(bool bands, bool scaled)
+{
+    return !bands ? kLevels2d : scaled ? kBands2d : kBandsAnyRange2d;
+}
 
 std::string f2s(double v) { return std::to_string(v); }
 
@@ -483,15 +490,14 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         EKX2_HIP(hipMemcpy(&p.srcSlowness,
                            h->S.ptr + (size_t) p.srcCellZ*ncx + p.srcCellX,
                            sizeof(double), hipMemcpyDeviceToHost));
+        p.route = route2d(h->W.ptr != nullptr, h->scaled);
+        Plan2D plan;
+        plan.add(p);
         EKX2_HIP(hipMemcpyAsync(h->dProblem.ptr, &p, sizeof(Problem2D),
                                 hipMemcpyHostToDevice, h->stream));
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
-        EKX2_HIP(launch_solve2d(h->dProblem.ptr, 1, h->geometry.nz,
-                                bands2d(h->geometry.nz),
-                                band_bytes2d(h->geometry.nx, h->geometry.nz),
-                                h->T.ptr, h->S.ptr,
-                                h->scaled ? h->W.ptr : nullptr, h->C.ptr,
-                                h->stream));
+        EKX2_HIP(launch_solve2d(h->dProblem.ptr, 1, plan, h->T.ptr, h->S.ptr,
+                                h->W.ptr, h->C.ptr, h->stream));
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         const int ns = (int) h->stations.size();
         if (ns > 0)
@@ -645,8 +651,7 @@ struct ekx_batch2d
     Buf<Problem2D> dProblems;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    int maxNz = 0;
-    int64_t totalBands = 0, recordBytes = 0;
+    Plan2D plan;
     bool initialized = false, haveField = false;
     ekx_solve_stats stats{};
     ~ekx_batch2d()
@@ -712,9 +717,7 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
         std::vector<int64_t> modelOffset, cellOffset;
         std::vector<Range2D> ranges;
         int64_t tTotal = 0, sTotal = 0, wTotal = 0, cTotal = 0;
-        bool bands = true;
-        h->maxNz = 0;
-        h->totalBands = h->recordBytes = 0;
+        std::vector<char> scaled(n, 0);
         for (int i = 0; i < n; ++i)
         {
             const ekx_geometry2d &g = in[i].geometry;
@@ -756,7 +759,8 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
                 modelOffset.push_back(sTotal);
                 sTotal += nCell;
                 cellOffset.push_back(cTotal);
-                cTotal += cell_values2d(g.nx, g.nz);
+                cTotal += fits_bands2d(g.nx, g.nz)
+                              ? cell_values2d(g.nx, g.nz) : 0;
             }
             else
             {
@@ -777,19 +781,24 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
             tTotal += (int64_t) g.nx*g.nz;
             p.cOffset = cellOffset[m];
             p.wOffset = wTotal;
-            wTotal += band_values2d(g.nx, g.nz);
-            bands = bands && fits_bands2d(g.nx, g.nz) && ranges[m].scaled(g);
+            wTotal += fits_bands2d(g.nx, g.nz) ? band_values2d(g.nx, g.nz)
+                                               : 0;
+            scaled[i] = ranges[m].scaled(g);
             h->geoms[i] = g;
             h->problems[i] = p;
-            h->maxNz = std::max(h->maxNz, g.nz);
-            h->totalBands += bands2d(g.nz);
-            h->recordBytes += band_bytes2d(g.nx, g.nz);
         }
         EKX2_CHECK(h->S.allocate((size_t) sTotal));
         EKX2_CHECK(h->T.allocate((size_t) tTotal));
         EKX2_CHECK(h->dProblems.allocate((size_t) n));
-        bands = allocate_bands(h->W, bands ? wTotal : 0, h->C,
-                               bands ? cTotal : 0) && bands;
+        const bool bands = allocate_bands(h->W, wTotal, h->C, cTotal);
+        h->plan = Plan2D{};
+        for (int i = 0; i < n; ++i)
+        {
+            Problem2D &p = h->problems[i];
+            p.route = route2d(bands && fits_bands2d(p.nx, p.nz),
+                              scaled[i] != 0);
+            h->plan.add(p);
+        }
         for (size_t m = 0; m < models.size(); ++m)
         {
             ekx_geometry2d g{};
@@ -805,7 +814,7 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
             EKX2_HIP(hipMemcpyAsync(h->S.ptr + modelOffset[m], models[m],
                                     (size_t) nCell*sizeof(double),
                                     hipMemcpyHostToDevice, h->stream));
-            if (bands)
+            if (bands && fits_bands2d(g.nx, g.nz))
             {
                 EKX2_HIP(launch_skew_cells2d(
                     g.nx, g.nz, h->S.ptr + modelOffset[m],
@@ -828,9 +837,8 @@ ekx_status ekx_batch2d_solve(ekx_batch2d *h)
         EKX2_CHECK(require_batch2d(h));
         const int n = (int) h->problems.size();
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
-        EKX2_HIP(launch_solve2d(h->dProblems.ptr, n, h->maxNz, h->totalBands,
-                                h->recordBytes, h->T.ptr, h->S.ptr, h->W.ptr,
-                                h->C.ptr, h->stream));
+        EKX2_HIP(launch_solve2d(h->dProblems.ptr, n, h->plan, h->T.ptr,
+                                h->S.ptr, h->W.ptr, h->C.ptr, h->stream));
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         EKX2_HIP(hipEventSynchronize(h->ev1));
         float ms = 0;
@@ -838,7 +846,7 @@ ekx_status ekx_batch2d_solve(ekx_batch2d *h)
         ekx_solve_stats st{};
         for (const Problem2D &p : h->problems) { st.updates += updates2d(p); }
         st.updates_fp64 = st.updates;
-        st.kernel_launches = 1;
+        st.kernel_launches = h->plan.launches();
         st.iterations_run = h->opt.number_of_sweeps;
         st.last_solve_ms = ms;
         h->stats = st;

@@ -281,7 +281,13 @@ struct Problem2D
     // band kernel: first values of the skewed travel times and cells
     int64_t wOffset;
     int64_t cOffset;
+    int route;                  // Route2D
 };
+
+// How a 2D problem is solved: by the level kernel, or by the band kernel
+// without or with range tests of its square roots (models out of
+// range, Range2D).
+enum Route2D { kLevels2d, kBands2d, kBandsAnyRange2d, kRoutes2d };
 
 // Band kernel of the 2D solve: bands of 64 rows, and per band step records
 // of 64 travel times (two buffers) and of 65 cells (one set per sweep
@@ -323,6 +329,30 @@ __host__ __device__ inline int64_t cell_values2d(int nx, int nz)
 {
     return 4*(int64_t) bands2d(nz)*cell_steps2d(nx)*kCellRecord2d;
 }
+
+// What a launch of the band kernel needs to know of its problems.
+struct Plan2D
+{
+    int problems[kRoutes2d] = {};       // by route
+    // of the problems that the band kernel takes: rows of the tallest, bands
+    // and bytes of records in all
+    int maxNz = 0;
+    int64_t bands = 0, recordBytes = 0;
+    void add(const Problem2D &p)
+    {
+        problems[p.route] += 1;
+        if (p.route == kLevels2d) { return; }
+        maxNz = p.nz > maxNz ? p.nz : maxNz;
+        bands += bands2d(p.nz);
+        recordBytes += band_bytes2d(p.nx, p.nz);
+    }
+    int launches() const
+    {
+        int n = 0;
+        for (int k : problems) { n += k > 0; }
+        return n;
+    }
+};
 
 // Grids that the band kernel takes: at most 16 bands (the waves of a
 // workgroup), and lane offsets that stay well within 32 bits.

@@ -169,15 +169,13 @@ hipError_t launch_layered_velocity(int nx, int ny, int nz, int nLayers,
                                    double mean, double sd, const double *g,
                                    double *v, hipStream_t stream);
 
-// The whole 2D solve, one workgroup per problem.  work and cells: the band
-// kernel's buffers (Problem2D::wOffset, cOffset; every grid within
-// fits_bands2d, at most maxNz rows, totalBands bands and recordBytes bytes of
-// records (band_bytes2d) in all, and models in range (Range2D)); work null:
-// the level kernel.
+// The whole 2D solve, one workgroup per problem, one launch per route that
+// the plan (of these problems) holds.  work and cells: the band kernel's
+// buffers (Problem2D::wOffset, cOffset; grids within fits_bands2d).
 hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
-                          int maxNz, int64_t totalBands, int64_t recordBytes,
-                          double *T, const double *S, double *work,
-                          const double *cells, hipStream_t stream);
+                          const Plan2D &plan, double *T, const double *S,
+                          double *work, const double *cells,
+                          hipStream_t stream);
 // The band kernel's cell records of one model (cell_values2d values).
 hipError_t launch_skew_cells2d(int nx, int nz, const double *s, double *out,
                                hipStream_t stream);

@@ -10,7 +10,7 @@
 //
 // One workgroup owns one problem for the whole solve, so one launch covers
 // it: the band kernel (64 rows per wave) up to 1024 rows, the level kernel
-// (global memory, a block barrier per level) for what it does not take.
+// (global memory, a block barrier per level) for taller and wider grids.
 #include "ekx_kernels.hpp"
 #include "ekx_sqrt.hpp"
 
@@ -82,7 +82,7 @@ __device__ __forceinline__ double valid_or_huge(double v, bool valid)
 // h s0 / sqrt 2), so their own tests are left out; 2 (hs0 hs0) is exact, so
 // the fused form of detc rounds once like the reference's subtraction.
 //
-// SCALED (models in range): 2^-700 <= hs0 hs0 in every cell, so every valid
+// SCALED (models in range, Route2D): 2^-700 <= hs0 hs0 in every cell, so every valid
 // determinant is in the range of sqrt_normal_range: deta and detb are at
 // least about half of hs0 hs0, and a positive detc = 2 q - c c is q-sized
 // or, where the terms cancel, a multiple of their last place, 2^-53 q.
@@ -444,27 +444,27 @@ struct Band2D
         }
         return v;
     }
-    template <bool UNIFORM>
+    template <bool UNIFORM, bool SCALED>
     __device__ __forceinline__ double cartesian(double s0, double s1,
                                                 double s3, double t1,
                                                 double t2, double t3) const
     {
         if constexpr (UNIFORM)
         {
-            return cartesian2d_uniform<true>(grid.dx, s0, s1, s3, t1, t2,
-                                             t3);
+            return cartesian2d_uniform<SCALED>(grid.dx, s0, s1, s3, t1,
+                                               t2, t3);
         }
         else
         {
-            return cartesian2d_nonuniform<true>(grid, s0, s1, s3, t1, t2,
-                                                t3);
+            return cartesian2d_nonuniform<SCALED>(grid, s0, s1, s3, t1,
+                                                  t2, t3);
         }
     }
 };
 
 // AHEAD steps.  ri: the previous band's last row (column t + u + 1 in
 // ri[u]); hp: where lane 63 leaves this band's.
-template <bool UNIFORM, Group2D KIND, int AHEAD>
+template <bool UNIFORM, bool SCALED, Group2D KIND, int AHEAD>
 __device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
                                            double *hp)
 {
@@ -487,7 +487,8 @@ __device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
         if constexpr (KIND == kIdle) { b.cur = t0; }
         else
         {
-            double v = b.template cartesian<UNIFORM>(s0, s1, s3, t1, t2, t3);
+            double v = b.template cartesian<UNIFORM, SCALED>(s0, s1, s3, t1,
+                                                             t2, t3);
             if constexpr (KIND == kFull)
             {
                 b.cur = fmin(fmax(v, b.floor), t0);
@@ -535,7 +536,7 @@ __device__ __forceinline__ void band_steps(Band2D<AHEAD> &b, const double *ri,
 // the sweep's cell records; out: this lane's result of step 0, the next
 // steps' each one record before it (last: the start of the lane's row in
 // the field).
-template <bool UNIFORM, int AHEAD>
+template <bool UNIFORM, bool SCALED, int AHEAD>
 __device__ __forceinline__ void band_sweep(
     const Problem2D &p, const Sweep2D &w, int band, int height, int lane,
     int groups, bool first, bool last, const GlobalDouble *old, const GlobalDouble *cells,
@@ -617,28 +618,28 @@ __device__ __forceinline__ void band_sweep(
         if (first || last || (g >= idleEnd && g >= boxGroup && g < boxEnd))
         {
             run(g, end, [&](const double *ri, double *hp)
-                { band_steps<UNIFORM, kRare>(b, ri, hp); });
+                { band_steps<UNIFORM, SCALED, kRare>(b, ri, hp); });
         }
         else if (g < idleEnd)
         {
             run(g, end, [&](const double *ri, double *hp)
-                { band_steps<UNIFORM, kIdle>(b, ri, hp); });
+                { band_steps<UNIFORM, SCALED, kIdle>(b, ri, hp); });
         }
         else if (g >= fullLo && g < fullHi)
         {
             run(g, end, [&](const double *ri, double *hp)
-                { band_steps<UNIFORM, kFull>(b, ri, hp); });
+                { band_steps<UNIFORM, SCALED, kFull>(b, ri, hp); });
         }
         else
         {
             run(g, end, [&](const double *ri, double *hp)
-                { band_steps<UNIFORM, kAny>(b, ri, hp); });
+                { band_steps<UNIFORM, SCALED, kAny>(b, ri, hp); });
         }
         g = end;
     }
 }
 
-template <int WAVES, int AHEAD>
+template <int WAVES, int AHEAD, bool SCALED>
 __global__ void __launch_bounds__(kBand2d*WAVES)
 solve2d_bands_kernel(const Problem2D *__restrict__ problems,
                      double *__restrict__ T, double *work,
@@ -648,6 +649,7 @@ solve2d_bands_kernel(const Problem2D *__restrict__ problems,
     __shared__ double ring[WAVES][kRing2d + 1];
     __shared__ double sinks[WAVES][kBand2d + kGroup2d];
     const Problem2D &p = problems[blockIdx.x];
+    if (p.route != (SCALED ? kBands2d : kBandsAnyRange2d)) { return; }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     const int nx = p.nx, nz = p.nz;
@@ -700,15 +702,16 @@ solve2d_bands_kernel(const Problem2D *__restrict__ problems,
             (int64_t) sweep*nb*cell_steps2d(nx)*kCellRecord2d;
         if (p.uniform)
         {
-            band_sweep<true, AHEAD>(p, w, wave, height, lane, groups, k == 0,
-                                    last, old, sc, out, ring[upstream],
-                                    ring[wave], sink);
+            band_sweep<true, SCALED, AHEAD>(p, w, wave, height, lane, groups,
+                                            k == 0, last, old, sc, out,
+                                            ring[upstream], ring[wave], sink);
         }
         else
         {
-            band_sweep<false, AHEAD>(p, w, wave, height, lane, groups, k == 0,
-                                     last, old, sc, out, ring[upstream],
-                                     ring[wave], sink);
+            band_sweep<false, SCALED, AHEAD>(p, w, wave, height, lane, groups,
+                                             k == 0, last, old, sc, out,
+                                             ring[upstream], ring[wave],
+                                             sink);
         }
         now += groups;
         // the next sweep reads this one's records, by other lanes of the
@@ -823,6 +826,7 @@ solve2d_kernel(const Problem2D *__restrict__ problems, double *__restrict__ T,
                const double *__restrict__ S)
 {
     const Problem2D &p = problems[blockIdx.x];
+    if (p.route != kLevels2d) { return; }
     double *Tp = T + p.tOffset;
     const double *Sp = S + p.sOffset;
     const int n = p.nx*p.nz;
@@ -935,15 +939,14 @@ nodal_to_cell2d(int nx, int nz, const double *__restrict__ v, int ordering,
 // 60 x 200 (98 MB) 13.7 13.1 - - -; of 120 x 128 (94 MB) 12.2 8.5 10.5 11.7 -;
 // of 300 x 60 (87 MB) 17.8 9.6 9.8 10.8 13.3; 8192 of 51 x 41 (19 MB) 13.9 7.5
 // 6.1 6.1 8.8.
-static size_t band_residency_lds(int nProblems, int64_t totalBands,
-                                 int64_t recordBytes, size_t own)
+static size_t band_residency_lds(const Plan2D &plan, size_t own)
 {
     constexpr size_t kLdsPerCU = 160*1024;
     constexpr int64_t kCUs = 256, kResidentBytes = (int64_t) 200 << 20;
-    const int64_t waves = 4*(int64_t) nProblems/std::max<int64_t>(totalBands,
-                                                                  1);
-    const int64_t cached = kResidentBytes*nProblems/
-                           std::max<int64_t>(kCUs*recordBytes, 1);
+    const int64_t n = plan.problems[kBands2d] +
+                      plan.problems[kBandsAnyRange2d];
+    const int64_t waves = 4*n/plan.bands;
+    const int64_t cached = kResidentBytes*n/(kCUs*plan.recordBytes);
     const int64_t groups = std::max<int64_t>(
         1, std::min(std::max<int64_t>(2, waves), cached));
     // (a margin of 2 KB for the allocation's granules)
@@ -951,49 +954,65 @@ static size_t band_residency_lds(int nProblems, int64_t totalBands,
     return share > own ? share - own : 0;
 }
 
-template <int WAVES, int AHEAD>
-static void launch_bands2d(const Problem2D *dProblems, int nProblems, int nb,
-                           int64_t totalBands, int64_t recordBytes,
-                           double *T, double *work,
+template <int WAVES, int AHEAD, bool SCALED>
+static void launch_bands2d(const Problem2D *dProblems, int nProblems,
+                           const Plan2D &plan, double *T, double *work,
                            const double *cells, hipStream_t stream)
 {
     constexpr size_t kOwn =
         WAVES*(kRing2d + 1 + kBand2d + kGroup2d)*sizeof(double);
-    hipLaunchKernelGGL((solve2d_bands_kernel<WAVES, AHEAD>),
-                       dim3((unsigned) nProblems), dim3(64*nb),
-                       band_residency_lds(nProblems, totalBands, recordBytes,
-                                          kOwn), stream, dProblems, T, work, cells);
+    hipLaunchKernelGGL((solve2d_bands_kernel<WAVES, AHEAD, SCALED>),
+                       dim3((unsigned) nProblems),
+                       dim3(kBand2d*bands2d(plan.maxNz)),
+                       band_residency_lds(plan, kOwn), stream, dProblems, T,
+                       work, cells);
 }
 
-hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
-                          int maxNz, int64_t totalBands, int64_t recordBytes,
-                          double *T, const double *S, double *work,
-                          const double *cells, hipStream_t stream)
+// Registers per wave set the read-ahead: 8 steps (223 registers) while
+// at most 2 waves share a SIMD, 4 steps (168) for 3 waves, 2 for 4 waves
+// (128).  201 x 41, one band: 266 ns a step with 4 steps, 239 with 8.
+template <bool SCALED>
+static void launch_bands2d(const Problem2D *dProblems, int nProblems,
+                           const Plan2D &plan, double *T, double *work,
+                           const double *cells, hipStream_t stream)
 {
-    const dim3 grid((unsigned) nProblems);
-    const int nb = bands2d(maxNz);
-    if (work == nullptr)
+    const int nb = bands2d(plan.maxNz);
+    if (nb <= 8)
     {
-        hipLaunchKernelGGL(solve2d_kernel, grid, dim3(256), 0, stream,
-                           dProblems, T, S);
-    }
-    // Registers per wave set the read-ahead: 8 steps (223 registers) while
-    // at most 2 waves share a SIMD, 4 steps (168) for 3 waves, 2 for 4 waves
-    // (128).  201 x 41, one band: 266 ns a step with 4 steps, 239 with 8.
-    else if (nb <= 8)
-    {
-        launch_bands2d<8, 8>(dProblems, nProblems, nb, totalBands, recordBytes,
-                             T, work, cells, stream);
+        launch_bands2d<8, 8, SCALED>(dProblems, nProblems, plan, T, work,
+                                     cells, stream);
     }
     else if (nb <= 12)
     {
-        launch_bands2d<12, 4>(dProblems, nProblems, nb, totalBands,
-                              recordBytes, T, work, cells, stream);
+        launch_bands2d<12, 4, SCALED>(dProblems, nProblems, plan, T, work,
+                                      cells, stream);
     }
     else
     {
-        launch_bands2d<kMaxBands2d, 2>(dProblems, nProblems, nb, totalBands,
-                                       recordBytes, T, work, cells, stream);
+        launch_bands2d<kMaxBands2d, 2, SCALED>(dProblems, nProblems, plan, T,
+                                               work, cells, stream);
+    }
+}
+
+hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
+                          const Plan2D &plan, double *T, const double *S,
+                          double *work, const double *cells,
+                          hipStream_t stream)
+{
+    if (plan.problems[kLevels2d] > 0)
+    {
+        hipLaunchKernelGGL(solve2d_kernel, dim3((unsigned) nProblems),
+                           dim3(256), 0, stream, dProblems, T, S);
+    }
+    if (plan.problems[kBands2d] > 0)
+    {
+        launch_bands2d<true>(dProblems, nProblems, plan, T, work, cells,
+                             stream);
+    }
+    if (plan.problems[kBandsAnyRange2d] > 0)
+    {
+        launch_bands2d<false>(dProblems, nProblems, plan, T, work, cells,
+                              stream);
     }
     return hipGetLastError();
 }
