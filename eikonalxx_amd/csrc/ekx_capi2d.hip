@@ -645,13 +645,20 @@ struct ekx_batch2d
     std::vector<ekx_geometry2d> geoms;
     std::vector<Problem2D> problems;
     Buf<double> S, T;
-    // band kernel: skewed travel times per problem and cells per model
-    // (empty: level kernel)
+    // band kernel: skewed travel times per problem of a slice and cells per
+    // model (empty: level kernel)
     Buf<double> W, C;
     Buf<Problem2D> dProblems;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    Plan2D plan;
+    // problems solved by one launch, which the slices after it share the
+    // band kernel's travel times with
+    struct Slice
+    {
+        int first = 0, problems = 0;
+        Plan2D plan;
+    };
+    std::vector<Slice> slices;
     bool initialized = false, haveField = false;
     ekx_solve_stats stats{};
     ~ekx_batch2d()
@@ -661,6 +668,48 @@ struct ekx_batch2d
         if (stream) { (void) hipStreamDestroy(stream); }
     }
 };
+
+// Cuts a batch into slices whose skewed travel times fit `values`, of about
+// the same size each, and sets the problems' first values in their slice;
+// returns the values that the largest needs (0: some problem does not fit).
+static int64_t cut_slices(ekx_batch2d &b, int64_t values)
+{
+    int64_t total = 0, most = 0;
+    auto need = [](const Problem2D &p)
+    {
+        return fits_bands2d(p.nx, p.nz) ? band_values2d(p.nx, p.nz) : 0;
+    };
+    for (const Problem2D &p : b.problems)
+    {
+        total += need(p);
+        most = std::max(most, need(p));
+    }
+    if (most > values) { return 0; }
+    // a slice begins with the first problem past its share of the total, or
+    // with the one that does not fit into the slice before
+    const int64_t slices = std::max<int64_t>(1, (total + values - 1)/values);
+    int64_t start = 0, used = 0, largest = 0, slice = 0;
+    b.slices.assign(1, ekx_batch2d::Slice{});
+    for (int i = 0; i < (int) b.problems.size(); ++i)
+    {
+        Problem2D &p = b.problems[i];
+        const int64_t at = total > 0 ? start*slices/total : 0;
+        const bool full = used + need(p) > values;
+        if ((at > slice || full) && b.slices.back().problems > 0)
+        {
+            b.slices.push_back(ekx_batch2d::Slice{});
+            b.slices.back().first = i;
+            used = 0;
+        }
+        slice = std::max(slice, full ? at + 1 : at);
+        p.wOffset = used;
+        used += need(p);
+        start += need(p);
+        b.slices.back().problems += 1;
+        largest = std::max(largest, used);
+    }
+    return largest;
+}
 
 static ekx_status require_batch2d(const ekx_batch2d *h)
 {
@@ -716,7 +765,7 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
         std::vector<const double *> models;
         std::vector<int64_t> modelOffset, cellOffset;
         std::vector<Range2D> ranges;
-        int64_t tTotal = 0, sTotal = 0, wTotal = 0, cTotal = 0;
+        int64_t tTotal = 0, sTotal = 0, cTotal = 0;
         std::vector<char> scaled(n, 0);
         for (int i = 0; i < n; ++i)
         {
@@ -780,9 +829,6 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
             p.tOffset = tTotal;
             tTotal += (int64_t) g.nx*g.nz;
             p.cOffset = cellOffset[m];
-            p.wOffset = wTotal;
-            wTotal += fits_bands2d(g.nx, g.nz) ? band_values2d(g.nx, g.nz)
-                                               : 0;
             scaled[i] = ranges[m].scaled(g);
             h->geoms[i] = g;
             h->problems[i] = p;
@@ -790,14 +836,27 @@ ekx_status ekx_batch2d_initialize(ekx_batch2d *h,
         EKX2_CHECK(h->S.allocate((size_t) sTotal));
         EKX2_CHECK(h->T.allocate((size_t) tTotal));
         EKX2_CHECK(h->dProblems.allocate((size_t) n));
-        const bool bands = allocate_bands(h->W, wTotal, h->C, cTotal);
-        h->plan = Plan2D{};
-        for (int i = 0; i < n; ++i)
+        // The skewed times, five fields a problem, are kept for as many
+        // problems as 4 GiB hold (2571 of 201 x 201, ten rounds of the
+        // device), or fewer where
+        // the device has less.
+        bool bands = false;
+        for (int64_t values = (int64_t) 1 << 29; !bands; values /= 2)
         {
-            Problem2D &p = h->problems[i];
-            p.route = route2d(bands && fits_bands2d(p.nx, p.nz),
-                              scaled[i] != 0);
-            h->plan.add(p);
+            const int64_t largest = cut_slices(*h, values);
+            if (largest == 0) { break; }
+            bands = allocate_bands(h->W, largest, h->C, cTotal);
+        }
+        if (!bands) { h->slices.assign(1, {0, n, Plan2D{}}); }
+        for (ekx_batch2d::Slice &slice : h->slices)
+        {
+            for (int i = slice.first; i < slice.first + slice.problems; ++i)
+            {
+                Problem2D &p = h->problems[i];
+                p.route = route2d(bands && fits_bands2d(p.nx, p.nz),
+                                  scaled[i] != 0);
+                slice.plan.add(p);
+            }
         }
         for (size_t m = 0; m < models.size(); ++m)
         {
@@ -835,18 +894,21 @@ ekx_status ekx_batch2d_solve(ekx_batch2d *h)
     return guarded([&]() -> ekx_status
     {
         EKX2_CHECK(require_batch2d(h));
-        const int n = (int) h->problems.size();
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
-        EKX2_HIP(launch_solve2d(h->dProblems.ptr, n, h->plan, h->T.ptr,
-                                h->S.ptr, h->W.ptr, h->C.ptr, h->stream));
+        ekx_solve_stats st{};
+        for (const ekx_batch2d::Slice &s : h->slices)
+        {
+            EKX2_HIP(launch_solve2d(h->dProblems.ptr + s.first, s.problems,
+                                    s.plan, h->T.ptr, h->S.ptr, h->W.ptr,
+                                    h->C.ptr, h->stream));
+            st.kernel_launches += s.plan.launches();
+        }
         EKX2_HIP(hipEventRecord(h->ev1, h->stream));
         EKX2_HIP(hipEventSynchronize(h->ev1));
         float ms = 0;
         EKX2_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
-        ekx_solve_stats st{};
         for (const Problem2D &p : h->problems) { st.updates += updates2d(p); }
         st.updates_fp64 = st.updates;
-        st.kernel_launches = h->plan.launches();
         st.iterations_run = h->opt.number_of_sweeps;
         st.last_solve_ms = ms;
         h->stats = st;
