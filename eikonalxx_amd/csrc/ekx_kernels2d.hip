@@ -731,30 +731,22 @@ __global__ void __launch_bounds__(256)
 skew_cells2d_kernel(int nx, int nz, const double *__restrict__ s,
                     double *__restrict__ out)
 {
+    // grid (x): the values of a band's steps; (y): bands of the four sweeps
     const int ncx = nx - 1, ncz = nz - 1;
-    const int nb = bands2d(nz), steps = cell_steps2d(nx);
-    const int64_t perSweep = (int64_t) nb*steps*kCellRecord2d;
-    const int64_t n = 4*perSweep;
-    for (int64_t e = (int64_t) blockIdx.x*blockDim.x + threadIdx.x; e < n;
-         e += (int64_t) gridDim.x*blockDim.x)
-    {
-        const int sweep = (int) (e/perSweep);
-        const int64_t r = e - sweep*perSweep;
-        const int64_t rec = r/kCellRecord2d;
-        const int i = (int) (r - rec*kCellRecord2d);
-        const int band = (int) (rec/steps);
-        const int t = (int) (rec - (int64_t) band*steps);
-        const bool negX = sweep & 1, negZ = sweep & 2;
-        // permuted row of lane 0 of the band (a band alone: as high as the
-        // grid)
-        const int jzBase = nb == 1 ? 0
-                           : negZ ? nz - kBand2d*(band + 1) : kBand2d*band;
-        const int pcx = min(max(t - i, 0), ncx - 1);
-        const int pcz = min(max(jzBase + i - 1, 0), ncz - 1);
-        const int cx = negX ? ncx - 1 - pcx : pcx;
-        const int cz = negZ ? ncz - 1 - pcz : pcz;
-        out[e] = s[(int64_t) cz*ncx + cx];
-    }
+    const int nb = bands2d(nz), values = cell_steps2d(nx)*kCellRecord2d;
+    const int e = blockIdx.x*blockDim.x + threadIdx.x;
+    if (e >= values) { return; }
+    const int sweep = (int) blockIdx.y/nb, band = (int) blockIdx.y - sweep*nb;
+    const int t = e/kCellRecord2d, i = e - t*kCellRecord2d;
+    const bool negX = sweep & 1, negZ = sweep & 2;
+    // permuted row of lane 0 of the band (a band alone: as high as the grid)
+    const int jzBase = nb == 1 ? 0
+                       : negZ ? nz - kBand2d*(band + 1) : kBand2d*band;
+    const int pcx = min(max(t - i, 0), ncx - 1);
+    const int pcz = min(max(jzBase + i - 1, 0), ncz - 1);
+    const int cx = negX ? ncx - 1 - pcx : pcx;
+    const int cz = negZ ? ncz - 1 - pcz : pcz;
+    out[(int64_t) blockIdx.y*values + e] = s[(int64_t) cz*ncx + cx];
 }
 
 // ---------------------------------------------------------------------------
@@ -1020,11 +1012,11 @@ hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
 hipError_t launch_skew_cells2d(int nx, int nz, const double *s, double *out,
                                hipStream_t stream)
 {
-    const int64_t n = cell_values2d(nx, nz);
-    const int64_t g = (n + 255)/256;
+    const int values = cell_steps2d(nx)*kCellRecord2d;
     hipLaunchKernelGGL(skew_cells2d_kernel,
-                       dim3((unsigned) (g < 4096 ? g : 4096)), dim3(256), 0,
-                       stream, nx, nz, s, out);
+                       dim3((unsigned) ((values + 255)/256),
+                            (unsigned) (4*bands2d(nz))),
+                       dim3(256), 0, stream, nx, nz, s, out);
     return hipGetLastError();
 }
 
