@@ -1406,7 +1406,8 @@ struct Engine3D
         EKX_CHECK(copy_out(&err, w, sizeof(err)));
         if (err != 0)
         {
-            EKX_HIP(hipMemset(w, 0, sizeof(err)));
+            EKX_HIP(launch_clear_words(w, 1, stream));
+            EKX_HIP(hipStreamSynchronize(stream));
             return fail(EKX_EHIP, "column work queue: a dependency wait "
                                   "exceeded its bound");
         }
@@ -2937,11 +2938,13 @@ ekx_status ekx_model3d_layered_gaussian(const ekx_geometry3d *geometry,
         if (rc == EKX_OK) { rc = generate_layered_gaussian(g, *model, dv.ptr, s); }
         if (rc == EKX_OK)
         {
-            hipError_t e = hipMemcpy(velocity, dv.ptr, (size_t) n*sizeof(double),
-                                     hipMemcpyDeviceToHost);
+            hipError_t e = hipMemcpyAsync(velocity, dv.ptr,
+                                          (size_t) n*sizeof(double),
+                                          hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) { e = hipStreamSynchronize(s); }
             if (e != hipSuccess)
             {
-                rc = fail(EKX_EHIP, std::string("hipMemcpy: ") +
+                rc = fail(EKX_EHIP, std::string("hipMemcpyAsync: ") +
                                         hipGetErrorString(e));
             }
         }

@@ -146,6 +146,16 @@ struct Range2D
     }
 };
 
+// A copy between host and device on the handle's own stream, and its end: on
+// the default stream it fails while another thread's solver captures.
+ekx_status copy2d(void *dst, const void *src, size_t bytes,
+                  hipStream_t stream)
+{
+    EKX2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, stream));
+    EKX2_HIP(hipStreamSynchronize(stream));
+    return EKX_OK;
+}
+
 // (201 x 201, out of range: 2.8 ms by levels in LDS, 3.1 by levels in
 // memory, 1.5 by bands with range tests, 1.2 without)
 int route2d(bool bands, bool scaled)
@@ -486,14 +496,14 @@ ekx_status ekx_solver2d_set_stations(ekx_solver2d *h, int n, const double *x,
         EKX2_CHECK(h->stationOut.allocate(m));
         if (n > 0)
         {
-            EKX2_HIP(hipMemcpy(h->stationX.ptr, xo.data(), n*sizeof(double),
-                               hipMemcpyHostToDevice));
-            EKX2_HIP(hipMemcpy(h->stationZ.ptr, zo.data(), n*sizeof(double),
-                               hipMemcpyHostToDevice));
-            EKX2_HIP(hipMemcpy(h->stationCX.ptr, cx.data(), n*sizeof(int),
-                               hipMemcpyHostToDevice));
-            EKX2_HIP(hipMemcpy(h->stationCZ.ptr, cz.data(), n*sizeof(int),
-                               hipMemcpyHostToDevice));
+            EKX2_CHECK(copy2d(h->stationX.ptr, xo.data(), n*sizeof(double),
+                              h->stream));
+            EKX2_CHECK(copy2d(h->stationZ.ptr, zo.data(), n*sizeof(double),
+                              h->stream));
+            EKX2_CHECK(copy2d(h->stationCX.ptr, cx.data(), n*sizeof(int),
+                              h->stream));
+            EKX2_CHECK(copy2d(h->stationCZ.ptr, cz.data(), n*sizeof(int),
+                              h->stream));
         }
         return EKX_OK;
     });
@@ -519,9 +529,9 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         p.srcOffX = h->source.off[0];
         p.srcOffZ = h->source.off[1];
         const int ncx = h->geometry.nx - 1;
-        EKX2_HIP(hipMemcpy(&p.srcSlowness,
-                           h->S.ptr + (size_t) p.srcCellZ*ncx + p.srcCellX,
-                           sizeof(double), hipMemcpyDeviceToHost));
+        EKX2_CHECK(copy2d(&p.srcSlowness,
+                          h->S.ptr + (size_t) p.srcCellZ*ncx + p.srcCellX,
+                          sizeof(double), h->stream));
         p.route = route2d(h->bands.work != nullptr, h->scaled);
         Plan2D plan;
         plan.add(p);
@@ -544,8 +554,8 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         h->stationTimes.assign((size_t) ns, 0.0);
         if (ns > 0)
         {
-            EKX2_HIP(hipMemcpy(h->stationTimes.data(), h->stationOut.ptr,
-                               ns*sizeof(double), hipMemcpyDeviceToHost));
+            EKX2_CHECK(copy2d(h->stationTimes.data(), h->stationOut.ptr,
+                              ns*sizeof(double), h->stream));
         }
         float ms = 0;
         EKX2_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
@@ -574,8 +584,8 @@ ekx_status ekx_solver2d_get_travel_times(const ekx_solver2d *h, int64_t n,
             return fail2(EKX_EINVAL, "output must hold the " +
                                          std::to_string(nGrid) + " grid points");
         }
-        EKX2_HIP(hipMemcpy(out, h->T.ptr, (size_t) n*sizeof(double),
-                           hipMemcpyDeviceToHost));
+        EKX2_CHECK(copy2d(out, h->T.ptr, (size_t) n*sizeof(double),
+                          h->stream));
         return EKX_OK;
     });
 }
@@ -648,8 +658,8 @@ ekx_status ekx_solver2d_get_travel_time_gradient_field(const ekx_solver2d *h,
             return fail2(EKX_EINVAL, "output must hold 2 x " +
                                          std::to_string(want/2) + " values");
         }
-        EKX2_HIP(hipMemcpy(out, h->G.ptr, (size_t) n*sizeof(double),
-                           hipMemcpyDeviceToHost));
+        EKX2_CHECK(copy2d(out, h->G.ptr, (size_t) n*sizeof(double),
+                          h->stream));
         return EKX_OK;
     });
 }
@@ -968,8 +978,8 @@ ekx_status ekx_batch2d_get_travel_times(const ekx_batch2d *h, int problem,
             return fail2(EKX_EINVAL, "output must hold the " +
                                          std::to_string(nGrid) + " grid points");
         }
-        EKX2_HIP(hipMemcpy(out, h->T.ptr + p.tOffset, (size_t) n*sizeof(double),
-                           hipMemcpyDeviceToHost));
+        EKX2_CHECK(copy2d(out, h->T.ptr + p.tOffset, (size_t) n*sizeof(double),
+                          h->stream));
         return EKX_OK;
     });
 }
