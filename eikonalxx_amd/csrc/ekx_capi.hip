@@ -4,6 +4,7 @@
 #include "eikonalxx_amd.h"
 #include "ekx_guard.hpp"
 #include "ekx_kernels.hpp"
+#include "ekx_reservation.hpp"
 #include "ekx_storage.hpp"
 
 #include <algorithm>
@@ -457,37 +458,8 @@ ekx_status scratch_address(Problem3D **out)
 
 namespace
 {
-// Waves of flow launches in progress per device.  A flow launch needs all
-// its waves resident together, so it takes place only if they fit beside
-// those of the other flow launches of the process (other threads' solvers);
-// otherwise the solve uses the launches per diagonal.
+// Waves of flow launches in progress per device (FlowReservation).
 std::atomic<int> g_flowWaves[kMaxDevices];
-
-struct FlowReservation
-{
-    int device = -1, waves = 0;
-    FlowReservation() = default;
-    FlowReservation(const FlowReservation &) = delete;
-    FlowReservation &operator=(const FlowReservation &) = delete;
-    ~FlowReservation() { release(); }
-    void release()
-    {
-        if (waves > 0) { g_flowWaves[device].fetch_sub(waves); }
-        waves = 0;
-    }
-    bool take(int dev, int n, int capacity)
-    {
-        if (dev < 0 || dev >= kMaxDevices) { return false; }
-        device = dev;
-        if (g_flowWaves[dev].fetch_add(n) + n > capacity)
-        {
-            g_flowWaves[dev].fetch_sub(n);
-            return false;
-        }
-        waves = n;
-        return true;
-    }
-};
 } // namespace
 
 // ===========================================================================
@@ -1087,8 +1059,10 @@ struct Engine3D
             if (!p.scaled) { return false; }
         }
         int device = 0;
-        return hipGetDevice(&device) == hipSuccess &&
-               r.take(device, std::min((int) flowColumns.size(), flowCapacity),
+        return hipGetDevice(&device) == hipSuccess && device >= 0 &&
+               device < kMaxDevices &&
+               r.take(g_flowWaves[device],
+                      std::min((int) flowColumns.size(), flowCapacity),
                       flowCapacity);
     }
 
