@@ -1418,18 +1418,36 @@ struct Engine3D
     }
 
     // Planes per z-chunk when the caller leaves the choice
-    // (chunk_planes = 0), by size class: the longest of whole
-    // columns, 128, 96, 64, 48, 32, 24, 16, 12 or 8 planes whose column
-    // diagonals hold on average at least 1.5 times (above 96 planes, 3 times)
-    // the column waves the device keeps resident of the bulk instance that
-    // also runs the box chunks.
+    // (chunk_planes = 0), by size class: the longest of whole columns, 128,
+    // 96, 64, 48, 32, 24, 16, 12 or 8 planes whose column diagonals hold on
+    // average at least a number of times the column waves the device keeps
+    // resident of the bulk instance that also runs the box chunks: 1.5 up to
+    // 96 planes, 3 up to 128, above that 2.5 in FP64, 4 in FP32 and 3.5 in
+    // scaled integers, whose steps are shorter against a launch's ends.
     // Shorter chunks put more column-chunks on each diagonal (a sweep's
     // dependency chain is nbx + nby + nbz - 2 launches) at the price of
     // the 15-step lane skew at both ends of every chunk.  Measured on the
-    // MI355X: the 256-source 385 x 385 x 193 tables run fastest with whole
-    // columns (FP64, 4 iterations: 1570 ms, chunks of 97 planes 1613), 128
-    // sources with 97 planes (1 iteration: 297 and 263 ms), a 64-problem
-    // batch of 96..320-point grids with 32 planes, a single 257 x 257 x 193 or 129^3 grid with 8 (4.5x and 3x faster than
+    // MI355X, 3 iterations, ms of whole columns / chunks of half their planes
+    // (/ of a third), with the ratio of whole columns (processes differ by up
+    // to 4%, the shapes within one by less than 1%):
+    // 385 x 385 x 193   FP64          FP32          scaled integers
+    //   128 (1.5)       727 664 677   468 395 387   780 642 633
+    //   192 (2.3)       954 946       568 537       929 887
+    //   224 (2.7)       1068 1084
+    //   256 (3.1)       1200 1217     685 678       1167 1143
+    //   320 (3.9)       1464 1520                   1370 1401
+    //   384 (4.6)       1739 1804     956 926       1622 1669
+    //     (again)                     915 952
+    //   512 (6.2)                     1168 1239
+    // 257 x 257 x 257
+    //   300 (2.5)       860 861       530 478       853 798
+    //   600 (4.9)                     845 833       1477 1495
+    // 201 x 201 x 120 (whole: 128 or less)
+    //   500 (3.2)       451 490       267 342       435 514
+    // 193 x 193 x 110
+    //   300 (1.9)       278 268       197 194       302 280
+    // A 64-problem batch of 96..320-point grids runs fastest with 32 planes,
+    // a single 257 x 257 x 193 or 129^3 grid with 8 (4.5x and 3x faster than
     // whole columns); every choice gives the same field.
     int auto_chunk(const std::vector<ekx_geometry3d> &geoms, int maxNz) const
     {
@@ -1450,7 +1468,8 @@ struct Engine3D
                         ? column_waves_per_cu<uint32_t>(depth(), true)
                         : column_waves_per_cu<float>(depth(), true);
         if (perCU <= 0) { perCU = 8; }
-        const double want = 1.5*cus*perCU;
+        const double resident = (double) cus*perCU;
+        const double deep = sweeps_f64() ? 2.5 : fixed32() ? 3.5 : 4.0;
         for (int c : kChunkCandidates)
         {
             const int h = c == 0 ? maxNz : std::min(c, maxNz);
@@ -1463,9 +1482,8 @@ struct Engine3D
                 items += (double) nbx*nby*nbz;
                 diags = std::max(diags, nbx + nby + nbz - 2);
             }
-            // (64 sources on 385 x 385 x 193: chunks of 97 planes 171 ms, 65
-            // 164; 128 sources: whole columns 297 ms, 97 planes 263)
-            if (items/diags >= (h > 96 ? 2*want : want)) { return h; }
+            const double want = h > 128 ? deep : h > 96 ? 3.0 : 1.5;
+            if (items/diags >= want*resident) { return h; }
         }
         return std::min(8, maxNz);
     }
