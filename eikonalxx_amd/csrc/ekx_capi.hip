@@ -830,7 +830,7 @@ struct Engine3D
     // FP64 and FP32 fields (mail keeps its tag in the sign bit, which the
     // scaled integers use), for problems that each fit the device's resident
     // waves.  There the sweeps are a chain of dependent steps, which a launch
-    // per diagonal lengthens: 257 x 257 x 193 FP64 46.5 ms by diagonals, 14.9
+    // per diagonal lengthens: 257 x 257 x 193 FP64 50.9 ms by diagonals, 14.3
     // ms in one launch.
     // With more columns than waves the problems follow each other through
     // the device, the longest chains first: a column waits only for columns

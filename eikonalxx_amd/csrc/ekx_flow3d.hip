@@ -55,15 +55,20 @@ namespace ekx
 // instruction count: branch-free updates, and group kinds for what a group
 // of 4 steps can meet.
 //
-// One 257 x 257 x 193 grid, FP64, 3 iterations: 46.5 ms with one launch per
-// diagonal of 8-plane chunks (89 a sweep), 14.9 ms here.  A step takes 0.46
+// One 257 x 257 x 193 grid, FP64, 3 iterations: 50.9 ms with one launch per
+// diagonal of 8-plane chunks (89 a sweep), 14.3 ms here.  A step takes 0.46
 // us alone (170 instructions of 5 cycles, and the wait for LDS), more where
 // waves share a CU (4: 0.52 us) or a SIMD (the younger one 0.7 us).
 //
-// Every wave must be resident at once: the host launches it only for as
-// many columns as the device holds and reserves them; each wait is bounded
-// in wall-clock time all the same, and past the bound flags an error, after
-// which no wave waits any more and the host solves with the diagonals.
+// A column waits for columns of its own problem only, so every column of a
+// problem must become resident: the host launches it only for problems that
+// each fit the device, and reserves their waves.  Problems beyond the resident
+// waves follow the earlier ones: the columns of each XCD are in problem order,
+// and its workgroups start in that order, so the first unfinished problem is
+// resident as a whole.  Where that does not hold (a device shared with other
+// work), each wait is bounded in wall-clock time, and past the bound flags an
+// error, after which no wave waits any more and the host solves with the
+// diagonals.
 // ---------------------------------------------------------------------------
 constexpr int kFlowAhead = 4;       // steps that records are loaded ahead
 // Steps that mail is loaded ahead: each one more is one step more a hop

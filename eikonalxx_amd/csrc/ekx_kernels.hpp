@@ -74,9 +74,11 @@ hipError_t launch_queued_columns3d(const Problem3D *dProblems,
 // nSweeps sweeps, the first nInit of them initialisation sweeps, from
 // rec (step records of sweep 0 in the first of two buffers of recCount
 // elements) to the buffer nSweeps & 1, in the order of sweep nSweeps & 7.
-// mail: kMailBuffers buffers of mailCount elements, zero before the launch.  Every
-// model's h s must be in range (Problem3D::scaled), every grid uniform or
-// every one not, and all nColumns waves resident together; error is set when a wait exceeded waitTicks.
+// mail: kMailBuffers buffers of mailCount elements, zero before the launch.
+// Every model must be in range (Problem3D::scaled), every grid uniform or
+// every one not, every problem's columns no more than the resident waves, and
+// the columns of each XCD (blocks of one index modulo 8) in the same order of
+// problems; error is set when a wait exceeded waitTicks.
 template <typename TS> int flow_waves_per_cu(bool uniform);
 template <typename TS>
 hipError_t launch_flow_init(const Problem3D *dProblems,
