@@ -921,28 +921,48 @@ nodal_to_cell2d(int nx, int nz, const double *__restrict__ v, int ordering,
     }
 }
 
-// LDS that a band workgroup asks for beyond its own, to bound how many a CU
-// holds: as many as keep the records of all resident problems in 200 of the
-// Infinity Cache's 256 MB, up to a wave a SIMD or two workgroups.  More only
-// spill: half of the sweeps write lane i's value two records from lane
-// i - 1's, so lines leave L2 partly written (4096 problems of 201 x 201 with
-// two workgroups a CU, 424 MB: 61 GB written for 27 GB of records).  ms with 1,
-// 2, 3, 4 and 8 a CU: 4096 of 201 x 201 (212 MB each) 28.0 31.8 - - -; 4096 of
-// 60 x 200 (98 MB) 13.7 13.1 - - -; of 120 x 128 (94 MB) 12.2 8.5 10.5 11.7 -;
-// of 300 x 60 (87 MB) 17.8 9.6 9.8 10.8 13.3; 8192 of 51 x 41 (19 MB) 13.9 7.5
-// 6.1 6.1 8.8.
+// Workgroups that a CU should hold, 0: as many as fit.  Half of the sweeps
+// write lane i's value two records from lane i - 1's, so lines leave L2 partly
+// written, and where the records of the resident problems spill from the 256
+// MB Infinity Cache each costs memory traffic (4096 problems of 201 x 201 with
+// two a CU, 424 MB: 61 GB written for 27 GB of records).  So no bound up to 128
+// MB in all, else what keeps 230 MB, up to a wave a SIMD or two workgroups
+// (three of two bands up to 128 MB).  ms with 1, 2, 3, 4 and 8 a CU, and the MB
+// of one on every CU:
+//   4096 of 201 x 201  212 MB  28.0 31.8
+//   4096 of 120 x 180  129     14.5 15.2
+//   4096 of 40 x 250   103     12.5 10.1
+//   4096 of 60 x 200    98     13.7 13.1
+//   4096 of 120 x 128   94     12.2  8.5 10.5 11.7
+//   4096 of 300 x 60    87     17.8  9.6  9.8 10.8 13.3
+//   4096 of 80 x 100    59     10.3  6.7  7.3  8.7
+//   4096 of 40 x 100    41      8.4  5.2  4.7  5.8
+//   8192 of 51 x 41     19     13.9  7.5  6.1  6.1  8.8
+//   4096 of 5 x 100     27      6.6  4.0  3.2  3.4
+//   1024 of 5 x 100 (109 MB in all)      1.66 1.06 1.00 0.72
+//   2048 of 20 x 40 (106 MB in all)      2.18 1.18 1.01 0.86 0.77
+static int64_t band_workgroups_per_cu(const Plan2D &plan)
+{
+    constexpr int64_t kCUs = 256, kMB = (int64_t) 1 << 20;
+    const int64_t n = plan.problems[kBands2d] +
+                      plan.problems[kBandsAnyRange2d];
+    if (plan.recordBytes <= 128*kMB) { return 0; }
+    const int64_t each = plan.recordBytes/n*kCUs;
+    const int64_t waves = 4*n/plan.bands;       // of one a SIMD
+    if (waves == 2 && 3*each <= 128*kMB) { return 3; }
+    return std::max<int64_t>(1, std::min(std::max<int64_t>(2, waves),
+                                         230*kMB/each));
+}
+
+// LDS that a band workgroup asks for beyond its own, so that a CU holds no
+// more of them.
 static size_t band_residency_lds(const Plan2D &plan, size_t own)
 {
     constexpr size_t kLdsPerCU = 160*1024;
-    constexpr int64_t kCUs = 256, kResidentBytes = (int64_t) 200 << 20;
-    const int64_t n = plan.problems[kBands2d] +
-                      plan.problems[kBandsAnyRange2d];
-    const int64_t waves = 4*n/plan.bands;
-    const int64_t cached = kResidentBytes*n/(kCUs*plan.recordBytes);
-    const int64_t groups = std::max<int64_t>(
-        1, std::min(std::max<int64_t>(2, waves), cached));
+    const size_t groups = (size_t) band_workgroups_per_cu(plan);
+    if (groups == 0) { return 0; }
     // (a margin of 2 KB for the allocation's granules)
-    const size_t share = kLdsPerCU/(size_t) groups/1024*1024 - 2048;
+    const size_t share = kLdsPerCU/groups/1024*1024 - 2048;
     return share > own ? share - own : 0;
 }
 
