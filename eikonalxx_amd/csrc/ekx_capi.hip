@@ -28,6 +28,8 @@ namespace
 
 // Blocks of the model-maximum reduction (FIXED32 modes).
 constexpr size_t kMaxPartials = 1024;
+// reads up to this size share the stream of the work (Engine3D::copy_out)
+constexpr size_t kSmallRead = (size_t) 1 << 20;
 // blocks of the reduction of one model's slowness range
 constexpr int kRangeBlocks = 256;
 // Column z-chunk depths the launch-shape choice considers (0: whole
@@ -555,6 +557,7 @@ struct Engine3D
     double flowWaitMs = -1;      // a caller's bound of one wait
     bool flowUniform = false;
     hipStream_t stream = nullptr;
+    mutable hipStream_t copyStream = nullptr;       // copy_out
     hipEvent_t evFork = nullptr;
     hipEvent_t evStart = nullptr, evStop = nullptr;
     // kernel_timing: event pairs around the bulk column launches
@@ -622,6 +625,7 @@ struct Engine3D
         {
             if (e) { (void) hipEventDestroy(e); }
         }
+        if (copyStream) { (void) hipStreamDestroy(copyStream); }
         if (stream) { (void) hipStreamDestroy(stream); }
     }
 
@@ -2426,13 +2430,31 @@ struct Engine3D
         return EKX_OK;
     }
 
-    // Device to host on the engine's own stream: a copy on the default
-    // stream fails while another thread's solver captures its graph.
+    // Device to host, after the engine's stream, on a stream of its own.  A
+    // copy on the default stream fails while another thread's solver captures
+    // its graph.  On the engine's stream the next upload paid for it: the
+    // runtime lets go of the host pages of a stream's last copy with the next
+    // one (a new solver's set_slowness after the first read of a 257 x 257 x
+    // 193 field: 19 ms, 8 so).  Small reads go through the runtime's own
+    // buffers, and creating the stream is 70 us.
     ekx_status copy_out(void *dst, const void *src, size_t bytes) const
     {
-        EKX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
-                               stream));
+        if (bytes <= kSmallRead)
+        {
+            EKX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
+                                   stream));
+            EKX_HIP(hipStreamSynchronize(stream));
+            return EKX_OK;
+        }
+        if (!copyStream)
+        {
+            EKX_HIP(hipStreamCreateWithFlags(&copyStream,
+                                             hipStreamNonBlocking));
+        }
         EKX_HIP(hipStreamSynchronize(stream));
+        EKX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
+                               copyStream));
+        EKX_HIP(hipStreamSynchronize(copyStream));
         return EKX_OK;
     }
 

@@ -146,8 +146,8 @@ struct Range2D
     }
 };
 
-// A copy between host and device on the handle's own stream, and its end: on
-// the default stream it fails while another thread's solver captures.
+// A copy between host and device on one of the handle's own streams, and its
+// end: on the default stream it fails while another thread's solver captures.
 ekx_status copy2d(void *dst, const void *src, size_t bytes,
                   hipStream_t stream)
 {
@@ -155,6 +155,32 @@ ekx_status copy2d(void *dst, const void *src, size_t bytes,
     EKX2_HIP(hipStreamSynchronize(stream));
     return EKX_OK;
 }
+
+// The stream that reads large fields back (the handle's work is done when a
+// call returns): on the stream of the uploads the next upload would pay for
+// letting go of the host pages (Engine3D::copy_out).
+struct ReadStream
+{
+    hipStream_t stream = nullptr;
+    ReadStream() = default;
+    ReadStream(const ReadStream &) = delete;
+    ReadStream &operator=(const ReadStream &) = delete;
+    ~ReadStream()
+    {
+        if (stream) { (void) hipStreamDestroy(stream); }
+    }
+    ekx_status read(void *dst, const void *src, size_t bytes,
+                    hipStream_t work)
+    {
+        constexpr size_t kSmallRead = (size_t) 1 << 20;
+        if (bytes <= kSmallRead) { return copy2d(dst, src, bytes, work); }
+        if (!stream)
+        {
+            EKX2_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
+        }
+        return copy2d(dst, src, bytes, stream);
+    }
+};
 
 // (201 x 201, out of range: 2.8 ms by levels in LDS, 3.1 by levels in
 // memory, 1.5 by bands with range tests, 1.2 without)
@@ -273,6 +299,7 @@ struct ekx_solver2d
     Buf<int> stationCX, stationCZ;
     Buf<Problem2D> dProblem;
     hipStream_t stream = nullptr;
+    mutable ReadStream reads;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool initialized = false, haveModel = false, haveSource = false;
     bool haveField = false;
@@ -584,8 +611,8 @@ ekx_status ekx_solver2d_get_travel_times(const ekx_solver2d *h, int64_t n,
             return fail2(EKX_EINVAL, "output must hold the " +
                                          std::to_string(nGrid) + " grid points");
         }
-        EKX2_CHECK(copy2d(out, h->T.ptr, (size_t) n*sizeof(double),
-                          h->stream));
+        EKX2_CHECK(h->reads.read(out, h->T.ptr, (size_t) n*sizeof(double),
+                                 h->stream));
         return EKX_OK;
     });
 }
@@ -658,8 +685,8 @@ ekx_status ekx_solver2d_get_travel_time_gradient_field(const ekx_solver2d *h,
             return fail2(EKX_EINVAL, "output must hold 2 x " +
                                          std::to_string(want/2) + " values");
         }
-        EKX2_CHECK(copy2d(out, h->G.ptr, (size_t) n*sizeof(double),
-                          h->stream));
+        EKX2_CHECK(h->reads.read(out, h->G.ptr, (size_t) n*sizeof(double),
+                                 h->stream));
         return EKX_OK;
     });
 }
@@ -692,6 +719,7 @@ struct ekx_batch2d
     Bands2D bands;
     Buf<Problem2D> dProblems;
     hipStream_t stream = nullptr;
+    mutable ReadStream reads;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // problems solved by one launch, which the slices after it share the
     // band kernel's travel times with
@@ -978,8 +1006,8 @@ ekx_status ekx_batch2d_get_travel_times(const ekx_batch2d *h, int problem,
             return fail2(EKX_EINVAL, "output must hold the " +
                                          std::to_string(nGrid) + " grid points");
         }
-        EKX2_CHECK(copy2d(out, h->T.ptr + p.tOffset, (size_t) n*sizeof(double),
-                          h->stream));
+        EKX2_CHECK(h->reads.read(out, h->T.ptr + p.tOffset,
+                                 (size_t) n*sizeof(double), h->stream));
         return EKX_OK;
     });
 }
