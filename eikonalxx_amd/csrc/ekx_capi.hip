@@ -8,7 +8,7 @@
 #include "ekx_storage.hpp"
 
 #include <algorithm>
-#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -460,8 +460,8 @@ ekx_status scratch_address(Problem3D **out)
 
 namespace
 {
-// Waves of flow launches in progress per device (FlowReservation).
-std::atomic<int> g_flowWaves[kMaxDevices];
+// Waves of flow launches in progress per device.
+FlowWaves g_flowWaves[kMaxDevices];
 } // namespace
 
 // ===========================================================================
@@ -871,13 +871,17 @@ struct Engine3D
     {
         if (flowWaitMs >= 0) { return (uint64_t) (clockKHz*flowWaitMs); }
         constexpr double kStepMs = 4e-3;
-        const double chain = 0.5*(double) flowChain;
-        double steps = 4*chain;
-        if (flowWaves > flowCapacity)
-        {
-            steps += nSweeps*(0.5*(double) flowSteps/flowCapacity + chain);
-        }
+        double steps = 2*(double) flowChain;
+        if (flowWaves > flowCapacity) { steps += nSweeps*flow_steps(); }
         return (uint64_t) (clockKHz*std::max(250.0, kStepMs*steps));
+    }
+
+    // Steps that a sweep of the launch takes.
+    double flow_steps() const
+    {
+        const double chain = 0.5*(double) flowChain;
+        return flowWaves > flowCapacity
+                   ? 0.5*(double) flowSteps/flowCapacity + chain : chain;
     }
 
     ekx_status set_wait_bound(double ms)
@@ -1065,8 +1069,12 @@ struct Engine3D
 
     // Whether this solve can run as flow launches; takes their waves: as if
     // every XCD had as many as the one with most, so that the columns of
-    // launches that run together are resident on each.
-    bool take_flow(FlowReservation &r) const
+    // launches that run together are resident on each.  Beside other threads'
+    // it waits for its turn, as long as the solve by diagonals takes (four
+    // times its own time, at 0.6 us a step), and then goes by diagonals: 257 x
+    // 257 x 97 on 3 threads, ms a solve: 12.6 when it went there at once, 8.2
+    // so, 11.3 all by diagonals; on 8 threads 15.0, 10.0 and 16.1.
+    bool take_flow(FlowReservation &r, int nSweeps) const
     {
         if (flowColumns.empty()) { return false; }
         for (const Problem3D &p : problems)
@@ -1078,7 +1086,8 @@ struct Engine3D
                device < kMaxDevices &&
                r.take(g_flowWaves[device],
                       std::min((int) flowColumns.size(), flowCapacity),
-                      flowCapacity);
+                      flowCapacity, std::chrono::duration<double>(
+                          4*0.6e-6*nSweeps*flow_steps()));
     }
 
     template <typename TS> DeviceBuffer<TS> &flow_records_buffer()
@@ -2182,7 +2191,7 @@ struct Engine3D
     {
         ms = -1;
         FlowReservation r;
-        if (!take_flow(r)) { return EKX_OK; }
+        if (!take_flow(r, 16)) { return EKX_OK; }
         EKX_CHECK(trial_ms(true, ms));
         unsigned int err = 0;
         EKX_CHECK(copy_out(&err, flowWords.ptr, sizeof(err)));
@@ -2314,7 +2323,10 @@ struct Engine3D
         bool flowFailed = false;
         {
             FlowReservation r;
-            if (take_flow(r)) { EKX_CHECK(solve_fields(true, flowFailed)); }
+            if (take_flow(r, 8*(1 + opt.number_of_sweeps)))
+            {
+                EKX_CHECK(solve_fields(true, flowFailed));
+            }
             else { EKX_CHECK(solve_fields(false, flowFailed)); }
         }
         // A wait of the flow launch exceeded its bound (the device is shared

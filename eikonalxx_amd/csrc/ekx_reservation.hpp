@@ -1,14 +1,68 @@
 // ekx_reservation.hpp -- waves of flow launches in progress, per device.
 #pragma once
-#include <atomic>
+#include <chrono>
+#include <condition_variable>
+#include <cstdint>
+#include <deque>
+#include <mutex>
 
 namespace ekx
 {
 
+// The resident waves of one device, as flow launches of the process's threads
+// take them.  Requests are served in the order they come.
+class FlowWaves
+{
+public:
+    // n waves out of `capacity`, waiting up to maxWait for others' to be
+    // given back; false: not granted.
+    bool take(int n, int capacity, std::chrono::duration<double> maxWait)
+    {
+        std::unique_lock<std::mutex> lock(mutex);
+        const uint64_t me = ++last;
+        waiting.push_back(me);
+        const bool granted = changed.wait_for(lock, maxWait, [&]()
+        {
+            return waiting.front() == me && n <= capacity - taken;
+        });
+        for (auto it = waiting.begin(); it != waiting.end(); ++it)
+        {
+            if (*it == me)
+            {
+                waiting.erase(it);
+                break;
+            }
+        }
+        if (granted) { taken += n; }
+        // (the next in line may fit beside, or was held up by this one)
+        changed.notify_all();
+        return granted;
+    }
+    void give(int n)
+    {
+        {
+            std::lock_guard<std::mutex> lock(mutex);
+            taken -= n;
+        }
+        changed.notify_all();
+    }
+    int in_use()
+    {
+        std::lock_guard<std::mutex> lock(mutex);
+        return taken;
+    }
+
+private:
+    std::mutex mutex;
+    std::condition_variable changed;
+    std::deque<uint64_t> waiting;
+    uint64_t last = 0;
+    int taken = 0;
+};
+
 // A flow launch needs the waves of a problem resident together, so it takes
 // place only if its waves fit beside those of the other flow launches of the
-// process (other threads' solvers); otherwise the solve uses the launches
-// per diagonal.
+// process (other threads' solvers).
 class FlowReservation
 {
 public:
@@ -16,28 +70,23 @@ public:
     FlowReservation(const FlowReservation &) = delete;
     FlowReservation &operator=(const FlowReservation &) = delete;
     ~FlowReservation() { release(); }
-    // n waves out of `capacity`, of which `taken` are in use.  Refused only
-    // if they do not fit: nothing is added before it is known to.
-    bool take(std::atomic<int> &taken, int n, int capacity)
+    bool take(FlowWaves &from_, int n, int capacity,
+              std::chrono::duration<double> maxWait)
     {
         release();
-        int now = taken.load();
-        do
-        {
-            if (n > capacity - now) { return false; }
-        } while (!taken.compare_exchange_weak(now, now + n));
-        from = &taken;
+        if (!from_.take(n, capacity, maxWait)) { return false; }
+        from = &from_;
         waves = n;
         return true;
     }
     void release()
     {
-        if (from) { from->fetch_sub(waves); }
+        if (from) { from->give(waves); }
         from = nullptr;
     }
 
 private:
-    std::atomic<int> *from = nullptr;
+    FlowWaves *from = nullptr;
     int waves = 0;
 };
 

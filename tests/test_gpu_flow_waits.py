@@ -83,3 +83,40 @@ def test_past_the_bound_by_diagonals(ekx, oracle, precision, batch):
     assert np.array_equal(field(), ref)
     with pytest.raises(ValueError):
         s.set_wait_bound(1e10)
+
+
+def test_threads_take_turns(ekx, oracle):
+    """Three solvers of 1089 columns on three threads: the device holds one at a
+    time, and the others wait for their turn instead of going by diagonals."""
+    import threading
+    dims, h = (257, 257, 40), 10.0
+    rng = np.random.default_rng(14)
+    slow = 1.0 / rng.uniform(1800.0, 5200.0, 256 * 256 * 39)
+    sources = [(310.0, 420.0, 55.0), (1900.0, 77.0, 11.0),
+               (1000.0, 2000.0, 90.0)]
+    launches, same = [[] for _ in sources], [False] * len(sources)
+    solvers = []
+    for x in sources:
+        s = ekx.Solver3D()
+        s.initialize(ekx.SolverOptions(number_of_sweeps=2, factored_radius=2),
+                     ekx.Geometry3D(*dims, h))
+        s.set_slowness(slow)
+        s.set_source(x)
+        solvers.append(s)
+    refs = [oracle.solve3d(oracle.geometry3d(*dims, h), slow, x, 2, 2)
+            for x in sources]
+
+    def work(k):
+        for _ in range(6):
+            solvers[k].solve()
+            launches[k].append(solvers[k].get_stats().kernel_launches)
+        same[k] = np.array_equal(solvers[k].get_travel_time_field(), refs[k])
+    threads = [threading.Thread(target=work, args=(k,))
+               for k in range(len(sources))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    print("launches", launches, flush=True)
+    assert all(same), same
+    assert launches == [[1] * 6] * 3
