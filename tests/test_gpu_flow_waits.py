@@ -102,6 +102,7 @@ def test_threads_take_turns(ekx, oracle):
                      ekx.Geometry3D(*dims, h))
         s.set_slowness(slow)
         s.set_source(x)
+        s.solve()
         solvers.append(s)
     refs = [oracle.solve3d(oracle.geometry3d(*dims, h), slow, x, 2, 2)
             for x in sources]
