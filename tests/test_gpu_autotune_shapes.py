@@ -17,7 +17,7 @@ def test_default_shape_is_the_one_timed(ekx):
     """1800 problems of 65 x 65 x 70 run by whole columns of 70 planes with the
     box in the bulk launches: the tuned solves are no slower than the default
     (with the box timed in launches of its own the tuner took another depth,
-    14% slower; the bar is 5%, shortest of four)."""
+    14% slower; the bar is 8%, shortest of four)."""
     dims, h, n = (65, 65, 70), 10.0, 1800
     rng, slow = _inputs(dims, 3)
     g = ekx.Geometry3D(*dims, h)
@@ -45,7 +45,7 @@ def test_default_shape_is_the_one_timed(ekx):
         assert st.updates_factored == default.updates_factored
     for i, f in zip((0, 899, 1799), fields):
         assert np.array_equal(b.get_travel_time_field(i), f), i
-    assert after <= 1.05 * before
+    assert after <= 1.08 * before
 
 
 @pytest.mark.parametrize("precision", ["FP64", "FP32_POLISH"])
