@@ -15,6 +15,7 @@
 #include <limits>
 #include <map>
 #include <mutex>
+#include <shared_mutex>
 #include <numeric>
 #include <string>
 #include <tuple>
@@ -460,6 +461,9 @@ ekx_status scratch_address(Problem3D **out)
 
 namespace
 {
+// Held shared by captures in progress: the device cannot be synchronised
+// meanwhile.
+std::shared_mutex g_captures;
 // Waves of flow launches in progress per device.
 FlowWaves g_flowWaves[kMaxDevices];
 } // namespace
@@ -2056,12 +2060,14 @@ struct Engine3D
             if (!g.valid)
             {
                 g.release();
+                std::shared_lock<std::shared_mutex> capturing(g_captures);
                 EKX_HIP(hipStreamBeginCapture(stream,
                                               hipStreamCaptureModeThreadLocal));
                 ekx_status s = enqueue_phase_sweeps<TS>(T, S, doInit,
                                                         iterations, local);
                 hipGraph_t captured = nullptr;
                 hipError_t e = hipStreamEndCapture(stream, &captured);
+                capturing.unlock();
                 if (s != EKX_OK)
                 {
                     if (captured) { (void) hipGraphDestroy(captured); }
@@ -2885,6 +2891,8 @@ ekx_status ekx_device_synchronize(void)
 {
     return guarded([&]() -> ekx_status
     {
+        // (not while a solver captures on another thread)
+        std::unique_lock<std::shared_mutex> quiet(g_captures);
         EKX_HIP(hipDeviceSynchronize());
         return EKX_OK;
     });

@@ -1,5 +1,6 @@
-"""2D solvers, 2D batches and generated models on one thread while another
-captures the launches of a 3D solver: neither disturbs the other."""
+"""2D solvers, 2D batches, generated models, a second 3D solver and the device's
+synchronisation on one thread while another captures the launches of a 3D
+solver: neither disturbs the other."""
 import threading
 
 import numpy as np
@@ -47,6 +48,15 @@ def test_2d_beside_a_capture(ekx, oracle):
         rel = np.abs(field - ref2) / np.maximum(ref2, slow2.min() * 10.0)
         assert rel.max() <= 1e-12
 
+    small = (9, 11, 10)
+    slow_small = 1.0 / rng.uniform(1800.0, 5200.0, 8 * 10 * 9)
+    s3 = ekx.Solver3D()
+    s3.initialize(ekx.SolverOptions(number_of_sweeps=1, factored_radius=2),
+                  ekx.Geometry3D(*small, h))
+    s3.set_slowness(slow_small)
+    s3.set_stations([(20.0, 30.0, 40.0)])
+    ref3 = oracle.solve3d(oracle.geometry3d(*small, h), slow_small,
+                          (31.0, 22.0, 13.0), 1, 2)
     model = ekx.LayeredGaussianModel([2500.0, 3500.0, 5000.0], 0.1, 40.0, 2)
     gm = ekx.Geometry3D(20, 9, 13, 5.0, 12.0, 7.0)
     velocity = model.generate(gm)
@@ -65,6 +75,13 @@ def test_2d_beside_a_capture(ekx, oracle):
             s.compute_travel_time_gradient_field()
             s.get_travel_time_gradient_field()
             assert np.array_equal(model.generate(gm), velocity)
+            ekx.synchronize()
+            s3.set_source((31.0, 22.0, 13.0))
+            s3.solve()
+            assert np.array_equal(s3.get_travel_time_field(), ref3)
+            assert len(s3.get_travel_times_at_stations()) == 1
+            s3.compute_travel_time_gradient_field()
+            s3.get_travel_time_gradient_field()
             b = ekx.Batch2D()
             b.initialize(o, [(g2, slow2, src2)] * 3)
             b.solve()
