@@ -4,6 +4,7 @@
 #include "eikonalxx_amd.h"
 #include "ekx_guard.hpp"
 #include "ekx_kernels.hpp"
+#include "ekx_reads.hpp"
 #include "ekx_reservation.hpp"
 #include "ekx_storage.hpp"
 
@@ -29,8 +30,6 @@ namespace
 
 // Blocks of the model-maximum reduction (FIXED32 modes).
 constexpr size_t kMaxPartials = 1024;
-// reads up to this size share the stream of the work (Engine3D::copy_out)
-constexpr size_t kSmallRead = (size_t) 1 << 20;
 // blocks of the reduction of one model's slowness range
 constexpr int kRangeBlocks = 256;
 // Column z-chunk depths the launch-shape choice considers (0: whole
@@ -571,7 +570,6 @@ struct Engine3D
     Counts flowCounts[2];
     bool flowUniform = false;
     hipStream_t stream = nullptr;
-    mutable hipStream_t copyStream = nullptr;       // copy_out
     hipEvent_t evFork = nullptr;
     hipEvent_t evStart = nullptr, evStop = nullptr;
     // kernel_timing: event pairs around the bulk column launches
@@ -639,7 +637,6 @@ struct Engine3D
         {
             if (e) { (void) hipEventDestroy(e); }
         }
-        if (copyStream) { (void) hipStreamDestroy(copyStream); }
         if (stream) { (void) hipStreamDestroy(stream); }
     }
 
@@ -2467,31 +2464,9 @@ struct Engine3D
         return EKX_OK;
     }
 
-    // Device to host, after the engine's stream, on a stream of its own.  A
-    // copy on the default stream fails while another thread's solver captures
-    // its graph.  On the engine's stream the next upload paid for it: the
-    // runtime lets go of the host pages of a stream's last copy with the next
-    // one (a new solver's set_slowness after the first read of a 257 x 257 x
-    // 193 field: 19 ms, 8 so).  Small reads go through the runtime's own
-    // buffers, and creating the stream is 70 us.
     ekx_status copy_out(void *dst, const void *src, size_t bytes) const
     {
-        if (bytes <= kSmallRead)
-        {
-            EKX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
-                                   stream));
-            EKX_HIP(hipStreamSynchronize(stream));
-            return EKX_OK;
-        }
-        if (!copyStream)
-        {
-            EKX_HIP(hipStreamCreateWithFlags(&copyStream,
-                                             hipStreamNonBlocking));
-        }
-        EKX_HIP(hipStreamSynchronize(stream));
-        EKX_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost,
-                               copyStream));
-        EKX_HIP(hipStreamSynchronize(copyStream));
+        EKX_HIP(read_back(dst, src, bytes, stream));
         return EKX_OK;
     }
 

@@ -2,6 +2,7 @@
 #include "eikonalxx_amd.h"
 #include "ekx_guard.hpp"
 #include "ekx_kernels.hpp"
+#include "ekx_reads.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -146,41 +147,15 @@ struct Range2D
     }
 };
 
-// A copy between host and device on one of the handle's own streams, and its
-// end: on the default stream it fails while another thread's solver captures.
-ekx_status copy2d(void *dst, const void *src, size_t bytes,
-                  hipStream_t stream)
+// Host to device on the handle's own stream, and its end: on the default
+// stream it fails while another thread's solver captures.
+ekx_status upload2d(void *dst, const void *src, size_t bytes,
+                    hipStream_t stream)
 {
-    EKX2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDefault, stream));
+    EKX2_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
     EKX2_HIP(hipStreamSynchronize(stream));
     return EKX_OK;
 }
-
-// The stream that reads large fields back (the handle's work is done when a
-// call returns): on the stream of the uploads the next upload would pay for
-// letting go of the host pages (Engine3D::copy_out).
-struct ReadStream
-{
-    hipStream_t stream = nullptr;
-    ReadStream() = default;
-    ReadStream(const ReadStream &) = delete;
-    ReadStream &operator=(const ReadStream &) = delete;
-    ~ReadStream()
-    {
-        if (stream) { (void) hipStreamDestroy(stream); }
-    }
-    ekx_status read(void *dst, const void *src, size_t bytes,
-                    hipStream_t work)
-    {
-        constexpr size_t kSmallRead = (size_t) 1 << 20;
-        if (bytes <= kSmallRead) { return copy2d(dst, src, bytes, work); }
-        if (!stream)
-        {
-            EKX2_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-        }
-        return copy2d(dst, src, bytes, stream);
-    }
-};
 
 // (201 x 201, out of range: 2.8 ms by levels in LDS, 3.1 by levels in
 // memory, 1.5 by bands with range tests, 1.2 without)
@@ -299,7 +274,6 @@ struct ekx_solver2d
     Buf<int> stationCX, stationCZ;
     Buf<Problem2D> dProblem;
     hipStream_t stream = nullptr;
-    mutable ReadStream reads;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     bool initialized = false, haveModel = false, haveSource = false;
     bool haveField = false;
@@ -523,14 +497,14 @@ ekx_status ekx_solver2d_set_stations(ekx_solver2d *h, int n, const double *x,
         EKX2_CHECK(h->stationOut.allocate(m));
         if (n > 0)
         {
-            EKX2_CHECK(copy2d(h->stationX.ptr, xo.data(), n*sizeof(double),
-                              h->stream));
-            EKX2_CHECK(copy2d(h->stationZ.ptr, zo.data(), n*sizeof(double),
-                              h->stream));
-            EKX2_CHECK(copy2d(h->stationCX.ptr, cx.data(), n*sizeof(int),
-                              h->stream));
-            EKX2_CHECK(copy2d(h->stationCZ.ptr, cz.data(), n*sizeof(int),
-                              h->stream));
+            EKX2_CHECK(upload2d(h->stationX.ptr, xo.data(), n*sizeof(double),
+                                h->stream));
+            EKX2_CHECK(upload2d(h->stationZ.ptr, zo.data(), n*sizeof(double),
+                                h->stream));
+            EKX2_CHECK(upload2d(h->stationCX.ptr, cx.data(), n*sizeof(int),
+                                h->stream));
+            EKX2_CHECK(upload2d(h->stationCZ.ptr, cz.data(), n*sizeof(int),
+                                h->stream));
         }
         return EKX_OK;
     });
@@ -556,9 +530,9 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         p.srcOffX = h->source.off[0];
         p.srcOffZ = h->source.off[1];
         const int ncx = h->geometry.nx - 1;
-        EKX2_CHECK(copy2d(&p.srcSlowness,
-                          h->S.ptr + (size_t) p.srcCellZ*ncx + p.srcCellX,
-                          sizeof(double), h->stream));
+        EKX2_HIP(read_back(&p.srcSlowness,
+                           h->S.ptr + (size_t) p.srcCellZ*ncx + p.srcCellX,
+                           sizeof(double), h->stream));
         p.route = route2d(h->bands.work != nullptr, h->scaled);
         Plan2D plan;
         plan.add(p);
@@ -581,8 +555,8 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         h->stationTimes.assign((size_t) ns, 0.0);
         if (ns > 0)
         {
-            EKX2_CHECK(copy2d(h->stationTimes.data(), h->stationOut.ptr,
-                              ns*sizeof(double), h->stream));
+            EKX2_HIP(read_back(h->stationTimes.data(), h->stationOut.ptr,
+                               ns*sizeof(double), h->stream));
         }
         float ms = 0;
         EKX2_HIP(hipEventElapsedTime(&ms, h->ev0, h->ev1));
@@ -611,8 +585,8 @@ ekx_status ekx_solver2d_get_travel_times(const ekx_solver2d *h, int64_t n,
             return fail2(EKX_EINVAL, "output must hold the " +
                                          std::to_string(nGrid) + " grid points");
         }
-        EKX2_CHECK(h->reads.read(out, h->T.ptr, (size_t) n*sizeof(double),
-                                 h->stream));
+        EKX2_HIP(read_back(out, h->T.ptr, (size_t) n*sizeof(double),
+                           h->stream));
         return EKX_OK;
     });
 }
@@ -685,8 +659,8 @@ ekx_status ekx_solver2d_get_travel_time_gradient_field(const ekx_solver2d *h,
             return fail2(EKX_EINVAL, "output must hold 2 x " +
                                          std::to_string(want/2) + " values");
         }
-        EKX2_CHECK(h->reads.read(out, h->G.ptr, (size_t) n*sizeof(double),
-                                 h->stream));
+        EKX2_HIP(read_back(out, h->G.ptr, (size_t) n*sizeof(double),
+                           h->stream));
         return EKX_OK;
     });
 }
@@ -719,7 +693,6 @@ struct ekx_batch2d
     Bands2D bands;
     Buf<Problem2D> dProblems;
     hipStream_t stream = nullptr;
-    mutable ReadStream reads;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // problems solved by one launch, which the slices after it share the
     // band kernel's travel times with
@@ -1006,8 +979,8 @@ ekx_status ekx_batch2d_get_travel_times(const ekx_batch2d *h, int problem,
             return fail2(EKX_EINVAL, "output must hold the " +
                                          std::to_string(nGrid) + " grid points");
         }
-        EKX2_CHECK(h->reads.read(out, h->T.ptr + p.tOffset,
-                                 (size_t) n*sizeof(double), h->stream));
+        EKX2_HIP(read_back(out, h->T.ptr + p.tOffset,
+                           (size_t) n*sizeof(double), h->stream));
         return EKX_OK;
     });
 }
