@@ -529,15 +529,14 @@ ekx_status ekx_solver2d_solve(ekx_solver2d *h)
         p.srcCellZ = h->source.cell[1];
         p.srcOffX = h->source.off[0];
         p.srcOffZ = h->source.off[1];
-        const int ncx = h->geometry.nx - 1;
-        EKX2_HIP(read_back(&p.srcSlowness,
-                           h->S.ptr + (size_t) p.srcCellZ*ncx + p.srcCellX,
-                           sizeof(double), h->stream));
         p.route = route2d(h->bands.work != nullptr, h->scaled);
         Plan2D plan;
         plan.add(p);
-        EKX2_HIP(hipMemcpyAsync(h->dProblem.ptr, &p, sizeof(Problem2D),
-                                hipMemcpyHostToDevice, h->stream));
+        // (the source cell's slowness comes from the device's model)
+        EKX2_HIP(launch_store_problem2d(
+            p, h->S.ptr + (size_t) p.srcCellZ*(h->geometry.nx - 1) +
+                   p.srcCellX,
+            h->dProblem.ptr, h->stream));
         EKX2_HIP(hipEventRecord(h->ev0, h->stream));
         EKX2_HIP(launch_solve2d(h->dProblem.ptr, 1, plan, h->T.ptr, h->S.ptr,
                                 h->bands.work, h->bands.cells, h->stream));

@@ -178,6 +178,9 @@ hipError_t launch_solve2d(const Problem2D *dProblems, int nProblems,
                           const Plan2D &plan, double *T, const double *S,
                           double *work, const double *cells,
                           hipStream_t stream);
+// Writes a problem's descriptor, with the slowness at `cell` as its source's.
+hipError_t launch_store_problem2d(const Problem2D &p, const double *cell,
+                                  Problem2D *dst, hipStream_t stream);
 // The band kernel's cell records of one model (cell_values2d values).
 hipError_t launch_skew_cells2d(int nx, int nz, const double *s, double *out,
                                hipStream_t stream);
